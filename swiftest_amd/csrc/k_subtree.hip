@@ -71,6 +71,7 @@ constexpr int L_T = 256;                  // threads of its workgroup
 constexpr int L_NB = 512, L_NE = 4096;    // pl bodies, pl entries (pairs = entries / 2)
 constexpr int L_NP = L_NE / 2;
 constexpr int L_NBT = 256, L_NET = 1024;  // tp bodies, tp entries
+constexpr int L_NS = L_NB + L_NBT;        // body slots
 
 __device__ inline bool lds_eligible(int nB, int nE, int nBt, int nEt)
 {
@@ -434,14 +435,16 @@ constexpr int L_KS = (L_NB + L_NBT + L_T - 1) / L_T;  // bodies folded per lane
 static_assert(L_KS * L_T == L_NB + L_NBT, "the kick-list arrays cover every lane slot");
 
 struct LdsSet {
-    double px[L_NB], py[L_NB], pz[L_NB], pvx[L_NB], pvy[L_NB], pvz[L_NB], ph[L_NB], pgm[L_NB], pR[L_NB];
-    int pg[L_NB], plev[L_NB], plm[L_NB], pst[L_NB], pO[L_NB + 1];
+    // bodies: massive ones at [0, L_NB), test particles from L_NB on
+    // the one at L_NS is nobody's: wave-mode lanes without a body use it
+    double px[L_NS + 1], py[L_NS + 1], pz[L_NS + 1], pvx[L_NS + 1], pvy[L_NS + 1], pvz[L_NS + 1];
+    double ph[L_NB], pgm[L_NB], pR[L_NB];
+    int pg[L_NB], plev[L_NS + 1], plm[L_NS + 1], pst[L_NS + 1], pO[L_NB + 1];
     uint32_t pE[L_NE];
     int16_t ppi[L_NP], ppj[L_NP];
     int ppg[L_NP];
     int8_t pps[L_NP], ppl[L_NP], ppv[L_NP];
-    double tx[L_NBT], ty[L_NBT], tz[L_NBT], tvx[L_NBT], tvy[L_NBT], tvz[L_NBT];
-    int tg[L_NBT], tlev[L_NBT], tlm[L_NBT], tst[L_NBT], tO[L_NBT + 1];
+    int tg[L_NBT], tO[L_NBT + 1];
     int16_t tpl[L_NET], tpt[L_NET];
     int tpg[L_NET];
     int8_t tps[L_NET], tpl_lev[L_NET], tpv[L_NET];
@@ -451,20 +454,32 @@ struct LdsSet {
     int16_t lst[L_NE + L_NET];
     union {
         KTerm kt[L_KC];
+        struct {
+            KTerm kt_wave[64];            // wave mode's terms (kt[0, 64))
+            double shr[MAXLEV + 1][64];  // and its entries' shell radii, by level from the one it started at
+        };
         int16_t posu[L_NE + L_NET];  // while the list is built
         int lab[L_NB + L_NBT];       // connected-component labels, profiling only
     };
     int jst[MAXLEV + 2];
     int wsum[L_T / 64 + 1];
-    // wave mode (one wavefront runs a small sub-recursion): the level it
-    // started at, that level's bodies (pl, then tp as nB + t), pl pairs, tp
-    // entries, and the kick entries of its bodies grouped by body
-    int16_t wB[64], wP[64], wT[64], wE[64];
-    int8_t wEs[64], wEe[64], wH[64];  // wH: slots of the bodies the second wavefront drifts
-    int wnB, wnP, wnT, wnE, wstop, wnH, wlenc;
+    // wave mode (one wavefront runs a small sub-recursion): the bodies (as
+    // indices of the state arrays), pl pairs, tp entries and kick entries of
+    // the level it started at, each body's slot in wB and stretch of wE, and
+    // the bodies each wavefront drifts
+    int16_t wB[64], wP[64], wT[64], wE[64], wH[L_T / 64][64];
+    int8_t wEs[64], wEe[64], slot[L_NS];
+    int wnB, wnP, wnT, wnE, wstop, wlenc;
+    // per level: its time step, the powers of RSHELL (ShellPowers); and the
+    // deepest level whose step is above double precision (symba_step.f90:196-201)
+    double dtl[MAXLEV + 2], ssq[MAXLEV + 2], rsh[MAXLEV + 2];
+    int dmax;
     int npair, flag_pp, flag_pt, bad, nact, nlst, lst_level, kmax;
     unsigned long long prof[(MAXLEV + 2) * NPROF];  // per-level phase ticks when profiling
 };
+
+// the slice of the workgroup
+static __shared__ LdsSet s_lds;
 
 __device__ inline int lds_lower_bound(const int *a, int n, int key)
 {
@@ -519,15 +534,15 @@ __device__ bool lds_check(LdsSet &S, const SubArgs &A, int nB, int nEt, int d, d
             if (S.tps[u] != ACTIVE || S.tpl_lev[u] != d) continue;
             const int i = S.tpl[u], t = S.tpt[u];
             bool lv;
-            bool le = check_pt_v(S.px[i], S.py[i], S.pz[i], S.pvx[i], S.pvy[i], S.pvz[i], S.ph[i], S.pR[i], S.tx[t],
-                                 S.ty[t], S.tz[t], S.tvx[t], S.tvy[t], S.tvz[t], irec, dtl, lv);
+            bool le = check_pt_v(S.px[i], S.py[i], S.pz[i], S.pvx[i], S.pvy[i], S.pvz[i], S.ph[i], S.pR[i], S.px[L_NB + t],
+                                 S.py[L_NB + t], S.pz[L_NB + t], S.pvx[L_NB + t], S.pvy[L_NB + t], S.pvz[L_NB + t], irec, dtl, lv);
             S.tpv[u] = lv;
             if (le) {
                 S.tpl_lev[u] = (int8_t)irec;
                 S.plev[i] = irec;
                 atomicMax(&S.plm[i], irec);
-                S.tlev[t] = irec;
-                atomicMax(&S.tlm[t], irec);
+                S.plev[L_NB + t] = irec;
+                atomicMax(&S.plm[L_NB + t], irec);
                 S.flag_pt = 1;
             }
         }
@@ -603,6 +618,15 @@ __device__ inline int lds_block_scan(LdsSet &S, int v, int *tot)
     return r;
 }
 
+// the body of entry u (pl entries, then test-particle entries), as an index
+// of the state arrays
+__device__ inline int lds_entry_body(const LdsSet &S, int u, int nE)
+{
+    if (u >= nE) return L_NB + S.tpt[u - nE];
+    const uint32_t e = S.pE[u];
+    return ((e >> 9) & 1u) ? S.ppi[e >> 10] : S.ppj[e >> 10];
+}
+
 // whether entry u (pl entries, then test-particle entries) takes part in the
 // shell kicks of level d: its body and its partner are both in the level
 __device__ inline bool lds_entry_in_level(const LdsSet &S, int u, int nE, int d)
@@ -614,7 +638,7 @@ __device__ inline bool lds_entry_in_level(const LdsSet &S, int u, int nE, int d)
         return S.plev[q] >= d && S.plev[pr] >= d;
     }
     const int v = u - nE;
-    return S.tlev[S.tpt[v]] >= d && S.plev[S.tpl[v]] >= d;
+    return S.plev[L_NB + S.tpt[v]] >= d && S.plev[S.tpl[v]] >= d;
 }
 
 // The kick list of level d: the entries that take part, in entry order
@@ -649,7 +673,7 @@ __device__ void lds_level_list(LdsSet &S, int nB, int nBt, int nE, int nEt, int 
     __syncthreads();
     for (int q = tid; q < nB + nBt; q += L_T) {
         const bool ispl = q < nB;
-        if ((ispl ? S.plev[q] : S.tlev[q - nB]) < d) continue;
+        if ((ispl ? S.plev[q] : S.plev[L_NB + q - nB]) < d) continue;
         const int e0 = ispl ? S.pO[q] : nE + S.tO[q - nB], e1 = ispl ? S.pO[q + 1] : nE + S.tO[q - nB + 1];
         if (e1 <= e0) continue;
         const int f0 = S.posu[e0], f1 = e1 < N ? S.posu[e1] : tot;
@@ -688,7 +712,7 @@ __device__ __attribute__((always_inline)) inline void lds_kicks(LdsSet &S, int n
             const int q = S.act[ai];
             const bool ap = (kc[k].fl & 1) != 0, am = (kc[k].fl & 2) != 0;
             if (q < nB) lds_apply(S.pvx[q], S.pvy[q], S.pvz[q], dth, ap, kc[k].p, am, kc[k].m);
-            else lds_apply(S.tvx[q - nB], S.tvy[q - nB], S.tvz[q - nB], dth, ap, kc[k].p, am, kc[k].m);
+            else lds_apply(S.pvx[L_NB + q - nB], S.pvy[L_NB + q - nB], S.pvz[L_NB + q - nB], dth, ap, kc[k].p, am, kc[k].m);
         }
         __syncthreads();
         return;
@@ -733,7 +757,7 @@ __device__ __attribute__((always_inline)) inline void lds_kicks(LdsSet &S, int n
             } else {
                 const int v = u - nE, i = S.tpl[v], tt = S.tpt[v];
                 if (S.tps[v] == ACTIVE)
-                    tp_shell_term_v(S.tx[tt], S.ty[tt], S.tz[tt], S.px[i], S.py[i], S.pz[i], S.ph[i], S.pgm[i], spp,
+                    tp_shell_term_v(S.px[L_NB + tt], S.py[L_NB + tt], S.pz[L_NB + tt], S.px[i], S.py[i], S.pz[i], S.ph[i], S.pgm[i], spp,
                                     spm, true, t);
             }
             KTerm &K = S.kt[w];
@@ -770,7 +794,7 @@ __device__ __attribute__((always_inline)) inline void lds_kicks(LdsSet &S, int n
         if (ai >= nact) continue;
         const int q = S.act[ai];
         if (q < nB) lds_apply(S.pvx[q], S.pvy[q], S.pvz[q], dth, anyp[k], p[k], anym[k], m[k]);
-        else lds_apply(S.tvx[q - nB], S.tvy[q - nB], S.tvz[q - nB], dth, anyp[k], p[k], anym[k], m[k]);
+        else lds_apply(S.pvx[L_NB + q - nB], S.pvy[L_NB + q - nB], S.pvz[L_NB + q - nB], dth, anyp[k], p[k], anym[k], m[k]);
         if (mode == 1) {
             kc[k].p = p[k];
             kc[k].m = m[k];
@@ -793,19 +817,18 @@ __device__ __attribute__((always_inline)) inline void lds_kicks(LdsSet &S, int n
     __syncthreads();
 }
 
-__device__ void lds_drift(LdsSet &S, const SubArgs &A, int nB, int nBt, int d, double dtl, int s, bool prof)
+__device__ void lds_drift(LdsSet &S, const SubArgs &A, int nB, int nBt, int d, double dtl, double mu, int s, bool prof)
 {
-    const double mu = A.st.sy.GMcb[s];
     int ndr = 0;
     unsigned long long tdr = 0;
     for (int q = threadIdx.x; q < nB + nBt; q += L_T) {
         const bool ispl = q < nB;
         const int t = q - nB;
-        const bool on = ispl ? (S.pst[q] != INACTIVE && S.plev[q] == d) : (S.tst[t] == ACTIVE && S.tlev[t] == d);
+        const bool on = ispl ? (S.pst[q] != INACTIVE && S.plev[q] == d) : (S.pst[L_NB + t] == ACTIVE && S.plev[L_NB + t] == d);
         if (!on) continue;
         ndr++;
-        double *x = ispl ? S.px : S.tx, *y = ispl ? S.py : S.ty, *z = ispl ? S.pz : S.tz;
-        double *vx = ispl ? S.pvx : S.tvx, *vy = ispl ? S.pvy : S.tvy, *vz = ispl ? S.pvz : S.tvz;
+        double *x = ispl ? S.px : S.px + L_NB, *y = ispl ? S.py : S.py + L_NB, *z = ispl ? S.pz : S.pz + L_NB;
+        double *vx = ispl ? S.pvx : S.pvx + L_NB, *vy = ispl ? S.pvy : S.pvy + L_NB, *vz = ispl ? S.pvz : S.pvz + L_NB;
         const int k = ispl ? q : t;
         double rx = x[k], ry = y[k], rz = z[k], ux = vx[k], uy = vy[k], uz = vz[k];
         const unsigned long long t0 = prof ? wall_clock64() : 0;
@@ -822,7 +845,7 @@ __device__ void lds_drift(LdsSet &S, const SubArgs &A, int nB, int nBt, int d, d
                 S.pst[q] = DISCARDED_DRIFTERR;
                 atomicOr(&A.st.sy.err[s], 2);
             } else {
-                S.tst[t] = DISCARDED_DRIFTERR;
+                S.pst[L_NB + t] = DISCARDED_DRIFTERR;
             }
         }
     }
@@ -856,16 +879,16 @@ __device__ void lds_store(LdsSet &S, const SubArgs &A, int nB, int nBt, int nEt,
     }
     for (int q = threadIdx.x; q < nBt; q += L_T) {
         const int g = S.tg[q];
-        a.tp.rh.x[g] = S.tx[q];
-        a.tp.rh.y[g] = S.ty[q];
-        a.tp.rh.z[g] = S.tz[q];
-        a.tp.vb.x[g] = S.tvx[q];
-        a.tp.vb.y[g] = S.tvy[q];
-        a.tp.vb.z[g] = S.tvz[q];
+        a.tp.rh.x[g] = S.px[L_NB + q];
+        a.tp.rh.y[g] = S.py[L_NB + q];
+        a.tp.rh.z[g] = S.pz[L_NB + q];
+        a.tp.vb.x[g] = S.pvx[L_NB + q];
+        a.tp.vb.y[g] = S.pvy[L_NB + q];
+        a.tp.vb.z[g] = S.pvz[L_NB + q];
         if (all) {
-            a.tp.levelg[g] = S.tlev[q];
-            a.tp.levelm[g] = S.tlm[q];
-            a.tp.status[g] = S.tst[q];
+            a.tp.levelg[g] = S.plev[L_NB + q];
+            a.tp.levelm[g] = S.plm[L_NB + q];
+            a.tp.status[g] = S.pst[L_NB + q];
         }
     }
     for (int lp = threadIdx.x; lp < S.npair; lp += L_T) {
@@ -892,7 +915,7 @@ __device__ void lds_collision(LdsSet &S, const SubArgs &A, int nB, int nBt, int 
     for (int q = threadIdx.x; q < nB + nBt; q += L_T) {
         if (q < nB) {
             if (A.has_pp && S.plev[q] >= d) rec_collide_pl(A.st, S.pg[q], dtl, s);
-        } else if (S.tlev[q - nB] >= d) {
+        } else if (S.plev[L_NB + q - nB] >= d) {
             rec_collide_tp(A.st, S.tg[q - nB], dtl, s);
         }
     }
@@ -908,7 +931,7 @@ __device__ void lds_set_levels(LdsSet &S, int nB, int nBt, int nEt, int d)
     for (int q = tid; q < nB; q += L_T)
         if (S.plev[q] == irecp) S.plev[q] = d;
     for (int q = tid; q < nBt; q += L_T)
-        if (S.tlev[q] == irecp) S.tlev[q] = d;
+        if (S.plev[L_NB + q] == irecp) S.plev[L_NB + q] = d;
     for (int lp = tid; lp < S.npair; lp += L_T)
         if (S.ppl[lp] == irecp) S.ppl[lp] = (int8_t)d;
     for (int u = tid; u < nEt; u += L_T)
@@ -937,16 +960,23 @@ __device__ inline void wave_sync()
 }
 
 // Collect the sets of level dn with the whole workgroup; true when all fit.
+// The kick entries come out in entry order (so grouped by body, each body's
+// in list order), with each body's stretch of them.
 __device__ bool wave_sets(LdsSet &S, int nB, int nBt, int nE, int nEt, int dn)
 {
     const int tid = threadIdx.x;
     if (tid == 0) S.wnB = S.wnP = S.wnT = S.wnE = 0;
     __syncthreads();
-    for (int q = tid; q < nB + nBt; q += L_T)
-        if ((q < nB ? S.plev[q] : S.tlev[q - nB]) >= dn) {
+    for (int q = tid; q < nB + nBt; q += L_T) {
+        const int b = q < nB ? q : L_NB + (q - nB);
+        if (S.plev[b] >= dn) {
             const int k = atomicAdd(&S.wnB, 1);
-            if (k < 64) S.wB[k] = (int16_t)q;
+            if (k < 64) {
+                S.wB[k] = (int16_t)b;
+                S.slot[b] = (int8_t)k;
+            }
         }
+    }
     for (int lp = tid; lp < S.npair; lp += L_T)
         if (S.ppl[lp] >= dn) {
             const int k = atomicAdd(&S.wnP, 1);
@@ -957,260 +987,255 @@ __device__ bool wave_sets(LdsSet &S, int nB, int nBt, int nE, int nEt, int dn)
             const int k = atomicAdd(&S.wnT, 1);
             if (k < 64) S.wT[k] = (int16_t)u;
         }
+    for (int u = tid; u < nE + nEt; u += L_T)
+        if (lds_entry_in_level(S, u, nE, dn)) {
+            const int k = atomicAdd(&S.wnE, 1);
+            if (k < 64) S.wE[k] = (int16_t)u;
+        }
     __syncthreads();
-    if (S.wnB > 64 || S.wnP > 64 || S.wnT > 64) return false;
+    if (S.wnB > 64 || S.wnP > 64 || S.wnT > 64 || S.wnE > 64) return false;
     if (tid < 64) {
-        // each body's entries whose partner is in the level, in entry order
-        const int k = tid;
-        int e0 = 0, e1 = 0, q = 0;
-        bool ispl = true;
-        if (k < S.wnB) {
-            q = S.wB[k];
-            ispl = q < nB;
-            e0 = ispl ? S.pO[q] : nE + S.tO[q - nB];
-            e1 = ispl ? S.pO[q + 1] : nE + S.tO[q - nB + 1];
+        // the entries into entry order: each goes to the place its rank gives
+        const int n = S.wnE, k = tid;
+        const int u = k < n ? S.wE[k] : 0;
+        int r = 0;
+        for (int o = 0; o < n; o++) r += __builtin_amdgcn_readlane(u, o) < u;
+        if (k < S.wnB) S.wEs[k] = S.wEe[k] = 0;
+        wave_sync();
+        if (k < n) S.wE[r] = (int16_t)u;
+        wave_sync();
+        // each body's stretch: from the first to past the last of its entries
+        int b = -1;
+        if (k < n) b = lds_entry_body(S, S.wE[k], nE);
+        const int before = __shfl_up(b, 1, 64), after = __shfl_down(b, 1, 64);
+        if (k < n) {
+            const int sl = S.slot[b];
+            if (k == 0 || before != b) S.wEs[sl] = (int8_t)k;
+            if (k == n - 1 || after != b) S.wEe[sl] = (int8_t)(k + 1);
         }
-        int c = 0;
-        for (int u = e0; u < e1; u++) c += (ispl ? S.plev[S.pE[u] & 511u] : S.plev[S.tpl[u - nE]]) >= dn;
-        int incl = c;
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(incl, o, 64);
-            if (k >= o) incl += t;
-        }
-        const int tot = __shfl(incl, 63, 64);
-        if (tot <= 64) {
-            int w = incl - c;
-            if (k < S.wnB) {
-                S.wEs[k] = (int8_t)w;
-                for (int u = e0; u < e1; u++)
-                    if ((ispl ? S.plev[S.pE[u] & 511u] : S.plev[S.tpl[u - nE]]) >= dn) S.wE[w++] = (int16_t)u;
-                S.wEe[k] = (int8_t)w;
-            }
-        }
-        if (k == 0) S.wnE = tot;
     }
     __syncthreads();
-    return S.wnE <= 64;
+    return true;
 }
 
-// the pair checks of level d (lds_check); returns lenc
-__device__ bool wave_check(LdsSet &S, const SubArgs &A, int d, double dtl)
+// The constants of one lane's roles in a wave-mode recursion: body slot,
+// pl-pl pair, pl-tp pair and kick entry number `lane` of the wave sets.  They
+// do not change while the recursion stays at or below the level the sets
+// were collected at (statuses change only in collision tests, which wave mode
+// does not run), so each phase waits for one LDS read (positions, velocities,
+// levels) instead of walking slot, index and state one after the other.
+// A lane without a role (or with an inactive pair) works on the state slot
+// L_NS, whose level of -1 is never reached, so that no phase needs a mask of
+// the lanes that have one.
+struct WaveLane {
+    int b;                 // body (index in the state arrays)
+    int es, ee;            // its stretch of the kick entries
+    int pi, pj, pl, pv;    // pl-pl pair: its bodies, level and lvdotr
+    double h6i, h6j, rs2;  // rhill * RHSCALE of each, (R_i + R_j)^2
+    int ti, tt, tl, tv;    // pl-tp pair
+    double th6, tR2;
+    int eb, ep;            // kick entry: its body and partner
+    int eu, ev;            // the separation is eu's position minus ev's
+    double s2, gp;         // gp: the partner's mass, with the sign of the term
+};
+
+__device__ inline void wave_load(const LdsSet &S, int nE, int k, WaveLane &W)
 {
-    const int k = threadIdx.x, irec = d + 1;
-    bool lp_enc = false;
-    if (k < S.wnP) {
+    W.pi = W.pj = W.ti = W.tt = W.eb = W.ep = W.eu = W.ev = L_NS;
+    W.pl = W.tl = -9;
+    W.pv = W.tv = 0;
+    W.h6i = W.h6j = W.rs2 = W.th6 = W.tR2 = W.s2 = W.gp = 0.0;
+    W.es = k < S.wnB ? S.wEs[k] : 0;
+    W.ee = k < S.wnB ? S.wEe[k] : 0;
+    if (k < S.wnP && S.pps[S.wP[k]] == ACTIVE) {
         const int lp = S.wP[k];
-        if (S.pps[lp] == ACTIVE && S.ppl[lp] == d) {
-            const int i = S.ppi[lp], j = S.ppj[lp];
-            bool lv;
-            lp_enc = check_pp_v(S.px[i], S.py[i], S.pz[i], S.pvx[i], S.pvy[i], S.pvz[i], S.ph[i], S.pR[i], S.px[j],
-                                S.py[j], S.pz[j], S.pvx[j], S.pvy[j], S.pvz[j], S.ph[j], S.pR[j], irec, dtl, lv);
-            S.ppv[lp] = lv;
-            if (lp_enc) {
-                S.ppl[lp] = (int8_t)irec;
-                S.plev[i] = irec;
-                S.plev[j] = irec;
-                atomicMax(&S.plm[i], irec);
-                atomicMax(&S.plm[j], irec);
-            }
-        }
+        W.pi = S.ppi[lp];
+        W.pj = S.ppj[lp];
+        W.pl = S.ppl[lp];
+        W.pv = S.ppv[lp];
+        W.h6i = S.ph[W.pi] * RHSCALE;
+        W.h6j = S.ph[W.pj] * RHSCALE;
+        const double rs = S.pR[W.pi] + S.pR[W.pj];
+        W.rs2 = rs * rs;
     }
-    const bool fpp = __ballot(lp_enc) != 0;
-    wave_sync();
-    bool tp_enc = false;
-    if (!(A.short_circuit && fpp) && k < S.wnT) {  // symba_step.f90:210 (.or. short-circuited)
+    if (k < S.wnT && S.tps[S.wT[k]] == ACTIVE) {
         const int u = S.wT[k];
-        if (S.tps[u] == ACTIVE && S.tpl_lev[u] == d) {
-            const int i = S.tpl[u], t = S.tpt[u];
-            bool lv;
-            tp_enc = check_pt_v(S.px[i], S.py[i], S.pz[i], S.pvx[i], S.pvy[i], S.pvz[i], S.ph[i], S.pR[i], S.tx[t],
-                                S.ty[t], S.tz[t], S.tvx[t], S.tvy[t], S.tvz[t], irec, dtl, lv);
-            S.tpv[u] = lv;
-            if (tp_enc) {
-                S.tpl_lev[u] = (int8_t)irec;
-                S.plev[i] = irec;
-                atomicMax(&S.plm[i], irec);
-                S.tlev[t] = irec;
-                atomicMax(&S.tlm[t], irec);
-            }
-        }
+        W.ti = S.tpl[u];
+        W.tt = L_NB + S.tpt[u];
+        W.tl = S.tpl_lev[u];
+        W.tv = S.tpv[u];
+        W.th6 = S.ph[W.ti] * RHSCALE;
+        W.tR2 = S.pR[W.ti] * S.pR[W.ti];
     }
-    const bool fpt = __ballot(tp_enc) != 0;
-    wave_sync();
-    return fpp || fpt;
-}
-
-// the +1 / -1 shell kicks of level d (lds_kicks).  mode 0: evaluate; 1:
-// evaluate and keep the sums in c; 2: apply the sums kept in c.
-__device__ void wave_kicks(LdsSet &S, int nB, int nE, int d, double dth, int mode, KCache &c)
-{
-    const int k = threadIdx.x;
-    if (mode == 2) {
-        if (k < S.wnB) {
-            const int q = S.wB[k];
-            const bool ispl = q < nB;
-            if ((ispl ? S.plev[q] : S.tlev[q - nB]) >= d) {
-                if (ispl) lds_apply(S.pvx[q], S.pvy[q], S.pvz[q], dth, (c.fl & 1) != 0, c.p, (c.fl & 2) != 0, c.m);
-                else
-                    lds_apply(S.tvx[q - nB], S.tvy[q - nB], S.tvz[q - nB], dth, (c.fl & 1) != 0, c.p, (c.fl & 2) != 0,
-                              c.m);
-            }
-        }
-        wave_sync();
-        return;
-    }
-    const double spp = shell_sq(d + 1), spm = shell_sq(d);
     if (k < S.wnE) {
-        const int u = S.wE[k];
-        ShellTerm t;
-        t.tp = t.tm = false;
-        t.dx = t.dy = t.dz = 0.0;
+        const int u = S.wE[k], eb = lds_entry_body(S, u, nE);
+        int ep;
+        bool bi = false, on;  // bi: the body is index1 of its pair
         if (u < nE) {
             const uint32_t e = S.pE[u];
-            const int lp = (int)(e >> 10), pr = (int)(e & 511u);
-            const bool bi = (e >> 9) & 1u;
-            const int q = bi ? S.ppi[lp] : S.ppj[lp];
-            if (S.plev[q] >= d && S.plev[pr] >= d && S.pps[lp] == ACTIVE)
-                pl_shell_term_v(bi, S.px[q], S.py[q], S.pz[q], S.ph[q], S.px[pr], S.py[pr], S.pz[pr], S.ph[pr],
-                                S.pgm[pr], spp, spm, true, t);
+            ep = (int)(e & 511u);
+            bi = (e >> 9) & 1u;
+            on = S.pps[e >> 10] == ACTIVE;
+            const double hb = S.ph[eb], hp = S.ph[ep];
+            const double sh = bi ? hb + hp : hp + hb;
+            W.s2 = (sh * sh) * (RHSCALE * RHSCALE);
         } else {
-            const int v = u - nE, i = S.tpl[v], tt = S.tpt[v];
-            if (S.tlev[tt] >= d && S.plev[i] >= d && S.tps[v] == ACTIVE)
-                tp_shell_term_v(S.tx[tt], S.ty[tt], S.tz[tt], S.px[i], S.py[i], S.pz[i], S.ph[i], S.pgm[i], spp, spm,
-                                true, t);
+            ep = S.tpl[u - nE];
+            on = S.tps[u - nE] == ACTIVE;
+            const double h = S.ph[ep];
+            W.s2 = (h * h) * (RHSCALE * RHSCALE);
         }
-        KTerm &K = S.kt[k];
-        K.dx = t.dx;
-        K.dy = t.dy;
-        K.dz = t.dz;
-        K.fp = t.tp ? t.fp : 0.0;
-        K.fm = t.tm ? t.fm : 0.0;
-        K.fl = (t.tp ? 1 : 0) | (t.tm ? 2 : 0);
-    }
-    wave_sync();
-    if (k < S.wnB) {
-        const int q = S.wB[k];
-        const bool ispl = q < nB;
-        if ((ispl ? S.plev[q] : S.tlev[q - nB]) >= d) {
-            double3 p = make_double3(0.0, 0.0, 0.0), m = p;
-            int fl = 0;
-            fold_terms(S.kt, S.wEs[k], S.wEe[k], p, m, fl);
-            if (ispl) lds_apply(S.pvx[q], S.pvy[q], S.pvz[q], dth, (fl & 1) != 0, p, (fl & 2) != 0, m);
-            else lds_apply(S.tvx[q - nB], S.tvy[q - nB], S.tvz[q - nB], dth, (fl & 1) != 0, p, (fl & 2) != 0, m);
-            if (mode == 1) {
-                c.p = p;
-                c.m = m;
-                c.fl = fl;
-            }
+        if (on) {
+            // pl_shell_term_v / tp_shell_term_v: the separation runs from
+            // index1 to index2, from the massive body to the particle, and
+            // the partner's mass enters with + on index1 alone
+            W.eb = eb;
+            W.ep = ep;
+            W.eu = bi ? ep : eb;
+            W.ev = bi ? eb : ep;
+            W.gp = bi ? S.pgm[ep] : -S.pgm[ep];
         }
     }
-    wave_sync();
 }
 
-// The drifts of level d (lds_drift), called by the whole workgroup.  A
-// wavefront runs a bound body's series solution (kepmd) and an unbound one's
-// iteration (kepu) one after the other, so the first wavefront keeps the bodies
-// that look bound and hands the others to the second, and the two drift side
-// by side.  The test only places the work (each drift is drift_one either
-// way): alpha > 0 of drift_dan is 2 mu / r0 > v0^2, taken here without the
-// square root and division as 4 mu^2 > v0^4 r0^2.
-// Returns S.wlenc, read between the two barriers (it is rewritten only after
-// the second).
-__device__ bool wave_drift(LdsSet &S, const SubArgs &A, int nB, int d, double dtl, int s)
+// pair states back to the slice
+__device__ inline void wave_store(LdsSet &S, int k, const WaveLane &W)
 {
-    const int tid = threadIdx.x;
-    const double mu = A.st.sy.GMcb[s];
-    bool on = false, far = false;
-    int q = 0;
-    if (tid < 64) {
-        if (tid < S.wnB) {
-            q = S.wB[tid];
-            const bool ispl = q < nB;
-            const int t = q - nB;
-            on = ispl ? (S.pst[q] != INACTIVE && S.plev[q] == d) : (S.tst[t] == ACTIVE && S.tlev[t] == d);
-            if (on) {
-                const double rx = ispl ? S.px[q] : S.tx[t], ry = ispl ? S.py[q] : S.ty[t], rz = ispl ? S.pz[q] : S.tz[t];
-                const double vx = ispl ? S.pvx[q] : S.tvx[t], vy = ispl ? S.pvy[q] : S.tvy[t],
-                             vz = ispl ? S.pvz[q] : S.tvz[t];
-                const double v2 = dot3(vx, vy, vz, vx, vy, vz);
-                far = !(4.0 * mu * mu > (v2 * v2) * dot3(rx, ry, rz, rx, ry, rz));
-            }
-        }
-        const uint64_t m = __ballot(far);
-        if (far) S.wH[__popcll(m & ((1ull << tid) - 1))] = (int8_t)tid;
-        if (tid == 0) S.wnH = __popcll(m);
+    if (W.pi != L_NS) {
+        S.ppl[S.wP[k]] = (int8_t)W.pl;
+        S.ppv[S.wP[k]] = (int8_t)W.pv;
     }
-    __syncthreads();
-    const bool lenc = S.wlenc != 0;
-    int k = -1;
-    if (tid < 64) {
-        if (on && !far) k = tid;
-    } else if (tid < 128 && tid - 64 < S.wnH) {
-        k = S.wH[tid - 64];
-        q = S.wB[k];
+    if (W.ti != L_NS) {
+        S.tpl_lev[S.wT[k]] = (int8_t)W.tl;
+        S.tpv[S.wT[k]] = (int8_t)W.tv;
     }
-    if (k >= 0) {
-        const bool ispl = q < nB;
-        const int t = q - nB;
-        double *x = ispl ? S.px : S.tx, *y = ispl ? S.py : S.ty, *z = ispl ? S.pz : S.tz;
-        double *vx = ispl ? S.pvx : S.tvx, *vy = ispl ? S.pvy : S.tvy, *vz = ispl ? S.pvz : S.tvz;
-        const int i = ispl ? q : t;
-        double rx = x[i], ry = y[i], rz = z[i], ux = vx[i], uy = vy[i], uz = vz[i];
-        const int fl = drift_one(mu, rx, ry, rz, ux, uy, uz, dtl);
-        x[i] = rx;
-        y[i] = ry;
-        z[i] = rz;
-        vx[i] = ux;
-        vy[i] = uy;
-        vz[i] = uz;
-        if (fl) {
-            if (ispl) {
-                S.pst[q] = DISCARDED_DRIFTERR;
-                atomicOr(&A.st.sy.err[s], 2);
-            } else {
-                S.tst[t] = DISCARDED_DRIFTERR;
-            }
-        }
-    }
-    __syncthreads();
-    return lenc;
 }
 
-// the level reset after a substep of level d (lds_set_levels)
-__device__ void wave_set_levels(LdsSet &S, int nB, int d)
+// The sums of the terms [u, hi), in order (fold_terms for few terms per body):
+// four are read at once, the ones past the end as zeros.
+__device__ inline void wave_fold(const KTerm *kt, int u, int hi, KCache &c)
 {
-    const int k = threadIdx.x, irecp = d + 1;
-    if (k < S.wnB) {
-        const int q = S.wB[k];
-        if (q < nB) {
-            if (S.plev[q] == irecp) S.plev[q] = d;
-        } else if (S.tlev[q - nB] == irecp) {
-            S.tlev[q - nB] = d;
+    c.p = c.m = make_double3(0.0, 0.0, 0.0);
+    c.fl = 0;
+    do {
+        KTerm a[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) a[q] = kt[min(u + q, 63)];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const bool on = u + q < hi;
+            const double fp = on ? a[q].fp : 0.0, fm = on ? a[q].fm : 0.0;
+            c.p.x = fma(fp, a[q].dx, c.p.x);
+            c.p.y = fma(fp, a[q].dy, c.p.y);
+            c.p.z = fma(fp, a[q].dz, c.p.z);
+            c.m.x = fma(fm, a[q].dx, c.m.x);
+            c.m.y = fma(fm, a[q].dy, c.m.y);
+            c.m.z = fma(fm, a[q].dz, c.m.z);
+            c.fl |= on ? a[q].fl : 0;
         }
-    }
-    if (k < S.wnP && S.ppl[S.wP[k]] == irecp) S.ppl[S.wP[k]] = (int8_t)d;
-    if (k < S.wnT && S.tpl_lev[S.wT[k]] == irecp) S.tpl_lev[S.wT[k]] = (int8_t)d;
-    wave_sync();
+        u += 4;
+    } while (u < hi);
+}
+
+// lds_apply of the sums in c to body b, by selection
+__device__ inline void wave_apply(LdsSet &S, int b, double dth, const KCache &c)
+{
+    double vx = S.pvx[b], vy = S.pvy[b], vz = S.pvz[b];
+    const bool ap = (c.fl & 1) != 0, am = (c.fl & 2) != 0;
+    vx = ap ? fma(dth, c.p.x, vx) : vx;
+    vy = ap ? fma(dth, c.p.y, vy) : vy;
+    vz = ap ? fma(dth, c.p.z, vz) : vz;
+    S.pvx[b] = am ? fma(-dth, c.m.x, vx) : vx;
+    S.pvy[b] = am ? fma(-dth, c.m.y, vy) : vy;
+    S.pvz[b] = am ? fma(-dth, c.m.z, vz) : vz;
+}
+
+// encounter_one and the physical-overlap exclusion for the relative motion of
+// body j with respect to i, without branches: every quotient is formed and the
+// reference's case selected.
+__device__ inline bool wave_encounter(const LdsSet &S, int i, int j, double renc, double rs2, double dtl, bool &lv)
+{
+    const double xr = S.px[j] - S.px[i], yr = S.py[j] - S.py[i], zr = S.pz[j] - S.pz[i];
+    const double vxr = S.pvx[j] - S.pvx[i], vyr = S.pvy[j] - S.pvy[i], vzr = S.pvz[j] - S.pvz[i];
+    const double r2 = dot3(xr, yr, zr, xr, yr, zr), r2crit = renc * renc;
+    const double vdotr = dot3(vxr, vyr, vzr, xr, yr, zr), v2 = dot3(vxr, vyr, vzr, vxr, vyr, vzr);
+    const double tmin = -vdotr / v2;
+    const double near = r2 - (vdotr * vdotr) / v2, end = (r2 + (2.0 * vdotr) * dtl) + v2 * (dtl * dtl);
+    const bool out = r2 > r2crit;
+    const bool moving = out & !(vdotr > 0.0) & !(v2 <= VSMALL);
+    const double r2min = moving ? (tmin < dtl ? near : end) : r2;
+    lv = !out | (vdotr < 0.0);
+    return lv & (r2min <= r2crit) & (r2 > rs2);
 }
 
 // Levels dw and below in wave mode, from the first substep of dw to the end
-// of dw (the loop of k_subtree_lds), called by the whole workgroup: the first
-// wavefront runs the checks, kicks and level resets, the drifts take the
-// second one as well, and the others only follow the loop.  Adds its substeps
-// to nsub and raises maxd; sets S.wstop when the recursion must stop (error
-// flagged).
-__device__ void wave_recursion(LdsSet &S, const SubArgs &A, int nB, int nE, int dw, int s, int &nsub, int &maxd)
+// of dw (the loop of k_subtree_lds), called by the whole workgroup.  The
+// first wavefront runs the checks, kicks and level resets.  The drifts take
+// all of them: a wavefront runs a bound body's series solution (kepmd) and an
+// unbound one's iteration (kepu) one after the other, so the bodies that look
+// bound drift on the first wavefront and the others on the rest, side by
+// side.  The test only places the work (each drift is drift_one either way):
+// alpha > 0 of drift_dan is 2 mu / r0 > v0^2, taken here without the square
+// root and division as 4 mu^2 > v0^4 r0^2.
+//
+// One wavefront's serial chain is all there is to run here, so its
+// instructions and LDS round trips are the time: a substep of about ten
+// bodies takes 3.7 us (check 0.4, opening kicks 0.35, drift 1.6-2.9, closing
+// kicks 0.8), against 6.9 us with the indices walked through LDS in every
+// phase, branches around each role and both cube roots of an unbound drift on
+// one lane; four steps of a 1024-body system among four, 117 ms instead of
+// 182.  The function is kept out of the kernel's body: inlined there, the
+// kernel's many pointers spill its scalars and addresses (154 ms).  Returns the substeps taken and the deepest level;
+// sets S.wstop when the recursion must stop (error flagged).
+__device__ __attribute__((noinline)) int2 wave_recursion(int nE, int dw, double mu, int short_circuit, int32_t *err,
+                                                         int prof_on)
 {
-    const bool w0 = threadIdx.x < 64;
-    const bool prof = A.prof && threadIdx.x == 0;
-    int d = dw, j = 1;
+    LdsSet &S = s_lds;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const bool w0 = wv == 0, prof = prof_on && threadIdx.x == 0;
+    int d = dw, j = 1, nsub = 0, maxd = dw;
     bool resume = false;
-    KCache kc{};
-    int kcd = -1;  // the level whose closing-kick sums kc holds (-1: none)
+    KCache c{};
+    int kcd = -1;       // the level whose closing-kick sums c holds (-1: none)
+    int ktop = dw - 1;  // the highest level whose shell radii S.shr holds
+    WaveLane W;
+    const int b = W.b = lane < S.wnB ? S.wB[lane] : L_NS;
+    const bool tps = S.wnT > 0;
+    const int dmax = min(S.dmax, MAXLEV);
+    if (w0) wave_load(S, nE, lane, W);
+    int dl = -1;  // the level the next five belong to
+    double dtl = 0.0, dth = 0.0, rsh = 0.0, sqp = 0.0, sqm = 0.0;
+    // shell-kick sums of level d for the body of this lane, into c
+    auto evaluate = [&]() __attribute__((always_inline)) {
+        for (; ktop < d + 1; ktop++) S.shr[ktop + 1 - dw][lane] = sqrt(W.s2 * S.ssq[ktop + 1]);
+        const bool in = min(S.plev[W.eb], S.plev[W.ep]) >= d;
+        const double sp = S.shr[d + 1 - dw][lane], sm = S.shr[d - dw][lane];
+        KTerm t;
+        t.dx = S.px[W.eu] - S.px[W.ev];
+        t.dy = S.py[W.eu] - S.py[W.ev];
+        t.dz = S.pz[W.eu] - S.pz[W.ev];
+        const double r2 = dot3(t.dx, t.dy, t.dz, t.dx, t.dy, t.dz);
+        bool okp, okm;
+        double fp, fm;
+        shell_facs_at(W.s2 * sqp, W.s2 * sqm, sp, sm, r2, true, okp, fp, okm, fm);
+        okp &= in;
+        okm &= in;
+        t.fp = okp ? fp * W.gp : 0.0;
+        t.fm = okm ? fm * W.gp : 0.0;
+        t.fl = (okp ? 1 : 0) | (okm ? 2 : 0);
+        S.kt[lane] = t;
+        wave_sync();
+        wave_fold(S.kt, W.es, W.ee, c);
+    };
     for (;;) {
-        double p3 = 1.0;
-        for (int q = 0; q < d; q++) p3 *= NTENC;
-        const double dtl = A.dt / p3, dth = 0.5 * dtl;
+        if (dl != d) {
+            dl = d;
+            dtl = S.dtl[d];
+            rsh = S.rsh[d + 1];
+            sqp = S.ssq[d + 1];
+            sqm = S.ssq[d];
+            dth = 0.5 * dtl;
+        }
         if (!resume) {
             if (j > NTENC) {
                 if (d == dw) break;
@@ -1219,9 +1244,9 @@ __device__ void wave_recursion(LdsSet &S, const SubArgs &A, int nB, int nE, int 
                 resume = true;
                 continue;
             }
-            if (dtl / A.dt < 2.220446049250313e-16) {  // symba_step.f90:196-201
+            if (d > dmax) {  // symba_step.f90:196-201, or past the level stack
                 if (threadIdx.x == 0) {
-                    atomicOr(&A.st.sy.err[s], 8);
+                    atomicOr(err, 8);
                     S.wstop = 1;
                 }
                 break;
@@ -1229,14 +1254,95 @@ __device__ void wave_recursion(LdsSet &S, const SubArgs &A, int nB, int nE, int 
             nsub++;
             const unsigned long long t0 = prof ? wall_clock64() : 0;
             if (w0) {
-                const bool le = wave_check(S, A, d, dtl);
-                if (threadIdx.x == 0) S.wlenc = le;
+                // the pair checks of level d (lds_check)
+                const int irec = d + 1;
+                bool lv;
+                bool enc = wave_encounter(S, W.pi, W.pj, W.h6i * rsh + W.h6j * rsh, W.rs2, dtl, lv);
+                const bool mine = W.pl == d;
+                enc &= mine;
+                W.pv = mine ? (int)lv : W.pv;
+                if (enc) {
+                    W.pl = irec;
+                    S.plev[W.pi] = irec;
+                    S.plev[W.pj] = irec;
+                    atomicMax(&S.plm[W.pi], irec);
+                    atomicMax(&S.plm[W.pj], irec);
+                }
+                bool any = __ballot(enc) != 0;
+                wave_sync();
+                if (tps && !(short_circuit && any)) {  // symba_step.f90:210 (.or. short-circuited)
+                    enc = wave_encounter(S, W.ti, W.tt, W.th6 * rsh, W.tR2, dtl, lv);
+                    const bool mt = W.tl == d;
+                    enc &= mt;
+                    W.tv = mt ? (int)lv : W.tv;
+                    if (enc) {
+                        W.tl = irec;
+                        S.plev[W.ti] = irec;
+                        atomicMax(&S.plm[W.ti], irec);
+                        S.plev[W.tt] = irec;
+                        atomicMax(&S.plm[W.tt], irec);
+                    }
+                    any |= __ballot(enc) != 0;
+                    wave_sync();
+                }
+                if (threadIdx.x == 0) S.wlenc = any;
             }
             const unsigned long long t1 = prof ? wall_clock64() : 0;
-            if (w0) wave_kicks(S, nB, nE, d, dth, kcd == d ? 2 : 0, kc);
+            if (w0) {
+                // the opening kicks, from the closing kicks before them where
+                // those were at this level
+                // (a body below level d has only unflagged zero terms)
+                if (kcd != d) evaluate();
+                wave_apply(S, b, dth, c);
+            }
             kcd = -1;
             const unsigned long long t2 = prof ? wall_clock64() : 0;
-            const bool lenc = wave_drift(S, A, nB, d, dtl, s);
+            __syncthreads();
+            // the drifts of level d (lds_drift)
+            const bool lenc = S.wlenc != 0;
+            {
+                double rx = S.px[b], ry = S.py[b], rz = S.pz[b], vx = S.pvx[b], vy = S.pvy[b], vz = S.pvz[b];
+                const int st = S.pst[b];
+                const bool on = S.plev[b] == d && (b < L_NB ? st != INACTIVE : st == ACTIVE);
+                const double v2 = dot3(vx, vy, vz, vx, vy, vz);
+                const bool far = !(4.0 * mu * mu > (v2 * v2) * dot3(rx, ry, rz, rx, ry, rz));
+                const uint64_t mf = __ballot(on && far);
+                const int rank = __popcll(mf & ((1ull << lane) - 1));
+                __syncthreads();  // every wavefront has placed the bodies before any moves one
+                // wavefronts 1, 2, ... take every third unbound-looking body,
+                // each on two lanes 32 apart, whose cube roots drift_one
+                // shares out; at most 22 bodies each
+                int q = b;
+                bool run = on && !far;
+                if (!w0) {
+                    constexpr int NF = L_T / 64 - 1;
+                    static_assert((64 + NF - 1) / NF <= 32, "a wavefront's bodies fit its lower lanes");
+                    if (on && far && rank % NF == wv - 1) S.wH[wv][rank / NF] = (int16_t)b;
+                    wave_sync();
+                    const int n = (__popcll(mf) + NF - wv) / NF, l = lane & 31;
+                    run = l < n;
+                    if (run) {
+                        q = S.wH[wv][l];
+                        rx = S.px[q], ry = S.py[q], rz = S.pz[q], vx = S.pvx[q], vy = S.pvy[q], vz = S.pvz[q];
+                    }
+                }
+                if (run) {
+                    const int fl = drift_one(mu, rx, ry, rz, vx, vy, vz, dtl, !w0);
+                    if (w0 || lane < 32) {
+                        S.px[q] = rx;
+                        S.py[q] = ry;
+                        S.pz[q] = rz;
+                        S.pvx[q] = vx;
+                        S.pvy[q] = vy;
+                        S.pvz[q] = vz;
+                        if (fl) {
+                            S.pst[q] = DISCARDED_DRIFTERR;
+                            if (q < L_NB) atomicOr(err, 2);
+                        }
+                    }
+                }
+            }
+            __syncthreads();
             if (prof) {
                 unsigned long long *P = S.prof + d * NPROF;
                 P[0] += 1;
@@ -1247,39 +1353,38 @@ __device__ void wave_recursion(LdsSet &S, const SubArgs &A, int nB, int nE, int 
                 P[5] += wall_clock64() - t2;
             }
             if (lenc) {
-                if (d + 1 > MAXLEV) {
-                    if (threadIdx.x == 0) {
-                        atomicOr(&A.st.sy.err[s], 8);
-                        S.wstop = 1;
-                    }
-                    break;
-                }
                 if (threadIdx.x == 0) S.jst[d] = j;
-                wave_sync();
                 d++;
-                if (d > maxd) maxd = d;
+                if (d > maxd && d <= MAXLEV) maxd = d;
                 j = 1;
                 continue;
             }
         }
         resume = false;
         const unsigned long long t0 = prof ? wall_clock64() : 0;
-        if (w0) wave_kicks(S, nB, nE, d, dth, 1, kc);
-        kcd = d;
-        const unsigned long long t1 = prof ? wall_clock64() : 0;
-        if (w0) wave_set_levels(S, nB, d);
-        if (prof) {
-            S.prof[d * NPROF + 6] += t1 - t0;
-            S.prof[d * NPROF + 7] += wall_clock64() - t1;
+        if (w0) {
+            // the closing kicks, and the level reset after them
+            // (lds_set_levels)
+            evaluate();
+            wave_apply(S, b, dth, c);
+            const int lev = S.plev[b];
+            if (lev == d + 1) S.plev[b] = d;
+            if (W.pl == d + 1) W.pl = d;
+            if (W.tl == d + 1) W.tl = d;
+            wave_sync();
         }
+        kcd = d;
+        if (prof) S.prof[d * NPROF + 6] += wall_clock64() - t0;
         j++;
     }
+    if (w0) wave_store(S, lane, W);
+    return make_int2(nsub, maxd);
 }
 
 __global__ __launch_bounds__(L_T) void k_subtree_lds(const SubArgs A)
 {
     const RecState &a = A.st;
-    __shared__ LdsSet S;
+    LdsSet &S = s_lds;
     const int s = blockIdx.x;
     const int tid = threadIdx.x;
     const int32_t *r = A.rng + 4 * s;
@@ -1289,7 +1394,19 @@ __global__ __launch_bounds__(L_T) void k_subtree_lds(const SubArgs A)
     const int32_t *gBt = A.start.Bt + r[2], *gOt = A.start.Ot + r[2];
     const int e0 = gO[0], nE = gO[nB] - e0, et0 = gOt[0], nEt = gOt[nBt] - et0;
     if (!A.lds || !lds_eligible(nB, nE, nBt, nEt)) return;
+    const double mu = a.sy.GMcb[s];
     // ---- load the slice ----
+    if (tid == 0) S.dmax = 0;
+    __syncthreads();
+    if (tid < MAXLEV + 2) {
+        double p3 = 1.0;
+        for (int q = 0; q < tid; q++) p3 *= NTENC;
+        const double dtl = A.dt / p3;
+        S.dtl[tid] = dtl;
+        S.ssq[tid] = shell_sq(tid);
+        S.rsh[tid] = shell_r(tid);
+        if (!(dtl / A.dt < 2.220446049250313e-16)) atomicMax(&S.dmax, tid);
+    }
     for (int q = tid; q < nB; q += L_T) {
         const int g = gB[q];
         S.pg[q] = g;
@@ -1310,18 +1427,21 @@ __global__ __launch_bounds__(L_T) void k_subtree_lds(const SubArgs A)
     for (int q = tid; q < nBt; q += L_T) {
         const int g = gBt[q];
         S.tg[q] = g;
-        S.tx[q] = a.tp.rh.x[g];
-        S.ty[q] = a.tp.rh.y[g];
-        S.tz[q] = a.tp.rh.z[g];
-        S.tvx[q] = a.tp.vb.x[g];
-        S.tvy[q] = a.tp.vb.y[g];
-        S.tvz[q] = a.tp.vb.z[g];
-        S.tlev[q] = a.tp.levelg[g];
-        S.tlm[q] = a.tp.levelm[g];
-        S.tst[q] = a.tp.status[g];
+        S.px[L_NB + q] = a.tp.rh.x[g];
+        S.py[L_NB + q] = a.tp.rh.y[g];
+        S.pz[L_NB + q] = a.tp.rh.z[g];
+        S.pvx[L_NB + q] = a.tp.vb.x[g];
+        S.pvy[L_NB + q] = a.tp.vb.y[g];
+        S.pvz[L_NB + q] = a.tp.vb.z[g];
+        S.plev[L_NB + q] = a.tp.levelg[g];
+        S.plm[L_NB + q] = a.tp.levelm[g];
+        S.pst[L_NB + q] = a.tp.status[g];
         S.tO[q] = gOt[q] - et0;
     }
     if (tid == 0) {
+        S.px[L_NS] = S.py[L_NS] = S.pz[L_NS] = S.pvx[L_NS] = S.pvy[L_NS] = S.pvz[L_NS] = 0.0;
+        S.plev[L_NS] = S.plm[L_NS] = -1;
+        S.pst[L_NS] = ACTIVE;
         S.pO[nB] = nE;
         S.tO[nBt] = nEt;
         S.npair = 0;
@@ -1467,9 +1587,7 @@ __global__ __launch_bounds__(L_T) void k_subtree_lds(const SubArgs A)
     KCache kc[L_KS];
     int kcd = -1;  // the level whose closing-kick sums kc holds (-1: none)
     for (;;) {
-        double p3 = 1.0;
-        for (int q = 0; q < d; q++) p3 *= NTENC;
-        const double dtl = A.dt / p3, dth = 0.5 * dtl;
+        const double dtl = S.dtl[d], dth = 0.5 * dtl;
         if (!resume) {
             if (j > NTENC) {  // level finished
                 if (d == d0) break;
@@ -1478,7 +1596,7 @@ __global__ __launch_bounds__(L_T) void k_subtree_lds(const SubArgs A)
                 resume = true;
                 continue;
             }
-            if (dtl / A.dt < 2.220446049250313e-16) {  // symba_step.f90:196-201
+            if (d > S.dmax) {  // symba_step.f90:196-201
                 if (tid == 0) atomicOr(&a.sy.err[s], 8);
                 break;
             }
@@ -1490,7 +1608,7 @@ __global__ __launch_bounds__(L_T) void k_subtree_lds(const SubArgs A)
             lds_kicks(S, nB, nBt, nE, nEt, d, dth, A.prof != nullptr, kcd == d ? 2 : 0, kc);
             kcd = -1;
             if (prof) t2 = wall_clock64();
-            lds_drift(S, A, nB, nBt, d, dtl, s, A.prof != nullptr);
+            lds_drift(S, A, nB, nBt, d, dtl, mu, s, A.prof != nullptr);
             if (prof) {
                 t3 = wall_clock64();
                 unsigned long long *P = S.prof + d * NPROF;
@@ -1520,7 +1638,9 @@ __global__ __launch_bounds__(L_T) void k_subtree_lds(const SubArgs A)
                 if (!A.lclose && A.wave && wave_sets(S, nB, nBt, nE, nEt, d)) {
                     // level d and below on the first wavefront; then level d
                     // is finished and the workgroup resumes level d - 1
-                    wave_recursion(S, A, nB, nE, d, s, nsub, maxd);
+                    const int2 r = wave_recursion(nE, d, mu, A.short_circuit, &a.sy.err[s], A.prof != nullptr);
+                    nsub += r.x;
+                    maxd = max(maxd, r.y);
                     __syncthreads();
                     if (S.wstop) break;
                     j = NTENC + 1;

@@ -298,8 +298,11 @@ __host__ __device__ inline double pow_third(double x)
     return pow_third_core(x);
 }
 
-// real root of the cubic for the hyperbolic first guess (:486-533)
-__device__ inline int kepu_p3solve(double dt, double r0, double mu, double alpha, double u, double &s)
+// real root of the cubic for the hyperbolic first guess (:486-533).  mirror:
+// lanes k and k + 32 of the wavefront hold the same body, and each takes one
+// of its two cube roots (a lane's two run one after the other, about 500
+// cycles each).
+__device__ inline int kepu_p3solve(double dt, double r0, double mu, double alpha, double u, double &s, bool mirror)
 {
     double denom = (mu - alpha * r0) * SIXTH;
     double a2 = (0.5 * u) / denom;
@@ -312,7 +315,16 @@ __device__ inline int kepu_p3solve(double dt, double r0, double mu, double alpha
         double sq = sqrt(sq2);
         // t <= 0 ? -(-t)**THIRD : t**THIRD, with -t == |t| in the first arm
         const double t1 = r + sq, t2 = r - sq;
-        const double w1 = pow_third(fabs(t1)), w2 = pow_third(fabs(t2));
+        double w1, w2;
+        if (mirror) {
+            const bool up = (threadIdx.x & 32u) != 0;
+            const double w = pow_third(fabs(up ? t2 : t1)), o = __shfl_xor(w, 32, 64);
+            w1 = up ? o : w;
+            w2 = up ? w : o;
+        } else {
+            w1 = pow_third(fabs(t1));
+            w2 = pow_third(fabs(t2));
+        }
         double p1 = (t1 <= 0.0) ? -w1 : w1;
         double p2 = (t2 <= 0.0) ? -w2 : w2;
         s = (p1 + p2) - a2 * THIRD;
@@ -323,7 +335,7 @@ __device__ inline int kepu_p3solve(double dt, double r0, double mu, double alpha
 }
 
 // initial guess (:337-378)
-__device__ inline double kepu_guess(double dt, double r0, double mu, double alpha, double u)
+__device__ inline double kepu_guess(double dt, double r0, double mu, double alpha, double u, bool mirror)
 {
     double s;
     if (alpha > 0.0) {
@@ -343,7 +355,7 @@ __device__ inline double kepu_guess(double dt, double r0, double mu, double alph
             s = x / sqrt(alpha);
         }
     } else {
-        if (kepu_p3solve(dt, r0, mu, alpha, u, s) != 0) s = dt / r0;
+        if (kepu_p3solve(dt, r0, mu, alpha, u, s, mirror) != 0) s = dt / r0;
     }
     return s;
 }
@@ -398,7 +410,7 @@ __device__ inline int kepu_lag(double &s, double dt, double r0, double mu, doubl
 
 // one Danby drift of (r, v) over dt0 (:141-231); returns iflag
 __device__ __attribute__((always_inline)) inline int drift_dan(double mu, double &rx0, double &ry0, double &rz0, double &vx0, double &vy0,
-                                double &vz0, double dt0)
+                                double &vz0, double dt0, bool mirror)
 {
     double dt = dt0;
     double r0 = sqrt(dot3(rx0, ry0, rz0, rx0, ry0, rz0));
@@ -432,7 +444,7 @@ __device__ __attribute__((always_inline)) inline int drift_dan(double mu, double
             return 0;
         }
     }
-    double s = kepu_guess(dt, r0, mu, alpha, u);
+    double s = kepu_guess(dt, r0, mu, alpha, u, mirror);
     double st = s, fp, c1, c2, c3;
     int iflag = kepu_new(s, dt, r0, mu, alpha, u, fp, c1, c2, c3);
     if (iflag != 0) {
@@ -457,14 +469,15 @@ __device__ __attribute__((always_inline)) inline int drift_dan(double mu, double
 // swiftest_drift_one (:111-138): on failure retry as ten dt/10 substeps,
 // stopping at the first substep that fails.  Written with a single call of
 // drift_dan so that the compiler inlines it (a call would save and restore
-// the caller's live registers around every drift).
+// the caller's live registers around every drift).  mirror (kepu_p3solve):
+// the caller runs each body on lanes k and k + 32.
 __device__ inline int drift_one(double mu, double &rx, double &ry, double &rz, double &vx, double &vy, double &vz,
-                                double dt)
+                                double dt, bool mirror = false)
 {
     double h = dt;
     int i = -1, fl;
     for (;;) {
-        fl = drift_dan(mu, rx, ry, rz, vx, vy, vz, h);
+        fl = drift_dan(mu, rx, ry, rz, vx, vy, vz, h, mirror);
         if (i < 0) {  // the full step
             if (fl == 0) break;
             h = 0.1 * dt;
@@ -610,13 +623,13 @@ __host__ __device__ inline double pow_m1p5(double x)
 // forms are computed for both radii and selected, with no branch: the two
 // shells' chains then overlap, and sqrt(r2) and r2^-1.5 are formed once.
 // Each selected factor is the expression the reference evaluates for it.
-__device__ inline void shell_facs(double rp, double rm, double r2, bool minus, bool &okp, double &facp, bool &okm,
-                                  double &facm)
+// shell_facs_at takes the shell radii sp = sqrt(rp), sm = sqrt(rm) as well.
+__device__ inline void shell_facs_at(double rp, double rm, double sp, double sm, double r2, bool minus, bool &okp,
+                                     double &facp, bool &okm, double &facm)
 {
     const double r = sqrt(r2);
     const double out = 1.0 / (r2 * r);
     const double p15 = pow_m1p5(r2);
-    const double sp = sqrt(rp), sm = sqrt(rm);
     const double rrp = (sp - r) / (sp * (1.0 - RSHELL)), rrm = (sm - r) / (sm * (1.0 - RSHELL));
     const double inp = p15 * ((1.0 - 3.0 * (rrp * rrp)) + 2.0 * ((rrp * rrp) * rrp));
     const double inm = p15 * ((1.0 - 3.0 * (rrm * rrm)) + 2.0 * ((rrm * rrm) * rrm));
@@ -624,6 +637,12 @@ __device__ inline void shell_facs(double rp, double rm, double r2, bool minus, b
     okm = minus && !(r2 < rm * (RSHELL * RSHELL));
     facp = r2 < rp ? inp : out;
     facm = r2 < rm ? inm : out;
+}
+
+__device__ inline void shell_facs(double rp, double rm, double r2, bool minus, bool &okp, double &facp, bool &okm,
+                                  double &facm)
+{
+    shell_facs_at(rp, rm, sqrt(rp), sqrt(rm), r2, minus, okp, facp, okm, facm);
 }
 
 // renc at recursion depth irec: rhill * RHSCALE * RSHELL**irec with the
