@@ -182,20 +182,21 @@ int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const in
         return fail(SWG_ERR_ARG, "pair_mode must be SWG_PAIR_EXACT or SWG_PAIR_FAST");
     if (!(p.gmtiny >= 0.0)) return fail(SWG_ERR_ARG, "gmtiny must be >= 0");
     tune.pair_fast = p.pair_mode == SWG_PAIR_FAST;
+    nsys = ns;
     if (const char *e = getenv("SWG_KICK_PL_EVAL")) {
         // exact-mode massive-body kernel before any autotuning: 0 one lane
-        // per body, 2 / 4 / 8 evaluating wavefronts per 64-body tile
+        // per body, 4 / 8 evaluating wavefronts per 16- / 64-body tile (2: as 4)
         const int k = atoi(e);
         if (k == 0 || k == 2 || k == 4 || k == 8) tune.kick_pl_eval = k;
-    }
-    nsys = ns;
-    {
-        // exact-mode massive-body kick before any autotuning: with fewer
-        // than two wavefronts per SIMD in the one-lane-per-body kernel, the
-        // terms go to 8 evaluating wavefronts per 64-body tile instead
-        int64_t npl_all = 0;
-        for (int s = 0; s < ns; s++) npl_all += npl_s[s] > 0 ? npl_s[s] : 0;
-        if (!getenv("SWG_KICK_PL_EVAL") && (npl_all + 63) / 64 < 2048) tune.kick_pl_eval = 8;
+    } else {
+        // with fewer than two wavefronts per SIMD in the one-lane-per-body
+        // kernel, the terms go to several wavefronts per tile instead
+        int64_t npl_all = 0, large = 0;
+        for (int s = 0; s < ns; s++) {
+            npl_all += npl_s[s] > 0 ? npl_s[s] : 0;
+            large += npl_s[s] > 0 ? npl_s[s] / RW_LARGE : 0;
+        }
+        if ((npl_all + 63) / 64 < 2048) tune.kick_pl_eval = large < RW_LARGE_TILES ? 4 : 8;
     }
     h_pl_off.assign(nsys + 1, 0);
     h_tp_off.assign(nsys + 1, 0);
@@ -428,7 +429,7 @@ int Ensemble::build_tiles()
 {
     // kick tiles: blocks of tuning.kick_*_block bodies of one system
     std::vector<Tile> tpl, ttp;
-    const int pl_tile = (tune.pair_fast || tune.kick_pl_eval) ? KPL_FAST_TILE : tune.kick_pl_block;
+    const int pl_tile = tune.pl_tile();
     for (int s = 0; s < nsys; s++) {
         if (h_frozen[s]) continue;
         // rows of the bodies a system holds; a slot's padding (inactive, at
@@ -1637,12 +1638,12 @@ int Ensemble::autotune(int reps, int32_t *pl_block, int32_t *tp_block)
         return 0;
     }
     // exact mode: the pl-tp tile size, and for the massive bodies one lane
-    // per body with 64, 128 or 256-body tiles or 64-body tiles shared by
-    // 2, 4 or 8 evaluating wavefronts (reported as -2, -4, -8)
-    const int evals[3] = {2, 4, 8};
+    // per body with 64, 128 or 256-body tiles, or 16- or 64-body tiles
+    // shared by 4 or 8 evaluating wavefronts (reported as -4, -8)
+    const int evals[2] = {4, 8};
     double best_tp = 1e300, best_pl = 1e300;
     int btp = tune.kick_tp_block, bpl = tune.kick_pl_block, bev = tune.kick_pl_eval;
-    for (int k = 0; k < 6; k++) {
+    for (int k = 0; k < 5; k++) {
         if (k < 3) {
             tune.kick_tp_block = cand[k];
             tune.kick_pl_block = cand[k];

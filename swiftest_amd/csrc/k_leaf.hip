@@ -15,6 +15,7 @@
 
 #include "swg_engine.h"
 #include "swg_math.h"
+#include "swg_rows.h"
 
 namespace swg {
 
@@ -52,59 +53,32 @@ __device__ inline void one_pl_half(double rji2, double xr, double yr, double zr,
     }
 }
 
-// swiftest_kick_getacch_int_all_tri_{rad,norad}_pl (swiftest_kick.f90:165-371)
-__global__ void k_leaf_tri(int npl, int nplm, const double *r, const double *Gm, const double *R, double *acc, int fast)
+// swiftest_kick_getacch_int_all_tri_{rad,norad}_pl (swiftest_kick.f90:165-371):
+// the rows of B bodies per workgroup, the terms evaluated by several
+// wavefronts and folded in partner order by others (swg_rows.h).
+template <int B, int KE, bool TRI, bool FAST>
+__global__ __launch_bounds__((RowsLds<B, KE>::THREADS), (RowsLds<B, KE>::WAVES)) void k_leaf_tri(int npl, int nplm, const double *r,
+                                                                      const double *Gm, const double *R, double *acc)
 {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= npl) return;
-    const int nplt = npl - nplm;
-    const double xb = r[3 * b], yb = r[3 * b + 1], zb = r[3 * b + 2];
-    if (nplt > nplm) {
-        // triangular loops with the (ahi, ahj) reduction, one-thread order
-        double hix = 0, hiy = 0, hiz = 0, hjx = 0, hjy = 0, hjz = 0;
-        for (int i = 0; i < min(b, nplm); i++) {  // pairs (i, b): b plays j
-            double xr = xb - r[3 * i], yr = yb - r[3 * i + 1], zr = zb - r[3 * i + 2];
-            double rji2 = dot3(xr, yr, zr, xr, yr, zr);
-            if (R) {
-                double s = R[i] + R[b];
-                if (!(rji2 > s * s)) continue;
-            }
-            one_pl_half(rji2, xr, yr, zr, Gm[i], false, hjx, hjy, hjz, fast);
-        }
-        if (b < nplm) {
-            for (int j = b + 1; j < npl; j++) {  // pairs (b, j)
-                double xr = r[3 * j] - xb, yr = r[3 * j + 1] - yb, zr = r[3 * j + 2] - zb;
-                double rji2 = dot3(xr, yr, zr, xr, yr, zr);
-                if (R) {
-                    double s = R[b] + R[j];
-                    if (!(rji2 > s * s)) continue;
-                }
-                one_pl_half(rji2, xr, yr, zr, Gm[j], true, hix, hiy, hiz, fast);
-            }
-        }
-        acc[3 * b] = (acc[3 * b] + hix) + hjx;
-        acc[3 * b + 1] = (acc[3 * b + 1] + hiy) + hjy;
-        acc[3 * b + 2] = (acc[3 * b + 2] + hiz) + hjz;
-        return;
-    }
-    double ax = acc[3 * b], ay = acc[3 * b + 1], az = acc[3 * b + 2];
-    const int jend = b < nplm ? npl : nplm;
-    for (int j = 0; j < jend; j++) {
-        if (j == b) continue;
-        double rx = r[3 * j] - xb, ry = r[3 * j + 1] - yb, rz = r[3 * j + 2] - zb;
-        double rji2 = dot3(rx, ry, rz, rx, ry, rz);
-        if (R) {
-            double s = R[b] + R[j];
-            if (!(rji2 > s * s)) continue;
-        }
-        double fac = fast ? gm_over_r3_fast(Gm[j], rji2) : gm_over_r3(Gm[j], rji2, pair_g_ok(Gm[j]));
-        ax = fma(fac, rx, ax);
-        ay = fma(fac, ry, ay);
-        az = fma(fac, rz, az);
-    }
-    acc[3 * b] = ax;
-    acc[3 * b + 1] = ay;
-    acc[3 * b + 2] = az;
+    __shared__ RowsLds<B, KE> S;
+    const int b0 = (int)blockIdx.x * B, b1 = min(b0 + B, npl);
+    const RowsSrc src{r, r + 1, r + 2, Gm, R, 3};
+    rows_sums<true, false>(S, src, [&](int comp, int i) { return acc[3 * (int64_t)i + comp]; }, b0, b1, nplm, npl, TRI, FAST,
+              R != nullptr);
+    const int bl = (int)threadIdx.x % B, b = b0 + bl, comp = (int)threadIdx.x / B;
+    if (comp >= 3 || b >= b1) return;
+    double *o = acc + 3 * (int64_t)b + comp;
+    const double v = S.out[0][comp][bl];
+    *o = TRI ? (*o + S.out[1][comp][bl]) + v : v;
+}
+
+template <int B, int KE>
+static void launch_leaf_tri(hipStream_t st, int npl, int nplm, const double *r, const double *Gm, const double *R,
+                            double *acc, bool fast)
+{
+    const auto kern = npl - nplm > nplm ? (fast ? k_leaf_tri<B, KE, true, true> : k_leaf_tri<B, KE, true, false>)
+                                        : (fast ? k_leaf_tri<B, KE, false, true> : k_leaf_tri<B, KE, false, false>);
+    kern<<<cdiv(npl, B), RowsLds<B, KE>::THREADS, 0, st>>>(npl, nplm, r, Gm, R, acc);
 }
 
 // swiftest_kick_getacch_int_all_flat_{rad,norad}_pl (swiftest_kick.f90:69-162)
@@ -1253,7 +1227,8 @@ int swg_kick_getacch_int_all_tri_pl(swg_ctx *ctx, int32_t npl, int32_t nplm, con
     HIPCHK(hipMemcpyAsync(dr, r, 3 * npl * sizeof(double), hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(dg, Gmass, npl * sizeof(double), hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(da, acc, 3 * npl * sizeof(double), hipMemcpyHostToDevice, st));
-    k_leaf_tri<<<cdiv(npl, 128), 128, 0, st>>>(npl, nplm, dr, dg, dR, da, ctx->pair_mode);
+    if (npl / RW_LARGE < RW_LARGE_TILES) launch_leaf_tri<RW_SMALL, 4>(st, npl, nplm, dr, dg, dR, da, ctx->pair_mode);
+    else launch_leaf_tri<RW_LARGE, 8>(st, npl, nplm, dr, dg, dR, da, ctx->pair_mode);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(acc, da, 3 * npl * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));

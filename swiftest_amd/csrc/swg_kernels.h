@@ -7,6 +7,7 @@
 
 #include "../../include/swiftest_hip.h"
 #include "swg_level.h"
+#include "swg_rows.h"
 #include "swg_state.h"
 
 namespace swg {
@@ -31,12 +32,28 @@ struct Tuning {
     int kick_tp_block = 256;
     int pair_fast = 0;         // 1: pair factors from the reciprocal square root (SWG_PAIR_FAST)
     int kick_pl_split = 8;     // fast mode: wavefronts sharing one 64-body tile's rows (1, 2, 4, 8, 16)
-    int kick_pl_eval = 0;      // exact mode: 0 one lane per body (k_kick_pl), else the evaluating
-                               // wavefronts per 64-body tile of k_kick_pl_split (2, 4, 8)
-    int any_tiny = 0;          // some system has semi-interacting bodies: k_kick_pl_tiny for every tile
+    int kick_pl_eval = 0;      // exact mode: 0 one lane per body (k_kick_pl), else k_kick_pl_rows with that
+                               // many evaluating wavefronts: 4 for 16-body tiles, 8 for 64-body tiles
+    int any_tiny = 0;          // some system has semi-interacting bodies: k_kick_pl_rows, 16-body tiles
+    // bodies per massive-body tile of the kernel launch_kick_pl takes
+    int pl_tile() const;
 };
 // bodies per massive-body tile of the fast pair kernel
 constexpr int KPL_FAST_TILE = 64;
+
+// the two tile sizes of k_kick_pl_rows and of the leaf rows
+constexpr int RW_SMALL = 16, RW_LARGE = 64;
+// 64-body tiles once they fill three quarters of the compute units (measured,
+// 16 / 64 bodies a tile: 2000 bodies 37 / 70 us, 10000 bodies 300 / 320 us,
+// 32000 bodies 2.7 / 2.0 ms)
+constexpr int RW_LARGE_TILES = 192;
+
+inline int Tuning::pl_tile() const
+{
+    if (any_tiny) return RW_SMALL;
+    if (pair_fast) return KPL_FAST_TILE;
+    return kick_pl_eval == 0 ? kick_pl_block : kick_pl_eval == 8 ? RW_LARGE : RW_SMALL;
+}
 
 // ---- step kernels (k_step.hip) ----
 void launch_reset_levels(hipStream_t st, PlDev pl, TpDev tp, int npl, int ntp);

@@ -85,6 +85,7 @@ __device__ inline double div_core(double a, double b)
 // IEEE operations run.  Separations of an N-body system in AU are far inside
 // that range.
 constexpr double PAIR_R2_LO = 0x1p-400, PAIR_R2_HI = 0x1p400;
+constexpr int PAIR_R2_LO_HI = (1023 - 400) << 20, PAIR_R2_HI_HI = (1023 + 400) << 20;  // their high words
 constexpr double PAIR_G_LO = 0x1p-500, PAIR_G_HI = 0x1p500;
 
 __host__ __device__ inline bool pair_g_ok(double g) { return g == 0.0 || (g >= PAIR_G_LO && g <= PAIR_G_HI); }
