@@ -137,36 +137,12 @@ int Ensemble::alloc_vec(Vec3p &v, size_t n)
     return 0;
 }
 
-static int upload_aos(hipStream_t st, Vec3p v, const double *aos, size_t n, std::vector<double> &tmp)
+// a host array to the device, queued on the stream (the array may be changed
+// on return)
+hipError_t Ensemble::put(void *dev, const void *host, size_t bytes)
 {
-    tmp.resize(3 * (n ? n : 1));
-    double *cx = tmp.data(), *cy = cx + n, *cz = cy + n;
-    for (size_t i = 0; i < n; i++) {
-        cx[i] = aos[3 * i];
-        cy[i] = aos[3 * i + 1];
-        cz[i] = aos[3 * i + 2];
-    }
-    HIPCHK(hipMemcpyAsync(v.x, cx, n * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(v.y, cy, n * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(v.z, cz, n * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipStreamSynchronize(st));
-    return 0;
-}
-
-static int download_aos(hipStream_t st, Vec3p v, double *aos, size_t n)
-{
-    std::vector<double> tmp(3 * (n ? n : 1));
-    double *cx = tmp.data(), *cy = cx + n, *cz = cy + n;
-    HIPCHK(hipMemcpyAsync(cx, v.x, n * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(cy, v.y, n * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(cz, v.z, n * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    for (size_t i = 0; i < n; i++) {
-        aos[3 * i] = cx[i];
-        aos[3 * i + 1] = cy[i];
-        aos[3 * i + 2] = cz[i];
-    }
-    return 0;
+    const XferItem x = xfer_i32((const int32_t *)host, (const int32_t *)dev, (int64_t)(bytes / sizeof(int32_t)));
+    return stage->in(stream, &x, 1);
 }
 
 int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const int32_t *ntp_s, const double *GMcb,
@@ -289,36 +265,37 @@ int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const in
         }
         nblk_pl = cbp[nsys];
         nblk_tp = cbt[nsys];
-        HIPCHK(copy_wait(stream, d_cb_pl, cbp.data(), (nsys + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
-        HIPCHK(copy_wait(stream, d_cb_tp, cbt.data(), (nsys + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
+        HIPCHK(put(d_cb_pl, cbp.data(), (nsys + 1) * sizeof(int32_t)));
+        HIPCHK(put(d_cb_tp, cbt.data(), (nsys + 1) * sizeof(int32_t)));
     }
-    std::vector<double> tmp;
-    if (upload_aos(st, pl.rh, rh.data(), npl, tmp) || upload_aos(st, pl.vh, vh.data(), npl, tmp)) return SWG_ERR_HIP;
-    if (upload_aos(st, tp.rh, tp_rh, ntp, tmp) || upload_aos(st, tp.vh, tp_vh, ntp, tmp)) return SWG_ERR_HIP;
-    HIPCHK(copy_wait(stream, pl.Gm, gm.data(), npl * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(stream, pl.R, rad.data(), npl * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(stream, pl.rhill, rhill.data(), npl * sizeof(double), hipMemcpyHostToDevice));
+    {
+        const XferItem x[] = {xfer_vec3(rh.data(), pl.rh, npl),    xfer_vec3(vh.data(), pl.vh, npl),
+                              xfer_words(gm.data(), pl.Gm, npl),   xfer_words(rad.data(), pl.R, npl),
+                              xfer_words(rhill.data(), pl.rhill, npl), xfer_vec3(tp_rh, tp.rh, ntp),
+                              xfer_vec3(tp_vh, tp.vh, ntp)};
+        HIPCHK(stage->in(st, x, 7));
+    }
     std::vector<int32_t> zeros(std::max(std::max(npl, ntp), 3 * nsys) + 1, 0);
     std::vector<int32_t> sys_pl(npl), sys_tp(ntp), ones(nsys, 1);
     for (int s = 0; s < nsys; s++) {
         for (int i = h_pl_off[s]; i < h_pl_off[s + 1]; i++) sys_pl[i] = s;
         for (int i = h_tp_off[s]; i < h_tp_off[s + 1]; i++) sys_tp[i] = s;
     }
-    HIPCHK(copy_wait(stream, pl.status, zeros.data(), npl * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(stream, tp.status, zeros.data(), ntp * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(stream, pl.sys, sys_pl.data(), npl * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(stream, tp.sys, sys_tp.data(), ntp * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(stream, sy.pl_off, h_pl_off.data(), (nsys + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(stream, sy.tp_off, h_tp_off.data(), (nsys + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(stream, sy.GMcb, GMcb, nsys * sizeof(double), hipMemcpyHostToDevice));
+    HIPCHK(put(pl.status, zeros.data(), npl * sizeof(int32_t)));
+    HIPCHK(put(tp.status, zeros.data(), ntp * sizeof(int32_t)));
+    HIPCHK(put(pl.sys, sys_pl.data(), npl * sizeof(int32_t)));
+    HIPCHK(put(tp.sys, sys_tp.data(), ntp * sizeof(int32_t)));
+    HIPCHK(put(sy.pl_off, h_pl_off.data(), (nsys + 1) * sizeof(int32_t)));
+    HIPCHK(put(sy.tp_off, h_tp_off.data(), (nsys + 1) * sizeof(int32_t)));
+    HIPCHK(put(sy.GMcb, GMcb, nsys * sizeof(double)));
     std::vector<double> dz(3 * (size_t)nsys, 0.0);
-    HIPCHK(copy_wait(stream, sy.ptbeg, dz.data(), 3 * nsys * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(stream, sy.ptend, dz.data(), 3 * nsys * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(stream, sy.cbvb, dz.data(), 3 * nsys * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(stream, sy.lfirst, ones.data(), nsys * sizeof(int32_t), hipMemcpyHostToDevice));
+    HIPCHK(put(sy.ptbeg, dz.data(), 3 * nsys * sizeof(double)));
+    HIPCHK(put(sy.ptend, dz.data(), 3 * nsys * sizeof(double)));
+    HIPCHK(put(sy.cbvb, dz.data(), 3 * nsys * sizeof(double)));
+    HIPCHK(put(sy.lfirst, ones.data(), nsys * sizeof(int32_t)));
     h_frozen.assign(nsys, 0);
     for (int32_t *q : {sy.enc_pp, sy.enc_pt, sy.flag_pp, sy.flag_pt, sy.err, sy.frozen})
-        HIPCHK(copy_wait(stream, q, zeros.data(), nsys * sizeof(int32_t), hipMemcpyHostToDevice));
+        HIPCHK(put(q, zeros.data(), nsys * sizeof(int32_t)));
     // semi-interacting bodies (symba_util.f90:191-202 with lmtiny_pl for
     // SyMBA, swiftest_io.f90:2663): after the mass sort the fully interacting
     // bodies of a system come first, nplm of them
@@ -336,8 +313,8 @@ int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const in
             nplm[s] = m;
             any_tiny |= m < n;
         }
-        HIPCHK(copy_wait(stream, pl.tiny, tiny.data(), npl * sizeof(int32_t), hipMemcpyHostToDevice));
-        HIPCHK(copy_wait(stream, sy.nplm, nplm.data(), nsys * sizeof(int32_t), hipMemcpyHostToDevice));
+        HIPCHK(put(pl.tiny, tiny.data(), npl * sizeof(int32_t)));
+        HIPCHK(put(sy.nplm, nplm.data(), nsys * sizeof(int32_t)));
         tune.any_tiny = any_tiny;
     }
 
@@ -361,8 +338,8 @@ int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const in
         if (own2(&pp.words, w) || own2(&pp.wpre, w) || own2(&pp.woff, nsys) || own2(&pp.nb, nsys) ||
             own2(&pp.rowcnt, npl) || own2(&pp.rowstart, npl) || own2(&pp.colcnt, npl) || own2(&pp.colstart, npl))
             return SWG_ERR_HIP;
-        HIPCHK(copy_wait(stream, pp.woff, woff.data(), nsys * sizeof(int64_t), hipMemcpyHostToDevice));
-        HIPCHK(copy_wait(stream, pp.nb, nb.data(), nsys * sizeof(int32_t), hipMemcpyHostToDevice));
+        HIPCHK(put(pp.woff, woff.data(), nsys * sizeof(int64_t)));
+        HIPCHK(put(pp.nb, nb.data(), nsys * sizeof(int32_t)));
     }
     {
         std::vector<int64_t> woff(nsys);
@@ -378,8 +355,8 @@ int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const in
         if (own2(&pt.woff, nsys) || own2(&pt.nb, nsys) || own2(&pt.rowcnt, npl) || own2(&pt.rowstart, npl) ||
             own2(&pt.colcnt, ntp) || own2(&pt.colstart, ntp))
             return SWG_ERR_HIP;
-        HIPCHK(copy_wait(stream, pt.woff, woff.data(), nsys * sizeof(int64_t), hipMemcpyHostToDevice));
-        HIPCHK(copy_wait(stream, pt.nb, nb.data(), nsys * sizeof(int32_t), hipMemcpyHostToDevice));
+        HIPCHK(put(pt.woff, woff.data(), nsys * sizeof(int64_t)));
+        HIPCHK(put(pt.nb, nb.data(), nsys * sizeof(int32_t)));
     }
     int mx = std::max(npl, ntp);
     HIPCHK(hipMalloc(&d_scan, scan_scratch_bytes(mx)));
@@ -453,7 +430,7 @@ int Ensemble::build_tiles()
     // SWG_FAIL_TILE_ALLOC=1 makes the allocation fail, for tests of this path.
     tiles_ok = false;
     const char *inject = getenv("SWG_FAIL_TILE_ALLOC");
-    auto put = [&](auto &vec, auto **dptr, int &cnt) -> int {
+    auto publish = [&](auto &vec, auto **dptr, int &cnt) -> int {
         using T = typename std::remove_reference<decltype(vec)>::type::value_type;
         cnt = 0;
         if (*dptr) (void)hipFree(*dptr);
@@ -461,13 +438,13 @@ int Ensemble::build_tiles()
         if (inject && inject[0] == '1')
             return fail(SWG_ERR_HIP, "hipMalloc (tile arrays): out of memory (injected by SWG_FAIL_TILE_ALLOC)");
         HIPCHK(hipMalloc((void **)dptr, sizeof(T) * (vec.size() ? vec.size() : 1)));
-        if (!vec.empty()) HIPCHK(copy_wait(stream, *dptr, vec.data(), sizeof(T) * vec.size(), hipMemcpyHostToDevice));
+        if (!vec.empty()) HIPCHK(put(*dptr, vec.data(), sizeof(T) * vec.size()));
         cnt = (int)vec.size();
         return 0;
     };
-    if (int rc = put(tpl, &d_tiles_pl, ntiles_pl)) return rc;
-    if (int rc = put(ttp, &d_tiles_tp, ntiles_tp)) return rc;
-    if (int rc = put(tpp, &d_tiles_pp, ntiles_pp)) return rc;
+    if (int rc = publish(tpl, &d_tiles_pl, ntiles_pl)) return rc;
+    if (int rc = publish(ttp, &d_tiles_tp, ntiles_tp)) return rc;
+    if (int rc = publish(tpp, &d_tiles_pp, ntiles_pp)) return rc;
     if (!d_tiles_pt) {
         int total = 0;
         for (int s = 0; s < nsys; s++) total += (h_tp_off[s + 1] - h_tp_off[s] + 63) / 64;
@@ -503,9 +480,7 @@ int Ensemble::detect_pp(double dt)
     launch_sys_flags(st, pp, sy.pl_off, sy.enc_pp, nsys);
     int64_t *ht = (int64_t *)h_small;
     int32_t *hf = (int32_t *)(h_small + 1024);
-    HIPCHK(hipMemcpyAsync(ht, d_total, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(hf, sy.enc_pp, nsys * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(hf + nsys, sy.err, nsys * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    launch_report(st, d_total, sy.enc_pp, sy.err, nsys, ht, hf);
     HIPCHK(hipStreamSynchronize(st));
     npp = npl ? ht[0] : 0;
     h_enc_pp.assign(hf, hf + nsys);
@@ -534,8 +509,7 @@ int Ensemble::detect_pp_sas(double dt)
     if (hipError_t e = sas_fill(st, sas, pp, pl, npl, npp)) return hipfail(e, "sort-and-sweep list");
     launch_sys_flags(st, pp, sy.pl_off, sy.enc_pp, nsys);
     int32_t *hf = (int32_t *)(h_small + 1024);
-    HIPCHK(hipMemcpyAsync(hf, sy.enc_pp, nsys * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(hf + nsys, sy.err, nsys * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    launch_report(st, nullptr, sy.enc_pp, sy.err, nsys, nullptr, hf);
     HIPCHK(hipStreamSynchronize(st));
     h_enc_pp.assign(hf, hf + nsys);
     h_err.assign(hf + nsys, hf + 2 * nsys);
@@ -561,16 +535,15 @@ int Ensemble::detect_pt(double dt, const std::vector<int32_t> &run)
         HIPCHK(dalloc(&pt.words, pt_words));
         HIPCHK(dalloc(&pt.wpre, pt_words));
     }
-    HIPCHK(hipMemcpyAsync(d_tiles_pt, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(d_pt_run, run.data(), nsys * sizeof(int32_t), hipMemcpyHostToDevice, st));
+    HIPCHK(put(d_tiles_pt, tiles.data(), tiles.size() * sizeof(int4)));
+    HIPCHK(put(d_pt_run, run.data(), nsys * sizeof(int32_t)));
     launch_pt_tiles(st, pl, tp, sy, pt, d_tiles_pt, (int)tiles.size(), dt);
     launch_rows_count(st, pt, pl.sys, 0, sy.pl_off, d_pt_run, npl);
     launch_scan_i32_i64(st, pt.rowcnt, pt.rowstart, npl, d_total, d_scan);
     launch_sys_flags(st, pt, sy.pl_off, sy.enc_pt, nsys);
     int64_t *ht = (int64_t *)h_small;
     int32_t *hf = (int32_t *)(h_small + 1024);
-    HIPCHK(hipMemcpyAsync(ht, d_total, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(hf, sy.enc_pt, nsys * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    launch_report(st, d_total, sy.enc_pt, nullptr, nsys, ht, hf);
     HIPCHK(hipStreamSynchronize(st));
     npt = npl ? ht[0] : 0;
     h_enc_pt.assign(hf, hf + nsys);
@@ -841,20 +814,20 @@ int Ensemble::energy(const double *cb_mass, const double *cb_radius, const doubl
             own(&en_tiles, (size_t)en_ntiles) || own(&en_toff, (size_t)nsys + 1))
             return SWG_ERR_HIP;
         if (en_ntiles)
-            HIPCHK(copy_wait(stream, en_tiles, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
-        HIPCHK(copy_wait(stream, en_toff, toff.data(), toff.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+            HIPCHK(put(en_tiles, tiles.data(), tiles.size() * sizeof(int4)));
+        HIPCHK(put(en_toff, toff.data(), toff.size() * sizeof(int32_t)));
         en_ready = true;
     }
-    if (npl) HIPCHK(hipMemcpyAsync(en_mass, pl_mass, npl * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(en_cb, cb_mass, nsys * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(en_cb + nsys, cb_radius, nsys * sizeof(double), hipMemcpyHostToDevice, st));
+    const XferItem in[] = {xfer_words(pl_mass, en_mass, npl), xfer_words(cb_mass, en_cb, nsys),
+                           xfer_words(cb_radius, en_cb + nsys, nsys)};
+    HIPCHK(stage->in(st, in, 3));
     // swiftest_io_conservation_report (swiftest_io.f90:135-141): WHM holds vh
     if (prm.integrator == SWG_WHM) launch_vh2vb(st, pl, sy, nsys, npl);
     launch_energy(st, pl, sy, nsys, en_mass, en_cb, en_cb + nsys, prm.lclose, en_rb, en_tiles, en_ntiles, en_toff,
                   en_part, en_out);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(out, en_out, (size_t)nsys * SWG_ENERGY_NOUT * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    const XferItem res = xfer_words(out, en_out, (int64_t)nsys * SWG_ENERGY_NOUT);
+    HIPCHK(stage->out(st, &res, 1));
     return 0;
 }
 
@@ -876,21 +849,21 @@ int Ensemble::discard(const swg_discard_params &dp, const double *cb_radius, int
         std::vector<int32_t> one(std::max(std::max(npl, ntp), nsys), 1);
         std::vector<double> zero(std::max(npl, ntp), 0.0);
         if (npl) {
-            HIPCHK(copy_wait(stream, dis_pl_isperi, one.data(), npl * sizeof(int32_t), hipMemcpyHostToDevice));
-            HIPCHK(copy_wait(stream, dis_pl_atp, zero.data(), npl * sizeof(double), hipMemcpyHostToDevice));
-            HIPCHK(copy_wait(stream, dis_pl_peri, zero.data(), npl * sizeof(double), hipMemcpyHostToDevice));
+            HIPCHK(put(dis_pl_isperi, one.data(), npl * sizeof(int32_t)));
+            HIPCHK(put(dis_pl_atp, zero.data(), npl * sizeof(double)));
+            HIPCHK(put(dis_pl_peri, zero.data(), npl * sizeof(double)));
         }
         if (ntp) {
-            HIPCHK(copy_wait(stream, dis_tp_isperi, one.data(), ntp * sizeof(int32_t), hipMemcpyHostToDevice));
-            HIPCHK(copy_wait(stream, dis_tp_atp, zero.data(), ntp * sizeof(double), hipMemcpyHostToDevice));
-            HIPCHK(copy_wait(stream, dis_tp_peri, zero.data(), ntp * sizeof(double), hipMemcpyHostToDevice));
+            HIPCHK(put(dis_tp_isperi, one.data(), ntp * sizeof(int32_t)));
+            HIPCHK(put(dis_tp_atp, zero.data(), ntp * sizeof(double)));
+            HIPCHK(put(dis_tp_peri, zero.data(), ntp * sizeof(double)));
         }
-        HIPCHK(copy_wait(stream, dis_lfirst, one.data(), nsys * sizeof(int32_t), hipMemcpyHostToDevice));
+        HIPCHK(put(dis_lfirst, one.data(), nsys * sizeof(int32_t)));
         if (dis_ntiles)
-            HIPCHK(copy_wait(stream, dis_tiles, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
+            HIPCHK(put(dis_tiles, tiles.data(), tiles.size() * sizeof(int4)));
         dis_ready = true;
     }
-    HIPCHK(hipMemcpyAsync(dis_rcb, cb_radius, nsys * sizeof(double), hipMemcpyHostToDevice, st));
+    HIPCHK(put(dis_rcb, cb_radius, nsys * sizeof(double)));
     const bool symba = prm.integrator == SWG_SYMBA;
     // pl%nplenc: the pairs of each body in the last step's level-0 list
     const bool enc = symba && npp > 0;
@@ -899,8 +872,8 @@ int Ensemble::discard(const swg_discard_params &dp, const double *cb_radius, int
                    dis_tp_peri, dis_lfirst, dis_gone, dis_sys, dis_count, dis_tiles, dis_ntiles);
     HIPCHK(hipGetLastError());
     unsigned long long c[2];
-    HIPCHK(hipMemcpyAsync(c, dis_count, sizeof c, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    const XferItem res = xfer_words(c, dis_count, 2);
+    HIPCHK(stage->out(st, &res, 1));
     if (npl_dis) *npl_dis = (int64_t)c[0];
     if (ntp_dis) *ntp_dis = (int64_t)c[1];
     return 0;
@@ -909,7 +882,8 @@ int Ensemble::discard(const swg_discard_params &dp, const double *cb_radius, int
 int Ensemble::check_errors()
 {
     int32_t *hf = (int32_t *)(h_small + 1024);
-    HIPCHK(hipMemcpyAsync(hf, sy.err, nsys * sizeof(int32_t), hipMemcpyDeviceToHost, stream));
+    launch_report(stream, nullptr, sy.err, nullptr, nsys, nullptr, hf);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(stream));
     h_err.assign(hf, hf + nsys);
     return err_code();
@@ -1148,15 +1122,16 @@ int Ensemble::snapshot()
     launch_snapshot(st, pl, tp, sy, nsys, npl, ntp);
     if (!prm.rhill_present) {
         std::vector<double> rh(3 * (size_t)npl), vh(3 * (size_t)npl), rhill(npl);
-        if (download_aos(st, pl.rh, rh.data(), npl) || download_aos(st, pl.vh, vh.data(), npl)) return SWG_ERR_HIP;
-        if (nfrozen) HIPCHK(hipMemcpyAsync(rhill.data(), pl.rhill, npl * sizeof(double), hipMemcpyDeviceToHost, st));
+        const XferItem get[] = {xfer_vec3(rh.data(), pl.rh, npl), xfer_vec3(vh.data(), pl.vh, npl),
+                                xfer_words(rhill.data(), pl.rhill, nfrozen ? npl : 0)};
+        HIPCHK(stage->out(st, get, 3));
         for (int s = 0; s < nsys; s++) {
             if (h_frozen[s]) continue;  // a frozen system keeps its state, rhill included
             int a = h_pl_off[s], n = h_pl_off[s + 1] - a;
             host_set_rhill(h_GMcb[s], n, &rh[3 * (size_t)a], &vh[3 * (size_t)a], &h_Gm[a], &rhill[a]);
         }
-        HIPCHK(hipMemcpyAsync(pl.rhill, rhill.data(), npl * sizeof(double), hipMemcpyHostToDevice, st));
-        HIPCHK(hipStreamSynchronize(st));
+        const XferItem put = xfer_words(rhill.data(), pl.rhill, npl);
+        HIPCHK(stage->in(st, &put, 1));
     }
     return 0;
 }
@@ -1204,28 +1179,26 @@ int Ensemble::run(int64_t nsteps)
 int Ensemble::get(double *pl_rh, double *pl_vh, double *pl_vb, double *tp_rh, double *tp_vh, double *tp_vb,
                   int32_t *pl_status, int32_t *tp_status, int32_t *pl_id)
 {
-    hipStream_t st = stream;
-    HIPCHK(hipStreamSynchronize(st));
-    if (pl_rh && download_aos(st, pl.rh, pl_rh, npl)) return SWG_ERR_HIP;
-    if (pl_vh && download_aos(st, pl.vh, pl_vh, npl)) return SWG_ERR_HIP;
-    if (pl_vb && download_aos(st, pl.vb, pl_vb, npl)) return SWG_ERR_HIP;
-    if (tp_rh && download_aos(st, tp.rh, tp_rh, ntp)) return SWG_ERR_HIP;
-    if (tp_vh && download_aos(st, tp.vh, tp_vh, ntp)) return SWG_ERR_HIP;
-    if (tp_vb && download_aos(st, tp.vb, tp_vb, ntp)) return SWG_ERR_HIP;
-    if (pl_status) HIPCHK(copy_wait(stream, pl_status, pl.status, npl * sizeof(int32_t), hipMemcpyDeviceToHost));
-    if (tp_status) HIPCHK(copy_wait(stream, tp_status, tp.status, ntp * sizeof(int32_t), hipMemcpyDeviceToHost));
+    const XferItem x[] = {xfer_vec3(pl_rh, pl.rh, pl_rh ? npl : 0),
+                          xfer_vec3(pl_vh, pl.vh, pl_vh ? npl : 0),
+                          xfer_vec3(pl_vb, pl.vb, pl_vb ? npl : 0),
+                          xfer_i32(pl_status, pl.status, pl_status ? npl : 0),
+                          xfer_vec3(tp_rh, tp.rh, tp_rh ? ntp : 0),
+                          xfer_vec3(tp_vh, tp.vh, tp_vh ? ntp : 0),
+                          xfer_vec3(tp_vb, tp.vb, tp_vb ? ntp : 0),
+                          xfer_i32(tp_status, tp.status, tp_status ? ntp : 0)};
+    HIPCHK(stage->out(stream, x, 8));
     if (pl_id) std::copy(h_pl_id.begin(), h_pl_id.end(), pl_id);
     return 0;
 }
 
 int Ensemble::get_misc(double *rhill, double *cb_vb, double *ptbeg, double *ptend, int32_t *lfirst)
 {
-    HIPCHK(hipStreamSynchronize(stream));
-    if (rhill) HIPCHK(copy_wait(stream, rhill, pl.rhill, npl * sizeof(double), hipMemcpyDeviceToHost));
-    if (cb_vb) HIPCHK(copy_wait(stream, cb_vb, sy.cbvb, 3 * nsys * sizeof(double), hipMemcpyDeviceToHost));
-    if (ptbeg) HIPCHK(copy_wait(stream, ptbeg, sy.ptbeg, 3 * nsys * sizeof(double), hipMemcpyDeviceToHost));
-    if (ptend) HIPCHK(copy_wait(stream, ptend, sy.ptend, 3 * nsys * sizeof(double), hipMemcpyDeviceToHost));
-    if (lfirst) HIPCHK(copy_wait(stream, lfirst, sy.lfirst, nsys * sizeof(int32_t), hipMemcpyDeviceToHost));
+    const XferItem x[] = {xfer_words(rhill, pl.rhill, rhill ? npl : 0), xfer_words(cb_vb, sy.cbvb, cb_vb ? 3 * nsys : 0),
+                          xfer_words(ptbeg, sy.ptbeg, ptbeg ? 3 * nsys : 0),
+                          xfer_words(ptend, sy.ptend, ptend ? 3 * nsys : 0),
+                          xfer_i32(lfirst, sy.lfirst, lfirst ? nsys : 0)};
+    HIPCHK(stage->out(stream, x, 5));
     return 0;
 }
 
@@ -1411,57 +1384,47 @@ int Ensemble::load(int s, int npl_new, int ntp_new, double GMcb_new, const doubl
             trh[3 * (size_t)q + 2] = pr[2];
         }
     }
-    // the slot's ranges of the SoA arrays
-    auto put3 = [&](Vec3p v, int off, const std::vector<double> &aos, int n) -> int {
-        if (!n) return 0;
-        std::vector<double> c(3 * (size_t)n);
-        for (int i = 0; i < n; i++)
-            for (int d = 0; d < 3; d++) c[(size_t)d * n + i] = aos[3 * (size_t)i + d];
-        HIPCHK(copy_wait(st, v.x + off, c.data(), n * sizeof(double), hipMemcpyHostToDevice));
-        HIPCHK(copy_wait(st, v.y + off, c.data() + n, n * sizeof(double), hipMemcpyHostToDevice));
-        HIPCHK(copy_wait(st, v.z + off, c.data() + 2 * (size_t)n, n * sizeof(double), hipMemcpyHostToDevice));
-        return 0;
-    };
-    // rbeg / rend of the padding are read as partner positions by the
-    // particle kicks, so the whole range gets the positions
-    for (Vec3p v : {pl.rh, pl.rbeg, pl.rend})
-        if (int rc = put3(v, p0, rh, cap_pl)) return rc;
-    if (int rc = put3(pl.vh, p0, vh, cap_pl)) return rc;
-    if (int rc = put3(tp.rh, t0, trh, cap_tp)) return rc;
-    if (int rc = put3(tp.vh, t0, tvh, cap_tp)) return rc;
-    if (cap_pl) {
-        HIPCHK(copy_wait(st, pl.Gm + p0, gm.data(), cap_pl * sizeof(double), hipMemcpyHostToDevice));
-        HIPCHK(copy_wait(st, pl.R + p0, rad.data(), cap_pl * sizeof(double), hipMemcpyHostToDevice));
-        HIPCHK(copy_wait(st, pl.rhill + p0, rhl.data(), cap_pl * sizeof(double), hipMemcpyHostToDevice));
-        HIPCHK(copy_wait(st, pl.status + p0, status.data(), cap_pl * sizeof(int32_t), hipMemcpyHostToDevice));
+    // the slot's ranges of the SoA arrays; rbeg / rend of the padding are read
+    // as partner positions by the particle kicks, so the whole range gets the
+    // positions
+    auto at = [](Vec3p v, int off) { return Vec3p{v.x + off, v.y + off, v.z + off}; };
+    {
+        const XferItem x[] = {xfer_vec3(rh.data(), at(pl.rh, p0), cap_pl),   xfer_vec3(rh.data(), at(pl.rbeg, p0), cap_pl),
+                              xfer_vec3(rh.data(), at(pl.rend, p0), cap_pl), xfer_vec3(vh.data(), at(pl.vh, p0), cap_pl),
+                              xfer_words(gm.data(), pl.Gm + p0, cap_pl),     xfer_words(rad.data(), pl.R + p0, cap_pl),
+                              xfer_words(rhl.data(), pl.rhill + p0, cap_pl), xfer_i32(status.data(), pl.status + p0, cap_pl),
+                              xfer_vec3(trh.data(), at(tp.rh, t0), cap_tp),  xfer_vec3(tvh.data(), at(tp.vh, t0), cap_tp),
+                              xfer_i32(tstatus.data(), tp.status + t0, cap_tp)};
+        HIPCHK(stage->in(st, x, 11));
     }
-    if (cap_tp) HIPCHK(copy_wait(st, tp.status + t0, tstatus.data(), cap_tp * sizeof(int32_t), hipMemcpyHostToDevice));
     // per-system scalars as create leaves them
     const double z3[3] = {0.0, 0.0, 0.0};
     const int32_t one = 1, zero = 0;
     h_GMcb[s] = GMcb_new;
-    HIPCHK(copy_wait(st, sy.GMcb + s, &GMcb_new, sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(st, sy.ptbeg + 3 * s, z3, sizeof z3, hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(st, sy.ptend + 3 * s, z3, sizeof z3, hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(st, sy.lfirst + s, &one, sizeof one, hipMemcpyHostToDevice));
-    for (int32_t *q : {sy.enc_pp, sy.enc_pt, sy.flag_pp, sy.flag_pt, sy.err, sy.frozen})
-        HIPCHK(copy_wait(st, q + s, &zero, sizeof zero, hipMemcpyHostToDevice));
-    HIPCHK(copy_wait(st, d_active + s, &one, sizeof one, hipMemcpyHostToDevice));
+    {
+        const XferItem x[] = {xfer_words(&GMcb_new, sy.GMcb + s, 1),  xfer_words(z3, sy.ptbeg + 3 * s, 3),
+                              xfer_words(z3, sy.ptend + 3 * s, 3),    xfer_i32(&one, sy.lfirst + s, 1),
+                              xfer_i32(&zero, sy.enc_pp + s, 1),      xfer_i32(&zero, sy.enc_pt + s, 1),
+                              xfer_i32(&zero, sy.flag_pp + s, 1),     xfer_i32(&zero, sy.flag_pt + s, 1),
+                              xfer_i32(&zero, sy.err + s, 1),         xfer_i32(&zero, sy.frozen + s, 1),
+                              xfer_i32(&one, d_active + s, 1)};
+        HIPCHK(stage->in(st, x, 11));
+    }
     if (dis_ready) {
         // pericentre-passage state of the discard checks starts afresh
         std::vector<int32_t> ones(std::max(std::max(cap_pl, cap_tp), 1), 1);
         std::vector<double> zd(std::max(std::max(cap_pl, cap_tp), 1), 0.0);
         if (cap_pl) {
-            HIPCHK(copy_wait(st, dis_pl_isperi + p0, ones.data(), cap_pl * sizeof(int32_t), hipMemcpyHostToDevice));
-            HIPCHK(copy_wait(st, dis_pl_atp + p0, zd.data(), cap_pl * sizeof(double), hipMemcpyHostToDevice));
-            HIPCHK(copy_wait(st, dis_pl_peri + p0, zd.data(), cap_pl * sizeof(double), hipMemcpyHostToDevice));
+            HIPCHK(put(dis_pl_isperi + p0, ones.data(), cap_pl * sizeof(int32_t)));
+            HIPCHK(put(dis_pl_atp + p0, zd.data(), cap_pl * sizeof(double)));
+            HIPCHK(put(dis_pl_peri + p0, zd.data(), cap_pl * sizeof(double)));
         }
         if (cap_tp) {
-            HIPCHK(copy_wait(st, dis_tp_isperi + t0, ones.data(), cap_tp * sizeof(int32_t), hipMemcpyHostToDevice));
-            HIPCHK(copy_wait(st, dis_tp_atp + t0, zd.data(), cap_tp * sizeof(double), hipMemcpyHostToDevice));
-            HIPCHK(copy_wait(st, dis_tp_peri + t0, zd.data(), cap_tp * sizeof(double), hipMemcpyHostToDevice));
+            HIPCHK(put(dis_tp_isperi + t0, ones.data(), cap_tp * sizeof(int32_t)));
+            HIPCHK(put(dis_tp_atp + t0, zd.data(), cap_tp * sizeof(double)));
+            HIPCHK(put(dis_tp_peri + t0, zd.data(), cap_tp * sizeof(double)));
         }
-        HIPCHK(copy_wait(st, dis_lfirst + s, &one, sizeof one, hipMemcpyHostToDevice));
+        HIPCHK(put(dis_lfirst + s, &one, sizeof one));
     }
     {
         std::vector<int32_t> tiny(std::max(cap_pl, 1), 0);
@@ -1473,10 +1436,10 @@ int Ensemble::load(int s, int npl_new, int ntp_new, double GMcb_new, const doubl
                 m += !tiny[q];
             }
         }
-        if (cap_pl) HIPCHK(copy_wait(st, pl.tiny + p0, tiny.data(), cap_pl * sizeof(int32_t), hipMemcpyHostToDevice));
+        if (cap_pl) HIPCHK(put(pl.tiny + p0, tiny.data(), cap_pl * sizeof(int32_t)));
         // the padding sits after the system's own bodies: as partners of
         // the fully interacting rows they add exact zeros
-        HIPCHK(copy_wait(st, sy.nplm + s, &m, sizeof m, hipMemcpyHostToDevice));
+        HIPCHK(put(sy.nplm + s, &m, sizeof m));
         if (m < npl_new) {
             any_tiny = true;
             tune.any_tiny = 1;
@@ -1503,18 +1466,17 @@ int Ensemble::get_slot(int s, double *pl_rh, double *pl_vh, double *pl_vb, doubl
                        double *tp_vb, int32_t *pl_status, int32_t *tp_status, int32_t *pl_id)
 {
     if (s < 0 || s >= nsys) return fail(SWG_ERR_ARG, "no such slot");
-    hipStream_t st = stream;
-    HIPCHK(hipStreamSynchronize(st));
     const int p0 = h_pl_off[s], n = h_nreal_pl[s], t0 = h_tp_off[s], m = h_nreal_tp[s];
     auto sub = [](Vec3p v, int off) { return Vec3p{v.x + off, v.y + off, v.z + off}; };
-    if (pl_rh && n && download_aos(st, sub(pl.rh, p0), pl_rh, n)) return SWG_ERR_HIP;
-    if (pl_vh && n && download_aos(st, sub(pl.vh, p0), pl_vh, n)) return SWG_ERR_HIP;
-    if (pl_vb && n && download_aos(st, sub(pl.vb, p0), pl_vb, n)) return SWG_ERR_HIP;
-    if (tp_rh && m && download_aos(st, sub(tp.rh, t0), tp_rh, m)) return SWG_ERR_HIP;
-    if (tp_vh && m && download_aos(st, sub(tp.vh, t0), tp_vh, m)) return SWG_ERR_HIP;
-    if (tp_vb && m && download_aos(st, sub(tp.vb, t0), tp_vb, m)) return SWG_ERR_HIP;
-    if (pl_status && n) HIPCHK(copy_wait(st, pl_status, pl.status + p0, n * sizeof(int32_t), hipMemcpyDeviceToHost));
-    if (tp_status && m) HIPCHK(copy_wait(st, tp_status, tp.status + t0, m * sizeof(int32_t), hipMemcpyDeviceToHost));
+    const XferItem x[] = {xfer_vec3(pl_rh, sub(pl.rh, p0), pl_rh ? n : 0),
+                          xfer_vec3(pl_vh, sub(pl.vh, p0), pl_vh ? n : 0),
+                          xfer_vec3(pl_vb, sub(pl.vb, p0), pl_vb ? n : 0),
+                          xfer_i32(pl_status, pl.status + p0, pl_status ? n : 0),
+                          xfer_vec3(tp_rh, sub(tp.rh, t0), tp_rh ? m : 0),
+                          xfer_vec3(tp_vh, sub(tp.vh, t0), tp_vh ? m : 0),
+                          xfer_vec3(tp_vb, sub(tp.vb, t0), tp_vb ? m : 0),
+                          xfer_i32(tp_status, tp.status + t0, tp_status ? m : 0)};
+    HIPCHK(stage->out(stream, x, 8));
     if (pl_id) std::copy(h_pl_id.begin() + p0, h_pl_id.begin() + p0 + n, pl_id);
     return 0;
 }
@@ -1546,8 +1508,8 @@ int Ensemble::accel(double *pl_acc, double *tp_acc)
     launch_kick_pl(st, tune, pl, sy, pp, d_tiles_pl, ntiles_pl, 1.0, 1, use_radius, 0);
     launch_kick_tp(st, tune, tp, pl, sy, pt, d_tiles_tp, ntiles_tp, 1.0, 1, 0);
     HIPCHK(hipGetLastError());
-    if (pl_acc && npl && download_aos(st, pl.vb, pl_acc, npl)) return SWG_ERR_HIP;
-    if (tp_acc && ntp && download_aos(st, tp.vb, tp_acc, ntp)) return SWG_ERR_HIP;
+    const XferItem x[] = {xfer_vec3(pl_acc, pl.vb, pl_acc ? npl : 0), xfer_vec3(tp_acc, tp.vb, tp_acc ? ntp : 0)};
+    HIPCHK(stage->out(st, x, 2));
     for (int k = 0; k < 2; k++) {
         if (!ns[k]) continue;
         const size_t b = ns[k] * sizeof(double);
@@ -1598,8 +1560,8 @@ int Ensemble::set_frozen(const int32_t *frozen)
         act[s] = !h_frozen[s];
         nfrozen += h_frozen[s];
     }
-    HIPCHK(hipMemcpyAsync(sy.frozen, h_frozen.data(), nsys * sizeof(int32_t), hipMemcpyHostToDevice, stream));
-    HIPCHK(hipMemcpyAsync(d_active, act.data(), nsys * sizeof(int32_t), hipMemcpyHostToDevice, stream));
+    HIPCHK(put(sy.frozen, h_frozen.data(), nsys * sizeof(int32_t)));
+    HIPCHK(put(d_active, act.data(), nsys * sizeof(int32_t)));
     HIPCHK(hipStreamSynchronize(stream));
     return build_tiles();
 }
@@ -1731,6 +1693,7 @@ int swg_system_create(swg_ctx *ctx, const swg_params *prm, int32_t nsys, const i
     std::lock_guard<std::mutex> lk(swg::g_capture_mu);
     swg::Ensemble *e = new swg::Ensemble();
     e->stream = ctx->stream;
+    e->stage = &ctx->leaf->stage;
     int rc = e->create(*prm, nsys, npl, ntp, GMcb, pl_rh, pl_vh, Gmass, radius, rhill, tp_rh, tp_vh);
     if (rc) {
         delete e;
@@ -1772,8 +1735,8 @@ int swg_system_stats(swg_system *sys, swg_stats *st)
     if (!sys || !st) return fail(SWG_ERR_ARG, "NULL argument");
     swg::Ensemble *e = sys->e;
     int32_t dev[4] = {0, 0, 0, 0};
-    HIPCHK(hipStreamSynchronize(e->stream));
-    HIPCHK(copy_wait(e->stream, dev, e->d_sub_stats, sizeof dev, hipMemcpyDeviceToHost));
+    const swg::XferItem res = swg::xfer_i32(dev, e->d_sub_stats, 4);
+    HIPCHK(e->stage->out(e->stream, &res, 1));
     *st = e->st_;
     st->nsubsteps += dev[0];  // substeps run by the persistent recursion kernel
     if (dev[1] > st->max_depth) st->max_depth = dev[1];

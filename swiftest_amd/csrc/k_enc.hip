@@ -340,6 +340,16 @@ __global__ __launch_bounds__(64) void k_rows_fill(ListDev L, const int32_t *row_
     }
 }
 
+__global__ void k_report(const int64_t *total, const int32_t *a, const int32_t *b, int nsys, int64_t *ht, int32_t *hf)
+{
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s == 0 && total) *ht = *total;
+    if (s >= nsys) return;
+    if (a) hf[s] = a[s];
+    if (b) hf[nsys + s] = b[s];
+}
+
+
 // per-system "any pair listed" flags
 __global__ void k_sys_flags(ListDev L, const int32_t *pl_off, int32_t *flag, int nsys)
 {
@@ -562,6 +572,11 @@ void launch_rows_fill(hipStream_t st, ListDev L, const int32_t *row_sys, int upp
 {
     if (nrows)
         k_rows_fill<<<nrows, 64, 0, st>>>(L, row_sys, upper, pl_off, col_off, nrows, lev1g, lev1m, lev2g, lev2m);
+}
+void launch_report(hipStream_t st, const int64_t *total, const int32_t *a, const int32_t *b, int nsys,
+                   int64_t *host_total, int32_t *host_flags)
+{
+    k_report<<<cdiv(nsys, 256), 256, 0, st>>>(total, a, b, nsys, host_total, host_flags);
 }
 void launch_sys_flags(hipStream_t st, ListDev L, const int32_t *pl_off, int32_t *flag, int nsys)
 {

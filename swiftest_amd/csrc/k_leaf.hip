@@ -957,25 +957,14 @@ int Ensemble::whm_snapshot()
     HIPCHK(hipGetLastError());
     if (!prm.rhill_present) {
         std::vector<double> rh(3 * (size_t)npl), vh(3 * (size_t)npl), rhill(npl);
-        HIPCHK(hipStreamSynchronize(stream));
-        std::vector<double> cx(npl), cy(npl), cz(npl);
-        for (int which = 0; which < 2; which++) {
-            Vec3p v = which == 0 ? pl.rh : pl.vh;
-            std::vector<double> &o = which == 0 ? rh : vh;
-            HIPCHK(copy_wait(stream, cx.data(), v.x, npl * sizeof(double), hipMemcpyDeviceToHost));
-            HIPCHK(copy_wait(stream, cy.data(), v.y, npl * sizeof(double), hipMemcpyDeviceToHost));
-            HIPCHK(copy_wait(stream, cz.data(), v.z, npl * sizeof(double), hipMemcpyDeviceToHost));
-            for (int i = 0; i < npl; i++) {
-                o[3 * i] = cx[i];
-                o[3 * i + 1] = cy[i];
-                o[3 * i + 2] = cz[i];
-            }
-        }
+        const XferItem get[] = {xfer_vec3(rh.data(), pl.rh, npl), xfer_vec3(vh.data(), pl.vh, npl)};
+        HIPCHK(stage->out(stream, get, 2));
         for (int s = 0; s < nsys; s++) {
             int b = h_pl_off[s], n = h_pl_off[s + 1] - b;
             host_set_rhill(h_GMcb[s], n, &rh[3 * (size_t)b], &vh[3 * (size_t)b], &h_Gm[b], &rhill[b]);
         }
-        HIPCHK(copy_wait(stream, pl.rhill, rhill.data(), npl * sizeof(double), hipMemcpyHostToDevice));
+        const XferItem put = xfer_words(rhill.data(), pl.rhill, npl);
+        HIPCHK(stage->in(stream, &put, 1));
     }
     return 0;
 }
@@ -1085,6 +1074,13 @@ __global__ void k_na_tiles(int4 *tiles, int nb)
         ib++;
     }
     tiles[t] = make_int4(0, ib, ib + rest, 0);
+}
+
+// the particle tiles (0, tb) of one system
+__global__ void k_pt_tile_list(int4 *tiles, int nb)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < nb) tiles[t] = make_int4(0, t, 0, 0);
 }
 
 // the staged AoS inputs (r, v as (3,n), then renc) into SoA
@@ -1222,16 +1218,15 @@ int swg_kick_getacch_int_all_tri_pl(swg_ctx *ctx, int32_t npl, int32_t nplm, con
     if (radius) {
         GETBUF(t, double, 3, npl);
         dR = t;
-        HIPCHK(hipMemcpyAsync(dR, radius, npl * sizeof(double), hipMemcpyHostToDevice, st));
     }
-    HIPCHK(hipMemcpyAsync(dr, r, 3 * npl * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dg, Gmass, npl * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(da, acc, 3 * npl * sizeof(double), hipMemcpyHostToDevice, st));
+    const XferItem in[] = {xfer_words(r, dr, 3 * (int64_t)npl), xfer_words(Gmass, dg, npl),
+                           xfer_words(acc, da, 3 * (int64_t)npl), xfer_words(radius, dR, radius ? npl : 0)};
+    HIPCHK(ctx->leaf->stage.in(st, in, 4));
     if (npl / RW_LARGE < RW_LARGE_TILES) launch_leaf_tri<RW_SMALL, 4>(st, npl, nplm, dr, dg, dR, da, ctx->pair_mode);
     else launch_leaf_tri<RW_LARGE, 8>(st, npl, nplm, dr, dg, dR, da, ctx->pair_mode);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(acc, da, 3 * npl * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    const XferItem out = xfer_words(acc, da, 3 * (int64_t)npl);
+    HIPCHK(ctx->leaf->stage.out(st, &out, 1));
     return 0;
 }
 
@@ -1304,15 +1299,13 @@ int swg_kick_getacch_int_all_tp(swg_ctx *ctx, int32_t ntp, int32_t npl, const do
     GETBUF(dg, double, 2, npl);
     GETBUF(dm, int32_t, 3, ntp);
     GETBUF(da, double, 4, 3 * ntp);
-    HIPCHK(hipMemcpyAsync(dt_, rtp, 3 * ntp * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dp, rpl, 3 * npl * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dg, GMpl, npl * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dm, lmask, ntp * sizeof(int32_t), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(da, acc, 3 * ntp * sizeof(double), hipMemcpyHostToDevice, st));
+    const XferItem in[] = {xfer_words(rtp, dt_, 3 * (int64_t)ntp), xfer_words(rpl, dp, 3 * (int64_t)npl),
+                           xfer_words(GMpl, dg, npl), xfer_i32(lmask, dm, ntp), xfer_words(acc, da, 3 * (int64_t)ntp)};
+    HIPCHK(ctx->leaf->stage.in(st, in, 5));
     k_leaf_tp<256><<<cdiv(ntp, 256), 256, 0, st>>>(ntp, npl, dt_, dp, dg, dm, da, ctx->pair_mode);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(acc, da, 3 * ntp * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    const XferItem out = xfer_words(acc, da, 3 * (int64_t)ntp);
+    HIPCHK(ctx->leaf->stage.out(st, &out, 1));
     return 0;
 }
 
@@ -1329,17 +1322,13 @@ int swg_drift_all(swg_ctx *ctx, const double *mu, double *x, double *v, int32_t 
     GETBUF(dv, double, 2, 3 * n);
     GETBUF(dm, int32_t, 3, n);
     GETBUF(df, int32_t, 4, n);
-    HIPCHK(hipMemcpyAsync(dmu, mu, n * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dx, x, 3 * n * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dv, v, 3 * n * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dm, lmask, n * sizeof(int32_t), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(df, iflag, n * sizeof(int32_t), hipMemcpyHostToDevice, st));
+    const XferItem in[] = {xfer_words(mu, dmu, n), xfer_words(x, dx, 3 * (int64_t)n), xfer_words(v, dv, 3 * (int64_t)n),
+                           xfer_i32(lmask, dm, n), xfer_i32(iflag, df, n)};
+    HIPCHK(ctx->leaf->stage.in(st, in, 5));
     k_leaf_drift<<<cdiv(n, 128), 128, 0, st>>>(dmu, dx, dv, n, dt, dm, df);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(x, dx, 3 * n * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(v, dv, 3 * n * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(iflag, df, n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    const XferItem out[] = {xfer_words(x, dx, 3 * (int64_t)n), xfer_words(v, dv, 3 * (int64_t)n), xfer_i32(iflag, df, n)};
+    HIPCHK(ctx->leaf->stage.out(st, out, 3));
     return 0;
 }
 
@@ -1373,23 +1362,17 @@ static int leaf_encounter(swg_ctx *ctx, int which, int32_t npl, int32_t ntp, con
     pl.vb = Vec3p{pvx, pvx + npl, pvx + 2 * npl};
     pl.renc = pre;
     pl.sys = psys;
-    std::vector<double> tmp(3 * (size_t)std::max(npl, ntp));
-    auto soa = [&](const double *aos, double *dst, int n) -> int {
-        for (int i = 0; i < n; i++) {
-            tmp[i] = aos[3 * i];
-            tmp[n + i] = aos[3 * i + 1];
-            tmp[2 * n + i] = aos[3 * i + 2];
-        }
-        HIPCHK(copy_wait(st, dst, tmp.data(), 3 * n * sizeof(double), hipMemcpyHostToDevice));
-        return 0;
-    };
-    if ((rc = soa(rpl, prx, npl)) || (rc = soa(vpl, pvx, npl))) return rc;
-    HIPCHK(copy_wait(st, pre, renc, npl * sizeof(double), hipMemcpyHostToDevice));
-    k_fill_i32<<<cdiv(std::max(npl, ntp), 256), 256, 0, st>>>(psys, std::max(npl, ntp), 0);
+    int nb = (ncol + 63) / 64;
+    int64_t z = 0;
     int32_t ho[4] = {0, npl, 0, ntp};
-    HIPCHK(hipMemcpyAsync(offs, ho, sizeof ho, hipMemcpyHostToDevice, st));
     sy.pl_off = offs;
     sy.tp_off = offs + 2;
+    k_fill_i32<<<cdiv(std::max(npl, ntp), 256), 256, 0, st>>>(psys, std::max(npl, ntp), 0);
+    {
+        const XferItem in[] = {xfer_vec3(rpl, pl.rh, npl), xfer_vec3(vpl, pl.vb, npl), xfer_words(renc, pre, npl),
+                               xfer_i32(ho, offs, 4), xfer_words(&z, woff, 1), xfer_i32(&nb, nbp, 1)};
+        HIPCHK(ls.stage.in(st, in, 6));
+    }
     if (which == 1) {
         GETBUF(trx, double, 20, 3 * ntp);
         GETBUF(tvx, double, 21, 3 * ntp);
@@ -1398,11 +1381,11 @@ static int leaf_encounter(swg_ctx *ctx, int which, int32_t npl, int32_t ntp, con
         tp.vb = Vec3p{tvx, tvx + ntp, tvx + 2 * ntp};
         tp.status = tst;
         tp.sys = psys;
-        if ((rc = soa(rtp, trx, ntp)) || (rc = soa(vtp, tvx, ntp))) return rc;
+        const XferItem in[] = {xfer_vec3(rtp, tp.rh, ntp), xfer_vec3(vtp, tp.vb, ntp)};
+        HIPCHK(ls.stage.in(st, in, 2));
         k_fill_i32<<<cdiv(ntp, 256), 256, 0, st>>>(tst, ntp, ACTIVE);
     }
     ListDev &L = ls.L;
-    int nb = (ncol + 63) / 64;
     int64_t words = (int64_t)npl * nb;
     GETBUF(w, uint64_t, 23, words);
     GETBUF(wp, int32_t, 24, words);
@@ -1414,26 +1397,19 @@ static int leaf_encounter(swg_ctx *ctx, int which, int32_t npl, int32_t ntp, con
     L.rowstart = rst;
     L.woff = woff;
     L.nb = nbp;
-    int64_t z = 0;
-    HIPCHK(hipMemcpyAsync(woff, &z, sizeof z, hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(nbp, &nb, sizeof nb, hipMemcpyHostToDevice, st));
-    std::vector<int4> ht;
+    const int ntiles = which == 0 ? nb * (nb + 1) / 2 : nb;
     if (which == 0) {
-        for (int ib = 0; ib < nb; ib++)
-            for (int jb = ib; jb < nb; jb++) ht.push_back(make_int4(0, ib, jb, 0));
+        k_na_tiles<<<cdiv(ntiles, 256), 256, 0, st>>>(tiles, nb);
+        launch_pp_tiles(st, pl, sy, L, tiles, ntiles, dt);
     } else {
-        for (int tb = 0; tb < nb; tb++) ht.push_back(make_int4(0, tb, 0, 0));
+        k_pt_tile_list<<<cdiv(ntiles, 256), 256, 0, st>>>(tiles, nb);
+        launch_pt_tiles(st, pl, tp, sy, L, tiles, ntiles, dt);
     }
-    HIPCHK(hipMemcpyAsync(tiles, ht.data(), ht.size() * sizeof(int4), hipMemcpyHostToDevice, st));
-    if (which == 0)
-        launch_pp_tiles(st, pl, sy, L, tiles, (int)ht.size(), dt);
-    else
-        launch_pt_tiles(st, pl, tp, sy, L, tiles, (int)ht.size(), dt);
     launch_rows_count(st, L, psys, which == 0, offs, nullptr, npl);
     launch_scan_i32_i64(st, rcnt, rst, npl, tot, scan);
     int64_t n = 0;
-    HIPCHK(hipMemcpyAsync(&n, tot, sizeof n, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    const XferItem total = xfer_words(&n, tot, 1);
+    HIPCHK(ls.stage.out(st, &total, 1));
     if (n > ls.cap) {
         for (void *q : {(void *)L.i1, (void *)L.i2, (void *)L.lvdotr, (void *)L.status, (void *)L.level})
             if (q) (void)hipFree(q);
@@ -1445,9 +1421,9 @@ static int leaf_encounter(swg_ctx *ctx, int which, int32_t npl, int32_t ntp, con
         HIPCHK(hipMalloc((void **)&L.level, c));
         ls.cap = c;
     }
+    // (the fill is waited for by swg_encounter_list_copy, on the same stream)
     if (n) launch_rows_fill(st, L, psys, which == 0, offs, offs + (which == 0 ? 0 : 2), npl);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(st));
     ls.nenc = n;
     *nenc = n;
     return 0;
@@ -1493,10 +1469,9 @@ int swg_encounter_list_copy(swg_ctx *ctx, int32_t *index1, int32_t *index2, int3
     k_copy_i32_plus1<<<cdiv(n, 256), 256, 0, st>>>(ls.L.i1, a, ls.L.lvdotr, c, n);
     k_copy_i32_plus1<<<cdiv(n, 256), 256, 0, st>>>(ls.L.i2, b, nullptr, nullptr, n);
     HIPCHK(hipGetLastError());
-    if (index1) HIPCHK(hipMemcpyAsync(index1, a, n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    if (index2) HIPCHK(hipMemcpyAsync(index2, b, n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    if (lvdotr) HIPCHK(hipMemcpyAsync(lvdotr, c, n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    const XferItem out[] = {xfer_i32(index1, a, index1 ? n : 0), xfer_i32(index2, b, index2 ? n : 0),
+                            xfer_i32(lvdotr, c, lvdotr ? n : 0)};
+    HIPCHK(ls.stage.out(st, out, 3));
     return 0;
 }
 

@@ -6,6 +6,7 @@
 
 #include "../../include/swiftest_hip.h"
 #include "swg_kernels.h"
+#include "swg_stage.h"
 
 namespace swg {
 
@@ -37,6 +38,7 @@ inline void pad_position(int k, double *r)
 // A resident ensemble of independent systems.
 struct Ensemble {
     hipStream_t stream = nullptr;
+    Stage *stage = nullptr;  // the context's transfer ring
     swg_params prm{};
     Tuning tune{};
     int nsys = 0, npl = 0, ntp = 0;
@@ -194,6 +196,7 @@ struct Ensemble {
     int get_bodies(int32_t *id, double *mass, double *Gmass, double *radius);
 
     // internals
+    hipError_t put(void *dev, const void *host, size_t bytes);
     template <class T> int own(T **p, size_t n);
     template <class T> int own2(T **p, size_t n);
     int alloc_vec(Vec3p &v, size_t n);
@@ -226,6 +229,7 @@ struct LeafState {
     int64_t nenc = 0, cap = 0;
     ~LeafState();
     void *get(int slot, size_t bytes, int *rc);
+    Stage stage;  // transfers of every call on the context, resident systems included
 };
 
 }  // namespace swg

@@ -117,6 +117,10 @@ void launch_scan_small(hipStream_t st, const ScanSmall &a, int na);
 void launch_rows_fill(hipStream_t st, ListDev L, const int32_t *row_sys, int upper, const int32_t *pl_off,
                       const int32_t *col_off, int nrows, int32_t *lev1g = nullptr, int32_t *lev1m = nullptr,
                       int32_t *lev2g = nullptr, int32_t *lev2m = nullptr);
+// a total and up to two per-system arrays (any may be NULL) straight into
+// pinned host memory: total[0], flags[0, nsys) and flags[nsys, 2 nsys)
+void launch_report(hipStream_t st, const int64_t *total, const int32_t *a, const int32_t *b, int nsys,
+                   int64_t *host_total, int32_t *host_flags);
 void launch_sys_flags(hipStream_t st, ListDev L, const int32_t *pl_off, int32_t *flag, int nsys);
 // index2-side adjacency (counts, then fill) of a list whose bit matrix is in
 // L.words; cb_off: each system's first 64-column block (nsys + 1 entries)
