@@ -516,7 +516,8 @@ int Ensemble::detect_pp_sas(double dt)
     return 0;
 }
 
-// Level-0 pl-tp detection for the systems in `run`.
+// Level-0 pl-tp detection for the systems in `run` (the flags of the others
+// stay clear).
 int Ensemble::detect_pt(double dt, const std::vector<int32_t> &run)
 {
     hipStream_t st = stream;
@@ -527,10 +528,7 @@ int Ensemble::detect_pt(double dt, const std::vector<int32_t> &run)
         int m = h_tp_off[s + 1] - h_tp_off[s];
         for (int tb = 0; tb < (m + 63) / 64; tb++) tiles.push_back(make_int4(s, tb, 0, 0));
     }
-    if (tiles.empty()) {
-        HIPCHK(hipMemsetAsync(sy.enc_pt, 0, nsys * sizeof(int32_t), st));
-        return 0;
-    }
+    if (tiles.empty()) return 0;
     if (!pt.words) {
         HIPCHK(dalloc(&pt.words, pt_words));
         HIPCHK(dalloc(&pt.wpre, pt_words));
@@ -1026,8 +1024,7 @@ int Ensemble::step_helio_symba()
     st_.npltp_enc = 0;
     st_.max_depth = -1;
     st_.nsubsteps = 0;
-    launch_reset_levels(st, pl, tp, npl, ntp);
-    HIPCHK(hipMemsetAsync(d_sub_stats, 0, 4 * sizeof(int32_t), st));
+    launch_reset_levels(st, pl, tp, sy, d_sub_stats, npl, ntp, nsys);
     npp = npt = 0;
     bool any = false;
     if (symba) {
@@ -1042,19 +1039,13 @@ int Ensemble::step_helio_symba()
             anyrun |= run[s] != 0;
         }
         h_enc_pt.assign(nsys, 0);
-        if (anyrun) {
+        if (anyrun)
             if (int rc = detect_pt(dt, run)) return rc;
-        } else {
-            HIPCHK(hipMemsetAsync(sy.enc_pt, 0, nsys * sizeof(int32_t), st));
-        }
         for (int s = 0; s < nsys; s++) any |= h_enc_pp[s] || h_enc_pt[s];
         st_.nplpl_enc = npp;
         st_.npltp_enc = npt;
         if (any) build_adjacency();
         trace_mark(st, "detect pl-tp+adj");
-    } else {
-        HIPCHK(hipMemsetAsync(sy.enc_pp, 0, nsys * sizeof(int32_t), st));
-        HIPCHK(hipMemsetAsync(sy.enc_pt, 0, nsys * sizeof(int32_t), st));
     }
     const int use_radius = symba || prm.lclose;
     auto kick_pl = [&](int lbeg) -> int {
@@ -1528,7 +1519,7 @@ int Ensemble::time_encounters(int reps, double *ms, int64_t *npairs, int64_t *nc
 {
     if (prm.integrator != SWG_SYMBA) return fail(SWG_ERR_ARG, "encounter checks run in SyMBA only");
     const double dt = prm.dt;
-    launch_reset_levels(stream, pl, tp, npl, ntp);  // the step's start: levels and level-0 renc
+    launch_reset_levels(stream, pl, tp, sy, nullptr, npl, ntp, nsys);  // the step's start: levels and level-0 renc
     if (int rc = prm.encounter_check == 1 ? detect_pp_sas(dt) : detect_pp(dt)) return rc;  // warm-up
     HIPCHK(hipStreamSynchronize(stream));
     auto t0 = std::chrono::steady_clock::now();

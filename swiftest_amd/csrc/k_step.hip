@@ -25,10 +25,25 @@ constexpr int KTP_G = SWG_KTP_G;
 __device__ inline bool pl_active(const PlDev &pl, int i) { return pl.status[i] != INACTIVE; }
 __device__ inline bool tp_active(const TpDev &tp, int j) { return tp.status[j] == ACTIVE; }
 
+// Block y copies array y.
+__global__ void k_copy_list(CopyList c)
+{
+    const CopyItem it = c.item[blockIdx.y];
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < it.n; i += (int64_t)gridDim.x * blockDim.x)
+        it.dst[i] = it.src[i];
+}
+
 // symba_step_reset_system (symba_step.f90:265-331): recursion levels to -1
-__global__ void k_reset_levels(PlDev pl, TpDev tp, int npl, int ntp)
+// and encounter radii of level 0; the systems' encounter flags and the
+// recursion's counters are cleared with them
+__global__ void k_reset_levels(PlDev pl, TpDev tp, SysDev sy, int32_t *sub_stats, int npl, int ntp, int nsys)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nsys) {
+        sy.enc_pp[i] = 0;
+        sy.enc_pt[i] = 0;
+    }
+    if (sub_stats && i < 4) sub_stats[i] = 0;
     if (i < npl) {
         pl.levelg[i] = -1;
         pl.levelm[i] = -1;
@@ -41,48 +56,110 @@ __global__ void k_reset_levels(PlDev pl, TpDev tp, int npl, int ntp)
 }
 
 // Per-system sums, one workgroup per system.  Each sum is a serial chain in
-// the reference's order.  The whole workgroup stages a chunk of the system's
-// bodies in LDS as the terms of the sums (products and quotients formed in
-// parallel, each exactly as the serial expression forms it), and one lane
-// per sum adds them in order (a chain streaming from HBM would wait on every
-// load, one forming its own terms on its serial path).
-constexpr int SUM_T = 256, SUM_CH = 1024;
+// the reference's order.  The bodies go through LDS a chunk at a time as the
+// terms of the sums (products and quotients formed in parallel, each exactly as
+// the serial expression forms it): three wavefronts stage a chunk while the
+// first one's lanes, one per sum, add the chunk before.  Bound: the chains'
+// dependent adds, about 10 cycles each.  Measured at 2000 bodies: k_sums_begin
+// (two walks, the second after the first) 61 -> 26 us, k_sums_end (its two walks
+// side by side) 53 -> 14.5 us, against staging and adding in turn with eight
+// terms read ahead.
+constexpr int SUM_T = 256, SUM_CH = 384;
 
 struct SumStage {
-    double t[4][SUM_CH];  // the terms of up to four sums
+    // the terms of up to six sums; two words more a row than the banks wrap at,
+    // so the lanes' reads fall on different ones
+    __align__(16) double t[2][6][SUM_CH + 2];
 };
 
-// The serial chains over a staged chunk, in order: acc + t[0] + ... + t[n-1]
-// (SUB false) or acc - t[0] - ... - t[n-1] (SUB true), walking t[n-1] down to
-// t[0] when BACK.  The reads of the next eight terms are issued before the
-// adds of the current eight.  A body a masked sum skips stages +0.0
-// instead: the chains start at +0.0, a sum that starts at +0 is never -0
-// (x + (-x) = +0 in round-to-nearest), and s + (+0) = s, s - (+0) = s bit
-// for bit for every other s, so the sums are the masked ones exactly.
-template <bool SUB, bool BACK>
+// The serial chain over a staged chunk: acc + t[0] + ... + t[n-1] in order.
+// The reads of the next 32 terms are issued before the adds of the current 32, in two sets of registers that change places.  A sum that subtracts
+// stages its terms negated (s - x = s + (-x) bit for bit), and a body a masked
+// sum skips stages +0.0 instead: the chains start at +0.0, a sum that starts at
+// +0 is never -0 (x + (-x) = +0 in round-to-nearest), and s + (+0) = s bit for
+// bit for every other s, so the sums are the masked ones exactly.
 __device__ inline double chain(double acc, const double *t, int n)
 {
-    auto at = [&](int k) { return BACK ? t[n - 1 - k] : t[k]; };
-    auto step = [](double s, double x) { return SUB ? s - x : s + x; };
-    int k = 0;
-    if (n >= 8) {
-        double v[8];
+    constexpr int G = 16;  // pairs of terms per set
+    const double2 *t2 = (const double2 *)t;
+    const int sets = n / (2 * G);
+    double2 v[G], w[G];
+    auto read = [&](double2 *o, int g) {
 #pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = at(u);
-        for (k = 8; k + 8 <= n; k += 8) {
-            double w[8];
+        for (int u = 0; u < G; u++) o[u] = t2[G * g + u];
+    };
+    auto add = [&](const double2 *o) {
 #pragma unroll
-            for (int u = 0; u < 8; u++) w[u] = at(k + u);
-#pragma unroll
-            for (int u = 0; u < 8; u++) acc = step(acc, v[u]);
-#pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = w[u];
+        for (int u = 0; u < G; u++) {
+            acc += o[u].x;
+            acc += o[u].y;
         }
-#pragma unroll
-        for (int u = 0; u < 8; u++) acc = step(acc, v[u]);
+    };
+    if (sets > 0) {
+        read(v, 0);
+        for (int g = 0; g < sets; g += 2) {
+            read(w, min(g + 1, sets - 1));
+            add(v);
+            if (g + 1 == sets) break;
+            read(v, min(g + 2, sets - 1));
+            add(w);
+        }
     }
-    for (; k < n; k++) acc = step(acc, at(k));
+    for (int k = 2 * G * sets; k < n; k++) acc += t[k];
     return acc;
+}
+
+// What the sums need of a body.
+struct SumBody {
+    double g, x, y, z;
+    bool act;
+};
+__device__ inline SumBody sum_body(const PlDev &pl, const Vec3p &v, int i)
+{
+    return SumBody{pl.Gm[i], v.x[i], v.y[i], v.z[i], pl.status[i] != INACTIVE};
+}
+
+// Chunks of bodies [p0, p1): for k = 0 ... n-1 the staging wavefronts call
+// stage(b, k, body k of the chunk), and a chunk later the first one calls
+// add(b, n); b is the buffer.  BOTH: stage also gets body k of the chunk as
+// counted from the end of the range.  The bodies' loads are issued a chunk
+// ahead of their staging, so that their latency passes behind the adds.
+template <bool BOTH, class StageF, class AddF>
+__device__ inline void sums_chunks(const PlDev &pl, const Vec3p &v, int p0, int p1, StageF stage, AddF add)
+{
+    constexpr int W = SUM_T - 64, U = SUM_CH / W;
+    static_assert(U * W == SUM_CH, "whole rounds");
+    const int tid = threadIdx.x, n = p1 - p0, nch = (n + SUM_CH - 1) / SUM_CH;
+    if (n <= 0) return;
+    if (tid >= 64) {
+        SumBody f[U], r[U];
+        auto load = [&](int c) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int k = min(c * SUM_CH + tid - 64 + u * W, n - 1);
+                f[u] = sum_body(pl, v, p0 + k);
+                if (BOTH) r[u] = sum_body(pl, v, p1 - 1 - k);
+            }
+        };
+        load(0);
+        for (int c = 0; c <= nch; c++) {
+            SumBody a[U], b[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) a[u] = f[u], b[u] = BOTH ? r[u] : f[u];
+            if (c + 1 < nch) load(c + 1);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int k = tid - 64 + u * W;
+                if (c * SUM_CH + k < n) stage(c & 1, k, a[u], b[u]);
+            }
+            __syncthreads();
+        }
+    } else {
+        for (int c = 0; c <= nch; c++) {
+            if (c > 0) add((c - 1) & 1, min(SUM_CH, n - (c - 1) * SUM_CH));
+            __syncthreads();
+        }
+    }
 }
 
 // The sums of vh2vb (swiftest_util.f90:424-459) over bodies [p0, p1): lane 0
@@ -91,23 +168,17 @@ __device__ inline double sums_gm_vh(SumStage &S, const PlDev &pl, int p0, int p1
 {
     const int tid = threadIdx.x;
     double acc = 0.0;
-    for (int c0 = p0; c0 < p1; c0 += SUM_CH) {
-        const int n = min(SUM_CH, p1 - c0);
-        for (int k = tid; k < n; k += SUM_T) {
-            const int i = c0 + k;
-            const double g = pl.Gm[i];
-            S.t[0][k] = g;
-            S.t[1][k] = g * pl.vh.x[i];
-            S.t[2][k] = g * pl.vh.y[i];
-            S.t[3][k] = g * pl.vh.z[i];
-        }
-        __syncthreads();
-        if (tid == 0)
-            acc = chain<false, false>(acc, S.t[0], n);
-        else if (tid <= 3)
-            acc = chain<true, false>(acc, S.t[tid], n);
-        __syncthreads();
-    }
+    sums_chunks<false>(
+        pl, pl.vh, p0, p1,
+        [&](int b, int k, const SumBody &q, const SumBody &) {
+            S.t[b][0][k] = q.g;
+            S.t[b][1][k] = -(q.g * q.x);
+            S.t[b][2][k] = -(q.g * q.y);
+            S.t[b][3][k] = -(q.g * q.z);
+        },
+        [&](int b, int n) {
+            if (tid < 4) acc = chain(acc, S.t[b][tid], n);
+        });
     return acc;
 }
 
@@ -137,23 +208,19 @@ __global__ __launch_bounds__(SUM_T) void k_sums_begin(PlDev pl, SysDev sy, int n
     }
     const Vec3p v = first ? pl.vh : pl.vb;
     double pt = 0.0;
-    for (int c0 = p0; c0 < p1; c0 += SUM_CH) {
-        const int n = min(SUM_CH, p1 - c0);
-        for (int k = tid; k < n; k += SUM_T) {
-            const int i = c0 + k;
-            const double g = pl.Gm[i];
-            const bool act = pl.status[i] != INACTIVE;
-            const double wx = first ? v.x[i] + scb[0] : v.x[i];
-            const double wy = first ? v.y[i] + scb[1] : v.y[i];
-            const double wz = first ? v.z[i] + scb[2] : v.z[i];
-            S.t[0][k] = act ? g * wx : 0.0;
-            S.t[1][k] = act ? g * wy : 0.0;
-            S.t[2][k] = act ? g * wz : 0.0;
-        }
-        __syncthreads();
-        if (tid < 3) pt = chain<false, false>(pt, S.t[tid], n);
-        __syncthreads();
-    }
+    sums_chunks<false>(
+        pl, v, p0, p1,
+        [&](int b, int k, const SumBody &q, const SumBody &) {
+            const double wx = first ? q.x + scb[0] : q.x;
+            const double wy = first ? q.y + scb[1] : q.y;
+            const double wz = first ? q.z + scb[2] : q.z;
+            S.t[b][0][k] = q.act ? q.g * wx : 0.0;
+            S.t[b][1][k] = q.act ? q.g * wy : 0.0;
+            S.t[b][2][k] = q.act ? q.g * wz : 0.0;
+        },
+        [&](int b, int n) {
+            if (tid < 3) pt = chain(pt, S.t[b][tid], n);
+        });
     if (tid < 3) sy.ptbeg[3 * s + tid] = pt / sy.GMcb[s];
 }
 
@@ -796,7 +863,8 @@ __global__ __launch_bounds__(BLK) void k_kick_tp(TpDev tp, PlDev pl, SysDev sy, 
 // Per-system sums at the end of a step:
 //   lindrift pt = sum_masked(Gm vb) / GM_cb -> ptend (forward, lanes 0-2)
 //   vb->vh (swiftest_util.f90:363-395): cb%vb -= Gm vb / GM_cb over
-//   i = npl..1, active only (backward, lanes 0-2)
+//   i = npl..1, active only (backward, lanes 3-5): the two walk the bodies
+//   from both ends side by side
 __global__ __launch_bounds__(SUM_T) void k_sums_end(PlDev pl, SysDev sy, int nsys)
 {
     __shared__ SumStage S;
@@ -804,38 +872,22 @@ __global__ __launch_bounds__(SUM_T) void k_sums_end(PlDev pl, SysDev sy, int nsy
     const int p0 = sy.pl_off[s], p1 = sy.pl_off[s + 1];
     if (p1 == p0 || sy.frozen[s]) return;
     const double gm = sy.GMcb[s];
-    double pt = 0.0;
-    for (int c0 = p0; c0 < p1; c0 += SUM_CH) {
-        const int n = min(SUM_CH, p1 - c0);
-        for (int k = tid; k < n; k += SUM_T) {
-            const int i = c0 + k;
-            const double g = pl.Gm[i];
-            const bool act = pl.status[i] != INACTIVE;
-            S.t[0][k] = act ? g * pl.vb.x[i] : 0.0;
-            S.t[1][k] = act ? g * pl.vb.y[i] : 0.0;
-            S.t[2][k] = act ? g * pl.vb.z[i] : 0.0;
-        }
-        __syncthreads();
-        if (tid < 3) pt = chain<false, false>(pt, S.t[tid], n);
-        __syncthreads();
-    }
-    if (tid < 3) sy.ptend[3 * s + tid] = pt / gm;
-    double c = 0.0;
-    for (int c1 = p1; c1 > p0; c1 -= SUM_CH) {
-        const int c0 = max(p0, c1 - SUM_CH), n = c1 - c0;
-        for (int k = tid; k < n; k += SUM_T) {
-            const int i = c0 + k;
-            const double g = pl.Gm[i];
-            const bool act = pl.status[i] != INACTIVE;
-            S.t[0][k] = act ? (g * pl.vb.x[i]) / gm : 0.0;
-            S.t[1][k] = act ? (g * pl.vb.y[i]) / gm : 0.0;
-            S.t[2][k] = act ? (g * pl.vb.z[i]) / gm : 0.0;
-        }
-        __syncthreads();
-        if (tid < 3) c = chain<true, true>(c, S.t[tid], n);
-        __syncthreads();
-    }
-    if (tid < 3) sy.cbvb[3 * s + tid] = c;
+    double acc = 0.0;
+    sums_chunks<true>(
+        pl, pl.vb, p0, p1,
+        [&](int b, int k, const SumBody &q, const SumBody &r) {
+            S.t[b][0][k] = q.act ? q.g * q.x : 0.0;
+            S.t[b][1][k] = q.act ? q.g * q.y : 0.0;
+            S.t[b][2][k] = q.act ? q.g * q.z : 0.0;
+            S.t[b][3][k] = r.act ? -((r.g * r.x) / gm) : 0.0;
+            S.t[b][4][k] = r.act ? -((r.g * r.y) / gm) : 0.0;
+            S.t[b][5][k] = r.act ? -((r.g * r.z) / gm) : 0.0;
+        },
+        [&](int b, int n) {
+            if (tid < 6) acc = chain(acc, S.t[b][tid], n);
+        });
+    if (tid < 3) sy.ptend[3 * s + tid] = acc / gm;
+    else if (tid < 6) sy.cbvb[3 * s + tid - 3] = acc;
 }
 
 // rh += ptend*dt (masked); vh = vb - cb%vb (all bodies)
@@ -961,10 +1013,16 @@ __global__ void k_init_tp_vb(TpDev tp, SysDev sy, int ntp)
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-void launch_reset_levels(hipStream_t st, PlDev pl, TpDev tp, int npl, int ntp)
+void launch_copy_list(hipStream_t st, const CopyList &c)
 {
-    int n = npl > ntp ? npl : ntp;
-    if (n) k_reset_levels<<<cdiv(n, 256), 256, 0, st>>>(pl, tp, npl, ntp);
+    int64_t n = 0;
+    for (int i = 0; i < c.n; i++) n = std::max(n, c.item[i].n);
+    if (n) k_copy_list<<<dim3((unsigned)std::min<int64_t>((n + 255) / 256, 256), c.n), 256, 0, st>>>(c);
+}
+void launch_reset_levels(hipStream_t st, PlDev pl, TpDev tp, SysDev sy, int32_t *sub_stats, int npl, int ntp, int nsys)
+{
+    const int n = std::max(std::max(npl, ntp), std::max(nsys, 4));
+    k_reset_levels<<<cdiv(n, 256), 256, 0, st>>>(pl, tp, sy, sub_stats, npl, ntp, nsys);
 }
 void launch_sums_begin(hipStream_t st, PlDev pl, SysDev sy, int nsys, int force)
 {

@@ -237,23 +237,27 @@ void Ensemble::merge_reset_system(int s)
 // step uses is rebuilt at its start (levels, renc, lists, flags).
 int Ensemble::merge_save(bool restore)
 {
-    hipStream_t st = stream;
-    auto cp = [&](void *a, void *b, size_t bytes) -> int {
-        if (bytes) MCHK(hipMemcpyAsync(restore ? a : b, restore ? b : a, bytes, hipMemcpyDeviceToDevice, st));
-        return 0;
+    // one launch for all arrays: they are short, and fifteen copies one by one
+    // were about 60 us of a step of 2000 bodies
+    CopyList c;
+    c.n = 0;
+    auto cp = [&](void *a, void *b, size_t words) {
+        c.item[c.n++] = CopyItem{(const uint32_t *)(restore ? b : a), (uint32_t *)(restore ? a : b), (int64_t)words};
     };
-    const size_t n = (size_t)npl * sizeof(double);
+    const size_t n = 2 * (size_t)npl, ns = nsys;
     for (auto pr : {std::make_pair(pl.rh, mb_rh), std::make_pair(pl.vh, mb_vh), std::make_pair(pl.vb, mb_vb)}) {
-        if (int rc = cp(pr.first.x, pr.second.x, n)) return rc;
-        if (int rc = cp(pr.first.y, pr.second.y, n)) return rc;
-        if (int rc = cp(pr.first.z, pr.second.z, n)) return rc;
+        cp(pr.first.x, pr.second.x, n);
+        cp(pr.first.y, pr.second.y, n);
+        cp(pr.first.z, pr.second.z, n);
     }
-    if (int rc = cp(pl.status, mb_status, (size_t)npl * sizeof(int32_t))) return rc;
-    if (int rc = cp(sy.lfirst, mb_sys, nsys * sizeof(int32_t))) return rc;
-    if (int rc = cp(sy.err, mb_sys + nsys, nsys * sizeof(int32_t))) return rc;
-    if (int rc = cp(sy.cbvb, mb_cb, 3 * nsys * sizeof(double))) return rc;
-    if (int rc = cp(sy.ptbeg, mb_cb + 3 * nsys, 3 * nsys * sizeof(double))) return rc;
-    if (int rc = cp(sy.ptend, mb_cb + 6 * nsys, 3 * nsys * sizeof(double))) return rc;
+    cp(pl.status, mb_status, npl);
+    cp(sy.lfirst, mb_sys, ns);
+    cp(sy.err, mb_sys + nsys, ns);
+    cp(sy.cbvb, mb_cb, 6 * ns);
+    cp(sy.ptbeg, mb_cb + 3 * nsys, 6 * ns);
+    cp(sy.ptend, mb_cb + 6 * nsys, 6 * ns);
+    launch_copy_list(stream, c);
+    MCHK(hipGetLastError());
     return 0;
 }
 

@@ -56,7 +56,18 @@ inline int Tuning::pl_tile() const
 }
 
 // ---- step kernels (k_step.hip) ----
-void launch_reset_levels(hipStream_t st, PlDev pl, TpDev tp, int npl, int ntp);
+void launch_reset_levels(hipStream_t st, PlDev pl, TpDev tp, SysDev sy, int32_t *sub_stats, int npl, int ntp, int nsys);
+// device arrays copied to others in one launch, counted in 4-byte words
+struct CopyItem {
+    const uint32_t *src;
+    uint32_t *dst;
+    int64_t n;
+};
+struct CopyList {
+    CopyItem item[16];
+    int n;
+};
+void launch_copy_list(hipStream_t st, const CopyList &c);
 void launch_sums_begin(hipStream_t st, PlDev pl, SysDev sy, int nsys, int force_vh2vb);
 void launch_pl_begin_apply(hipStream_t st, PlDev pl, SysDev sy, int npl, double dth, int force_vh2vb);
 void launch_kick_pl(hipStream_t st, const Tuning &tu, PlDev pl, SysDev sy, ListDev pp, const Tile *tiles,
