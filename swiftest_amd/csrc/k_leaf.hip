@@ -56,14 +56,14 @@ __device__ inline void one_pl_half(double rji2, double xr, double yr, double zr,
 // swiftest_kick_getacch_int_all_tri_{rad,norad}_pl (swiftest_kick.f90:165-371):
 // the rows of B bodies per workgroup, the terms evaluated by several
 // wavefronts and folded in partner order by others (swg_rows.h).
-template <int B, int KE, bool TRI, bool FAST>
-__global__ __launch_bounds__((RowsLds<B, KE>::THREADS), (RowsLds<B, KE>::WAVES)) void k_leaf_tri(int npl, int nplm, const double *r,
+template <int B, int KE, int A, bool TRI, bool FAST>
+__global__ __launch_bounds__((RowsLds<B, KE, A>::THREADS), (RowsLds<B, KE, A>::WAVES)) void k_leaf_tri(int npl, int nplm, const double *r,
                                                                       const double *Gm, const double *R, double *acc)
 {
-    __shared__ RowsLds<B, KE> S;
+    __shared__ RowsLds<B, KE, A> S;
     const int b0 = (int)blockIdx.x * B, b1 = min(b0 + B, npl);
-    const RowsSrc src{r, r + 1, r + 2, Gm, R, 3};
-    rows_sums<true, false>(S, src, [&](int comp, int i) { return acc[3 * (int64_t)i + comp]; }, b0, b1, nplm, npl, TRI, FAST,
+    const RowsSrc src{r, r + 1, r + 2, Gm, R ? R : Gm, 3};
+    rows_sums<true, false, true>(S, src, src, [&](int comp, int i) { return acc[3 * (int64_t)i + comp]; }, b0, b1, nplm, npl, TRI, FAST,
               R != nullptr);
     const int bl = (int)threadIdx.x % B, b = b0 + bl, comp = (int)threadIdx.x / B;
     if (comp >= 3 || b >= b1) return;
@@ -72,12 +72,11 @@ __global__ __launch_bounds__((RowsLds<B, KE>::THREADS), (RowsLds<B, KE>::WAVES))
     *o = TRI ? (*o + S.out[1][comp][bl]) + v : v;
 }
 
-template <int B, int KE>
+template <int B, int KE, int A, bool TRI>
 static void launch_leaf_tri(hipStream_t st, int npl, int nplm, const double *r, const double *Gm, const double *R,
                             double *acc, bool fast)
 {
-    const auto kern = npl - nplm > nplm ? (fast ? k_leaf_tri<B, KE, true, true> : k_leaf_tri<B, KE, true, false>)
-                                        : (fast ? k_leaf_tri<B, KE, false, true> : k_leaf_tri<B, KE, false, false>);
+    const auto kern = fast ? k_leaf_tri<B, KE, A, TRI, true> : k_leaf_tri<B, KE, A, TRI, false>;
     kern<<<cdiv(npl, B), RowsLds<B, KE>::THREADS, 0, st>>>(npl, nplm, r, Gm, R, acc);
 }
 
@@ -119,48 +118,105 @@ __global__ void k_leaf_flat(int npl, const int32_t *k, const double *r, const do
 }
 
 // swiftest_kick_getacch_int_all_tp (swiftest_kick.f90:374-415): particle sum
-// from zero over pl ascending, added to acc once (OpenMP reduction).
-template <int BLK>
-__global__ __launch_bounds__(BLK) void k_leaf_tp(int ntp, int npl, const double *rtp, const double *rpl,
-                                                 const double *Gm, const int32_t *lmask, double *acc, int fast)
+// from zero over pl ascending, added to acc once (OpenMP reduction).  A
+// wavefront of 64 particles, one lane each; the massive bodies pass through LDS
+// 64 at a time, the next ones loaded meanwhile, and the factors of four at a
+// time are formed side by side without branches (the rare out-of-range ones
+// redone with the IEEE operations under a wave-uniform test).  Bound: FP64
+// issue, one or two wavefronts a SIMD.  Measured, 100003 particles x 500
+// bodies, term by term before: 136 -> 90 us.
+template <bool FAST>
+__global__ __launch_bounds__(64) void k_leaf_tp(int ntp, int npl, const double *rtp, const double *rpl, const double *Gm,
+                                                const int32_t *lmask, double *acc)
 {
-    __shared__ double sx[BLK], sy[BLK], sz[BLK], sg[BLK];
-    int t = blockIdx.x * BLK + threadIdx.x;
-    bool valid = t < ntp && lmask[t] != 0;
-    double xt = 0, yt = 0, zt = 0;
-    if (valid) {
-        xt = rtp[3 * t];
-        yt = rtp[3 * t + 1];
-        zt = rtp[3 * t + 2];
-    }
-    double px = 0.0, py = 0.0, pz = 0.0;
-    for (int j0 = 0; j0 < npl; j0 += BLK) {
-        int j = j0 + threadIdx.x;
-        if (j < npl) {
-            sx[threadIdx.x] = rpl[3 * j];
-            sy[threadIdx.x] = rpl[3 * j + 1];
-            sz[threadIdx.x] = rpl[3 * j + 2];
-            sg[threadIdx.x] = Gm[j];
-        }
+    constexpr int G = 4;
+    __shared__ __align__(16) double sb[64][4];
+    const int lane = threadIdx.x, t = blockIdx.x * 64 + lane, tc = min(t, ntp - 1);
+    const double xt = rtp[3 * (int64_t)tc], yt = rtp[3 * (int64_t)tc + 1], zt = rtp[3 * (int64_t)tc + 2];
+    const bool valid = t < ntp && lmask[tc] != 0;
+    double px = 0.0, py = 0.0, pz = 0.0, nx[4];
+    auto fetch = [&](int j0) {
+        const int64_t j = min(j0 + lane, npl - 1);
+        nx[0] = rpl[3 * j];
+        nx[1] = rpl[3 * j + 1];
+        nx[2] = rpl[3 * j + 2];
+        nx[3] = Gm[j];
+    };
+    fetch(0);
+    for (int j0 = 0; j0 < npl; j0 += 64) {
         __syncthreads();
-        int jn = min(BLK, npl - j0);
-        if (valid) {
-            for (int q = 0; q < jn; q++) {
-                double rx = xt - sx[q], ry = yt - sy[q], rz = zt - sz[q];
-                double rji2 = dot3(rx, ry, rz, rx, ry, rz);
-                double fac = fast ? gm_over_r3_fast(sg[q], rji2) : gm_over_r3(sg[q], rji2, pair_g_ok(sg[q]));
-                px = fma(-fac, rx, px);
-                py = fma(-fac, ry, py);
-                pz = fma(-fac, rz, pz);
+#pragma unroll
+        for (int a = 0; a < 4; a++) sb[lane][a] = nx[a];
+        const bool gok = __all(pair_g_ok_int(nx[3]));
+        if (j0 + 64 < npl) fetch(j0 + 64);
+        __syncthreads();
+        const int jn = min(64, npl - j0);
+        int q = 0;
+        for (; q + G <= jn; q += G) {
+            double rx[G], ry[G], rz[G], r2[G], m[G], f[G];
+            uint32_t far = 0;
+#pragma unroll
+            for (int u = 0; u < G; u++) {
+                rx[u] = xt - sb[q + u][0];
+                ry[u] = yt - sb[q + u][1];
+                rz[u] = zt - sb[q + u][2];
+                m[u] = sb[q + u][3];
+                r2[u] = dot3(rx[u], ry[u], rz[u], rx[u], ry[u], rz[u]);
+                if (FAST) f[u] = gm_over_r3_fast(m[u], r2[u]);
+                else far = max(far, (uint32_t)(__double2hiint(r2[u]) - PAIR_R2_LO_HI));
+            }
+            if (!FAST) {
+                pair_factors<G>(m, r2, f);
+                if (!gok || __any(far > PAIR_R2_HI_HI - PAIR_R2_LO_HI)) {
+#pragma unroll
+                    for (int u = 0; u < G; u++) f[u] = m[u] / (r2[u] * sqrt(r2[u]));
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < G; u++) {
+                px = fma(-f[u], rx[u], px);
+                py = fma(-f[u], ry[u], py);
+                pz = fma(-f[u], rz[u], pz);
             }
         }
-        __syncthreads();
+        for (; q < jn; q++) {
+            const double g = sb[q][3], rx = xt - sb[q][0], ry = yt - sb[q][1], rz = zt - sb[q][2];
+            const double r2 = dot3(rx, ry, rz, rx, ry, rz);
+            const double f = FAST ? gm_over_r3_fast(g, r2) : gm_over_r3(g, r2, gok);
+            px = fma(-f, rx, px);
+            py = fma(-f, ry, py);
+            pz = fma(-f, rz, pz);
+        }
     }
     if (!valid) return;
-    acc[3 * t] = acc[3 * t] + px;
-    acc[3 * t + 1] = acc[3 * t + 1] + py;
-    acc[3 * t + 2] = acc[3 * t + 2] + pz;
+    double *a = acc + 3 * (int64_t)t;
+    a[0] = a[0] + px;
+    a[1] = a[1] + py;
+    a[2] = a[2] + pz;
 }
+
+// The same for few particles, 16 of them per workgroup with one massive body
+// per lane (swg_rows.h).
+template <bool FAST>
+__global__ __launch_bounds__((RowsLds<RW_SMALL, 4>::THREADS), (RowsLds<RW_SMALL, 4>::WAVES)) void k_leaf_tp_rows(
+    int ntp, int npl, const double *rtp, const double *rpl, const double *Gm, const int32_t *lmask, double *acc)
+{
+    constexpr int B = RW_SMALL;
+    __shared__ RowsLds<B, 4> S;
+    const int b0 = (int)blockIdx.x * B, b1 = min(b0 + B, ntp);
+    const RowsSrc pl{rpl, rpl + 1, rpl + 2, Gm, Gm, 3}, tp{rtp, rtp + 1, rtp + 2, rtp, rtp, 3};
+    rows_sums<true, true, false>(S, pl, tp, [](int, int) { return 0.0; }, b0, b1, npl, npl, false, FAST, false);
+    const int bl = (int)threadIdx.x % B, t = b0 + bl, comp = (int)threadIdx.x / B;
+    if (comp >= 3 || t >= b1 || !lmask[t]) return;
+    double *o = acc + 3 * (int64_t)t + comp;
+    *o = *o + S.out[0][comp][bl];
+}
+
+// The rows where the particles alone leave SIMDs idle and the massive bodies fill
+// at least half of a 64-partner chunk.  Measured, lanes / rows in us: 500 bodies
+// with 1000 particles 51 / 10, 32000 55 / 42, 65536 61 / 82, 100003 90 / 121;
+// 64 bodies with 16000 particles 8.5 / 6.1; 8 bodies with 16000 2.9 / 5.3.
+constexpr int LEAF_TP_ROWS = 40960, LEAF_TP_ROWS_NPL = 32;
 
 // swiftest_drift_all (swiftest_drift.f90:60-108), GR off
 __global__ __launch_bounds__(256) void k_leaf_drift(const double *mu, double *x, double *v, int n, double dt, const int32_t *lmask,
@@ -1222,8 +1278,14 @@ int swg_kick_getacch_int_all_tri_pl(swg_ctx *ctx, int32_t npl, int32_t nplm, con
     const XferItem in[] = {xfer_words(r, dr, 3 * (int64_t)npl), xfer_words(Gmass, dg, npl),
                            xfer_words(acc, da, 3 * (int64_t)npl), xfer_words(radius, dR, radius ? npl : 0)};
     HIPCHK(ctx->leaf->stage.in(st, in, 4));
-    if (npl / RW_LARGE < RW_LARGE_TILES) launch_leaf_tri<RW_SMALL, 4>(st, npl, nplm, dr, dg, dR, da, ctx->pair_mode);
-    else launch_leaf_tri<RW_LARGE, 8>(st, npl, nplm, dr, dg, dR, da, ctx->pair_mode);
+    // the triangular sums take 16-body tiles at any size: two copies of the fold
+    // leave 64-body ones no registers (13000 bodies, 5000 of them fully
+    // interacting: 0.63 ms, 3.6 ms with 64)
+    const bool fast = ctx->pair_mode != 0;
+    if (npl - nplm > nplm) launch_leaf_tri<RW_SMALL, 4, 2, true>(st, npl, nplm, dr, dg, dR, da, fast);
+    else if (cdiv(npl, RW_SMALL) <= RW_FEW) launch_leaf_tri<RW_SMALL, 4, 2, false>(st, npl, nplm, dr, dg, dR, da, fast);
+    else if (npl / RW_LARGE < RW_LARGE_TILES) launch_leaf_tri<RW_SMALL, 4, 1, false>(st, npl, nplm, dr, dg, dR, da, fast);
+    else launch_leaf_tri<RW_LARGE, 8, 1, false>(st, npl, nplm, dr, dg, dR, da, fast);
     HIPCHK(hipGetLastError());
     const XferItem out = xfer_words(acc, da, 3 * (int64_t)npl);
     HIPCHK(ctx->leaf->stage.out(st, &out, 1));
@@ -1302,7 +1364,14 @@ int swg_kick_getacch_int_all_tp(swg_ctx *ctx, int32_t ntp, int32_t npl, const do
     const XferItem in[] = {xfer_words(rtp, dt_, 3 * (int64_t)ntp), xfer_words(rpl, dp, 3 * (int64_t)npl),
                            xfer_words(GMpl, dg, npl), xfer_i32(lmask, dm, ntp), xfer_words(acc, da, 3 * (int64_t)ntp)};
     HIPCHK(ctx->leaf->stage.in(st, in, 5));
-    k_leaf_tp<256><<<cdiv(ntp, 256), 256, 0, st>>>(ntp, npl, dt_, dp, dg, dm, da, ctx->pair_mode);
+    const bool fast = ctx->pair_mode != 0;
+    if (npl >= LEAF_TP_ROWS_NPL && ntp <= LEAF_TP_ROWS) {
+        const auto kern = fast ? k_leaf_tp_rows<true> : k_leaf_tp_rows<false>;
+        kern<<<cdiv(ntp, RW_SMALL), RowsLds<RW_SMALL, 4>::THREADS, 0, st>>>(ntp, npl, dt_, dp, dg, dm, da);
+    } else {
+        const auto kern = fast ? k_leaf_tp<true> : k_leaf_tp<false>;
+        kern<<<cdiv(ntp, 64), 64, 0, st>>>(ntp, npl, dt_, dp, dg, dm, da);
+    }
     HIPCHK(hipGetLastError());
     const XferItem out = xfer_words(acc, da, 3 * (int64_t)ntp);
     HIPCHK(ctx->leaf->stage.out(st, &out, 1));

@@ -404,17 +404,18 @@ __global__ __launch_bounds__(BLK) void k_kick_pl(PlDev pl, SysDev sy, ListDev pp
 // fast: the factors from gm_over_r3_fast.
 // ---------------------------------------------------------------------------
 
+
 typedef const __attribute__((address_space(4))) double cdouble;
 __device__ inline const cdouble *cview(const double *p) { return (const cdouble *)p; }
 
-template <int B, int KE, bool TINY, bool fast>
-__global__ __launch_bounds__((RowsLds<B, KE>::THREADS), (RowsLds<B, KE>::WAVES)) void k_kick_pl_rows(PlDev pl, SysDev sy, ListDev pp,
+template <int B, int KE, int A, bool TINY, bool fast>
+__global__ __launch_bounds__((RowsLds<B, KE, A>::THREADS), (RowsLds<B, KE, A>::WAVES)) void k_kick_pl_rows(PlDev pl, SysDev sy, ListDev pp,
                                                                           const Tile *tiles, double dt, int lbeg,
                                                                           int use_radius, int do_pairs)
 {
     constexpr int WK = B / 16;  // wavefronts walking each side of the encounter pairs, 16 bodies each
     static_assert(KE >= 2 * WK, "the evaluation wavefronts walk the encounter pairs");
-    __shared__ RowsLds<B, KE> S;
+    __shared__ RowsLds<B, KE, A> S;
     __shared__ double hpart[2][3][B];
     const Tile tl = tiles[blockIdx.x];
     const int p0 = sy.pl_off[tl.s], n = sy.pl_off[tl.s + 1] - p0;
@@ -423,8 +424,8 @@ __global__ __launch_bounds__((RowsLds<B, KE>::THREADS), (RowsLds<B, KE>::WAVES))
     const int lane = (int)(threadIdx.x & 63u), w = (int)(threadIdx.x >> 6);
     const RowsSrc src{pl.rh.x + p0, pl.rh.y + p0, pl.rh.z + p0, pl.Gm + p0, pl.R + p0, 1};
     const auto zero = [](int, int) { return 0.0; };
-    if (tri) rows_sums<!TINY, !TINY>(S, src, zero, tl.b0 - p0, tl.b1 - p0, nm, n, true, fast ? 2 : 0, use_radius != 0);
-    else rows_sums<!TINY, !TINY>(S, src, zero, tl.b0 - p0, tl.b1 - p0, nm, n, false, fast ? 2 : 0, use_radius != 0);
+    if (tri) rows_sums<!TINY, !TINY, true>(S, src, src, zero, tl.b0 - p0, tl.b1 - p0, nm, n, true, fast ? 2 : 0, use_radius != 0);
+    else rows_sums<!TINY, !TINY, true>(S, src, src, zero, tl.b0 - p0, tl.b1 - p0, nm, n, false, fast ? 2 : 0, use_radius != 0);
     if (do_pairs && w < 2 * WK) {
         // the first WK wavefronts: ahj over pairs (p, i), p < i; the next: ahi
         // over pairs (i, j)
@@ -1037,7 +1038,7 @@ void launch_kick_pl(hipStream_t st, const Tuning &tu, PlDev pl, SysDev sy, ListD
 {
     if (!ntiles) return;
     if (tu.any_tiny) {
-        const auto kern = tu.pair_fast ? k_kick_pl_rows<RW_SMALL, 4, true, true> : k_kick_pl_rows<RW_SMALL, 4, true, false>;
+        const auto kern = tu.pair_fast ? k_kick_pl_rows<RW_SMALL, 4, 2, true, true> : k_kick_pl_rows<RW_SMALL, 4, 2, true, false>;
         kern<<<ntiles, RowsLds<RW_SMALL, 4>::THREADS, 0, st>>>(pl, sy, pp, tiles, dt, lbeg, use_radius, do_pairs);
         return;
     }
@@ -1053,10 +1054,13 @@ void launch_kick_pl(hipStream_t st, const Tuning &tu, PlDev pl, SysDev sy, ListD
     }
     if (tu.kick_pl_eval) {
         if (tu.kick_pl_eval == 8)
-            k_kick_pl_rows<RW_LARGE, 8, false, false><<<ntiles, RowsLds<RW_LARGE, 8>::THREADS, 0, st>>>(
+            k_kick_pl_rows<RW_LARGE, 8, 1, false, false><<<ntiles, RowsLds<RW_LARGE, 8>::THREADS, 0, st>>>(
+                pl, sy, pp, tiles, dt, lbeg, use_radius, do_pairs);
+        else if (ntiles <= RW_FEW)
+            k_kick_pl_rows<RW_SMALL, 4, 2, false, false><<<ntiles, RowsLds<RW_SMALL, 4>::THREADS, 0, st>>>(
                 pl, sy, pp, tiles, dt, lbeg, use_radius, do_pairs);
         else
-            k_kick_pl_rows<RW_SMALL, 4, false, false><<<ntiles, RowsLds<RW_SMALL, 4>::THREADS, 0, st>>>(
+            k_kick_pl_rows<RW_SMALL, 4, 1, false, false><<<ntiles, RowsLds<RW_SMALL, 4>::THREADS, 0, st>>>(
                 pl, sy, pp, tiles, dt, lbeg, use_radius, do_pairs);
         return;
     }

@@ -44,9 +44,14 @@ constexpr int KPL_FAST_TILE = 64;
 // the two tile sizes of k_kick_pl_rows and of the leaf rows
 constexpr int RW_SMALL = 16, RW_LARGE = 64;
 // 64-body tiles once they fill three quarters of the compute units (measured,
-// 16 / 64 bodies a tile: 2000 bodies 37 / 70 us, 10000 bodies 300 / 320 us,
-// 32000 bodies 2.7 / 2.0 ms)
+// 16 / 64 bodies a tile: 10000 bodies 267 / 320 us, 13000 bodies 450 / 405 us,
+// 32000 bodies 2.7 / 2.0 ms).
 constexpr int RW_LARGE_TILES = 192;
+// Up to one 16-body tile per compute unit the fold takes the registers to read
+// two sets of terms ahead (2000 bodies 32.6 us, 36.2 one set ahead); from two
+// tiles on the other wavefronts fill the waits, and the registers cost the third
+// tile its place (6000 bodies 122 / 119 us, 10000 bodies 320 / 267 us).
+constexpr int RW_FEW = 256;
 
 inline int Tuning::pl_tile() const
 {

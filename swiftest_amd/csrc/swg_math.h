@@ -87,13 +87,83 @@ __device__ inline double div_core(double a, double b)
 constexpr double PAIR_R2_LO = 0x1p-400, PAIR_R2_HI = 0x1p400;
 constexpr int PAIR_R2_LO_HI = (1023 - 400) << 20, PAIR_R2_HI_HI = (1023 + 400) << 20;  // their high words
 constexpr double PAIR_G_LO = 0x1p-500, PAIR_G_HI = 0x1p500;
+constexpr int PAIR_G_LO_HI = (1023 - 500) << 20, PAIR_G_HI_HI = (1023 + 500) << 20;
 
 __host__ __device__ inline bool pair_g_ok(double g) { return g == 0.0 || (g >= PAIR_G_LO && g <= PAIR_G_HI); }
+
+// the same without branches, by integers (2^500 itself is left to the IEEE
+// operations)
+__device__ inline bool pair_g_ok_int(double g)
+{
+    const int h = __double2hiint(g);
+    return ((uint32_t)(h - PAIR_G_LO_HI) < (uint32_t)(PAIR_G_HI_HI - PAIR_G_LO_HI)) | ((h | __double2loint(g)) == 0);
+}
 
 __device__ inline double gm_over_r3(double g, double r2, bool gok)
 {
     if (gok && r2 >= PAIR_R2_LO && r2 <= PAIR_R2_HI) return div_core(g, r2 * sqrt_core(r2));
     return g / (r2 * sqrt(r2));
+}
+
+// Holds two or four values in registers at this point of the program: the
+// empty asm statement (no instruction) keeps the compiler from moving their
+// computation past it, so that their chains advance side by side.
+template <int G>
+__device__ inline void side_by_side(double (&a)[G])
+{
+    static_assert(G == 2 || G == 4, "two or four");
+    if constexpr (G == 2) asm volatile("" : "+v"(a[0]), "+v"(a[1]));
+    else asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
+}
+
+// f = div_core(g, r2 * sqrt_core(r2)) of G pairs, step by step.  Each chain is
+// 20 operations deep and the compiler, left to itself, takes one after another,
+// which a wavefront alone on its SIMD spends waiting (64 particles' 500 terms
+// 66 -> 50 us; the rows of 10007 bodies, several wavefronts to a SIMD, 315 -> 298).
+template <int G>
+__device__ inline void pair_factors(const double (&gm)[G], const double (&r2)[G], double (&f)[G])
+{
+    double y[G], g[G], h[G], d[G], b[G];
+#define EACH(stmt)                        \
+    _Pragma("unroll") for (int u = 0; u < G; u++) stmt;
+    EACH(y[u] = __builtin_amdgcn_rsq(r2[u]))
+    side_by_side(y);
+    EACH(g[u] = r2[u] * y[u])
+    EACH(h[u] = y[u] * 0.5)
+    side_by_side(g);
+    side_by_side(h);
+    EACH(d[u] = fma(-h[u], g[u], 0.5))
+    side_by_side(d);
+    EACH(g[u] = fma(g[u], d[u], g[u]))
+    EACH(h[u] = fma(h[u], d[u], h[u]))
+    side_by_side(g);
+    side_by_side(h);
+    EACH(d[u] = fma(-g[u], g[u], r2[u]))
+    side_by_side(d);
+    EACH(g[u] = fma(d[u], h[u], g[u]))
+    side_by_side(g);
+    EACH(d[u] = fma(-g[u], g[u], r2[u]))
+    side_by_side(d);
+    EACH(g[u] = fma(d[u], h[u], g[u]))
+    side_by_side(g);
+    EACH(b[u] = r2[u] * g[u])
+    side_by_side(b);
+    EACH(y[u] = __builtin_amdgcn_rcp(b[u]))
+    side_by_side(y);
+    EACH(d[u] = fma(-b[u], y[u], 1.0))
+    side_by_side(d);
+    EACH(y[u] = fma(y[u], d[u], y[u]))
+    side_by_side(y);
+    EACH(d[u] = fma(-b[u], y[u], 1.0))
+    side_by_side(d);
+    EACH(y[u] = fma(y[u], d[u], y[u]))
+    side_by_side(y);
+    EACH(g[u] = gm[u] * y[u])
+    side_by_side(g);
+    EACH(d[u] = fma(-b[u], g[u], gm[u]))
+    side_by_side(d);
+    EACH(f[u] = fma(d[u], y[u], g[u]))
+#undef EACH
 }
 
 // g * r2^-1.5 for the fast pair mode (SWG_PAIR_FAST), not bit-identical to

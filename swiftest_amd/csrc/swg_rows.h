@@ -20,9 +20,9 @@
 // of B = 64 (a fold wavefront per component, every lane of it in use): the
 // first is bound by the fold's chain of about 10 cycles a term, the second,
 // for systems that fill the chip either way, by FP64 issue.
-// Measured: 2000 bodies 38 us (64-body tiles with the partners staged in LDS
-// and read there for every term: 69), 10000 bodies 300 us (338), 32000 bodies
-// 2.03 ms (2.03); the leaf rows of 10007 bodies 315 us (one lane a body: 4466);
+// Measured: 2000 bodies 32.6 us (64-body tiles with the partners staged in LDS
+// and read there for every term: 69), 10000 bodies 267 us (338), 32000 bodies
+// 2.0 ms (2.0); the leaf rows of 10007 bodies 267 us (one lane a body: 4466);
 // half of 2000 bodies semi-interacting 60 us (one lane a body: 930).
 #pragma once
 #include "swg_math.h"
@@ -32,12 +32,14 @@ namespace swg {
 constexpr int RW_C = 64;       // partners per chunk, one per lane
 constexpr int RW_S = RW_C + 2; // row stride of the factors: 16-byte aligned, rows 4 banks apart
 
-template <int B, int KE>
+// B bodies, KE evaluation wavefronts; A: sets of eight terms the fold reads ahead
+template <int B, int KE, int A = 1>
 struct RowsLds {
     static constexpr int NF = (3 * B + 63) / 64;  // fold wavefronts
     static constexpr int THREADS = 64 * (KE + NF);
-    // wavefronts per SIMD the registers leave room for: two workgroups of 64 bodies
-    static constexpr int WAVES = B == 64 ? 6 : 2;
+    // wavefronts per SIMD the registers leave room for: two workgroups of 64
+    // bodies, four of 16; one of 16 that reads two sets of terms ahead
+    static constexpr int WAVES = B == 64 ? 6 : A == 2 ? 2 : 5;
     __align__(16) double fac[2][B][RW_S];
     __align__(16) double pj[2][3][RW_C];  // the partners' positions
     uint64_t take[2][B];                  // bit q: the body takes its term with partner q ...
@@ -45,15 +47,15 @@ struct RowsLds {
     double out[2][3][B];
 };
 
-// Where rows_sums reads component a (x, y, z, Gm, R) of body j; a missing
-// array (no radii) reads as zero.
+// Where rows_sums reads component a (x, y, z, Gm, R) of body j.  Every array is
+// there, R too where radii are not tested (any array of the length).
 struct RowsSrc {
     const double *x, *y, *z, *g, *R;
     int stride;  // of x, y and z
     __device__ double operator()(int a, int j) const
     {
         const double *p = a == 0 ? x : a == 1 ? y : a == 2 ? z : a == 3 ? g : R;
-        return p ? p[(int64_t)j * (a < 3 ? stride : 1)] : 0.0;
+        return p[(int64_t)j * (a < 3 ? stride : 1)];
     }
 };
 
@@ -79,17 +81,19 @@ __device__ inline double rows_uniform(double v)
 // factor, fma(0, d, s) = s bit for bit (d finite; a sum that starts at +0 is
 // never -0); otherwise the sum is kept by selection, also for a first value
 // of -0 and for partners at infinity.
-template <bool FULL, bool ZERO, int B, int KE, class Init>
-__device__ __attribute__((always_inline)) inline void rows_sums(RowsLds<B, KE> &S, const RowsSrc &load, Init init,
-                                                                int b0, int b1, int nplm, int npl, bool tri, int fast,
-                                                                bool use_radius)
+// SELF: the bodies are the partners themselves and leave themselves out;
+// otherwise tgt holds others (test particles; nplm = npl, rows).
+template <bool FULL, bool ZERO, bool SELF, int B, int KE, int A, class Init>
+__device__ __attribute__((always_inline)) inline void rows_sums(RowsLds<B, KE, A> &S, const RowsSrc &load, const RowsSrc &tgt,
+                                                                Init init, int b0, int b1, int nplm, int npl, bool tri,
+                                                                int fast, bool use_radius)
 {
     constexpr int NB = B / KE, G = NB < 4 ? NB : 4;
     static_assert(NB * KE == B && NB % G == 0, "whole groups of bodies per wavefront");
     static_assert(B == 16 || B == 64, "a chunk holds all of a tile's bodies or none");
     const int lane = (int)(threadIdx.x & 63u), w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     // partners any body of the tile needs
-    const int jend = b0 < nplm ? npl : nplm, nch = (jend + RW_C - 1) / RW_C;
+    const int jend = !SELF || b0 < nplm ? npl : nplm, nch = (jend + RW_C - 1) / RW_C;
     if (w < KE) {
         // ---- evaluation: this lane's partner against bodies e0 .. e0 + NB - 1
         const int e0 = w * NB;
@@ -98,11 +102,11 @@ __device__ __attribute__((always_inline)) inline void rows_sums(RowsLds<B, KE> &
 #pragma unroll
         for (int k = 0; k < NB; k++) {
             const int i = min(b0 + e0 + k, b1 - 1);
-            xb[k] = rows_uniform<(NB > 4)>(load(0, i));
-            yb[k] = rows_uniform<(NB > 4)>(load(1, i));
-            zb[k] = rows_uniform<(NB > 4)>(load(2, i));
-            Rb[k] = rows_uniform<(NB > 4)>(load(4, i));
-            if (i >= nplm) jmin = min(npl, nplm);
+            xb[k] = rows_uniform<(NB > 4)>(tgt(0, i));
+            yb[k] = rows_uniform<(NB > 4)>(tgt(1, i));
+            zb[k] = rows_uniform<(NB > 4)>(tgt(2, i));
+            Rb[k] = rows_uniform<(NB > 4)>(tgt(4, i));
+            if (SELF && i >= nplm) jmin = min(npl, nplm);
         }
         double n[5], p[5];
         auto fetch = [&](int c) __attribute__((always_inline)) {
@@ -117,11 +121,11 @@ __device__ __attribute__((always_inline)) inline void rows_sums(RowsLds<B, KE> &
             if (c < nch && !idle) {
 #pragma unroll
                 for (int a = 0; a < 5; a++) p[a] = n[a];
-                if (c + 1 < nch) fetch(c + 1);
+                fetch(c + 1);
                 const int jt = c * RW_C, j = jt + lane;
                 // neither the end of any body's partners nor the tile itself
-                const bool plain = jt + RW_C <= jmin && (jt + RW_C <= b0 || jt >= b0 + B);
-                const bool gok = tri || __all(pair_g_ok(p[3]));
+                const bool plain = jt + RW_C <= jmin && (!SELF || jt + RW_C <= b0 || jt >= b0 + B);
+                const bool gok = tri || __all(pair_g_ok_int(p[3]));
                 double(*f)[RW_S] = S.fac[c & 1];
                 if (w == 0) {
                     S.pj[c & 1][0][lane] = p[0];
@@ -131,29 +135,51 @@ __device__ __attribute__((always_inline)) inline void rows_sums(RowsLds<B, KE> &
                 uint64_t m[NB], full = ~0ull;
 #pragma unroll
                 for (int k0 = 0; k0 < NB; k0 += G) {
-                    double r2[G], fc[G];
-                    uint32_t far = 0;
+                    // step by step for all of the group's bodies, so that their
+                    // chains of operations run side by side
+                    double r2[G], gm[G], fc[G];
 #pragma unroll
                     for (int u = 0; u < G; u++) {
-                        const int k = k0 + u;
-                        const double rx = p[0] - xb[k], ry = p[1] - yb[k], rz = p[2] - zb[k];
+                        const double rx = p[0] - xb[k0 + u], ry = p[1] - yb[k0 + u], rz = p[2] - zb[k0 + u];
                         r2[u] = dot3(rx, ry, rz, rx, ry, rz);
-                        const double rs = Rb[k] + p[4];
-                        m[k] = use_radius ? __ballot(r2[u] > rs * rs) : ~0ull;
-                        if (!plain) {
-                            const int i = b0 + e0 + k;
-                            m[k] &= __ballot((j < (i < nplm ? npl : nplm)) & (j != i));
+                    }
+#pragma unroll
+                    for (int u = 0; u < G; u++) m[k0 + u] = ~0ull;
+                    if (use_radius) {
+#pragma unroll
+                        for (int u = 0; u < G; u++) {
+                            const double rs = Rb[k0 + u] + p[4];
+                            m[k0 + u] = __ballot(r2[u] > rs * rs);
                         }
-                        full &= m[k];
-                        if (fast) {
-                            const bool one = fast == 2 && tri;
+                    }
+                    if (!plain) {
+#pragma unroll
+                        for (int u = 0; u < G; u++) {
+                            const int i = b0 + e0 + k0 + u;
+                            m[k0 + u] &= __ballot((j < (!SELF || i < nplm ? npl : nplm)) & (!SELF | (j != i)));
+                        }
+                    }
+#pragma unroll
+                    for (int u = 0; u < G; u++) full &= m[k0 + u];
+                    uint32_t far = 0;
+                    if (fast) {
+                        const bool one = fast == 2 && tri;
+#pragma unroll
+                        for (int u = 0; u < G; u++) {
                             const double g = gm_over_r3_fast(one ? 1.0 : p[3], r2[u]);
                             fc[u] = one ? p[3] * g : g;
-                        } else {
-                            const double g = div_core(tri ? 1.0 : p[3], r2[u] * sqrt_core(r2[u]));
-                            fc[u] = tri ? p[3] * g : g;
+                        }
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < G; u++) {
+                            gm[u] = tri ? 1.0 : p[3];
                             // by the high word: the exponent alone decides
                             far = max(far, (uint32_t)(__double2hiint(r2[u]) - PAIR_R2_LO_HI));
+                        }
+                        pair_factors<G>(gm, r2, fc);
+                        if (tri) {
+#pragma unroll
+                            for (int u = 0; u < G; u++) fc[u] = p[3] * fc[u];
                         }
                     }
                     // the IEEE operations where the cores' range does not hold
@@ -182,29 +208,32 @@ __device__ __attribute__((always_inline)) inline void rows_sums(RowsLds<B, KE> &
         // ---- fold: the fold wavefronts' lanes are component by body
         // (lanes past the last repeat it)
         const int l = min((w - KE) * 64 + lane, 3 * B - 1), comp = l / B, bl = l % B, i = min(b0 + bl, b1 - 1);
-        const double cb = load(comp, i);
+        const double cb = tgt(comp, i);
         double acc = tri ? 0.0 : init(comp, i), hi = 0.0;
-        // one side's sums over a chunk whose terms are all taken, the reads of
-        // the next eight factors and coordinates issued before the current
-        // eight are folded
+        // one side's sums over a chunk whose terms are all taken.  The reads of
+        // factors and coordinates run AHEAD sets of eight terms before the fold:
+        // two sets where the registers are there (a set's adds take less time
+        // than a read comes back)
         auto fold64 = [&](double v, const double *f, const double *dc) __attribute__((always_inline)) {
+            constexpr int SETS = RW_C / 8, AHEAD = FULL ? A : 1, NB2 = AHEAD + 1;
             const double2 *f2 = (const double2 *)f, *d2 = (const double2 *)dc;
-            double2 fa[4], da[4];
+            double2 fa[NB2][4], da[NB2][4];
+            auto read = [&](int q) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < 4; u++) fa[u] = f2[u], da[u] = d2[u];
-#pragma unroll (FULL ? RW_C / 8 : 2)
-            for (int q = 4; q <= RW_C / 2; q += 4) {
-                double2 fn[4], dn[4];
-                const int qn = min(q, RW_C / 2 - 4);
+                for (int u = 0; u < 4; u++) fa[q % NB2][u] = f2[4 * q + u], da[q % NB2][u] = d2[4 * q + u];
+            };
 #pragma unroll
-                for (int u = 0; u < 4; u++) fn[u] = f2[qn + u], dn[u] = d2[qn + u];
+            for (int q = 0; q < AHEAD; q++) read(q);
+#pragma unroll (FULL ? SETS : 2)
+            for (int q = 0; q < SETS; q++) {
+                if (q + AHEAD < SETS) read(q + AHEAD);
+                // an empty statement that no read passes
+                if (AHEAD > 1) asm volatile("" ::: "memory");
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-                    v = fma(fa[u].x, da[u].x - cb, v);
-                    v = fma(fa[u].y, da[u].y - cb, v);
+                    v = fma(fa[q % NB2][u].x, da[q % NB2][u].x - cb, v);
+                    v = fma(fa[q % NB2][u].y, da[q % NB2][u].y - cb, v);
                 }
-#pragma unroll
-                for (int u = 0; u < 4; u++) fa[u] = fn[u], da[u] = dn[u];
             }
             return v;
         };

@@ -77,3 +77,42 @@ def test_rows_with_encounter_pairs(n, q, pm):
             else:
                 assert np.array_equal(a[key], b[key]), (k, key)
     assert g.stats()["nplpl_enc"] > 0
+
+
+@pytest.mark.parametrize("npl,ntp", [(1, 1), (3, 65), (4, 63), (31, 16), (32, 1), (32, 16), (33, 17), (63, 15), (64, 64),
+                                     (65, 100), (129, 33), (500, 1000), (67, 40960), (67, 40961)])
+def test_particles_at_tile_edges(npl, ntp):
+    """Particle sums by rows and by lanes (few massive bodies, many particles),
+    with masked particles, massless bodies and some separations and masses
+    outside the exact cores' range."""
+    print(f"particles npl={npl} ntp={ntp}", flush=True)
+    rng, r, Gm, _ = _bodies(npl, npl + ntp)
+    rt = rng.normal(0, 2.0, (ntp, 3))
+    mask = (rng.random(ntp) > 0.1).astype(np.int32)
+    acc = rng.normal(0, 1e-3, (ntp, 3))
+    acc[0] = -0.0
+    ref = O.accel_pltp(rt, r, Gm, mask, acc)
+    got = S.swiftest_kick_getacch_int_all_tp(ntp, npl, rt, r, Gm, mask, acc)
+    assert np.array_equal(ref.view(np.int64), got.view(np.int64))
+    Gm[npl // 2] = 0.0
+    Gm[-1] = 1e-200
+    rt[ntp // 2] *= 1e130
+    rt[-1] = r[0] + 1e-130
+    ref = O.accel_pltp(rt, r, Gm, mask, acc)
+    got = S.swiftest_kick_getacch_int_all_tp(ntp, npl, rt, r, Gm, mask, acc)
+    assert np.array_equal(ref, got, equal_nan=True)
+    if ntp > 1000:
+        return
+    S.set_pair_mode(S.PAIR_FAST)
+    try:
+        fast = S.swiftest_kick_getacch_int_all_tp(ntp, npl, rt, r, Gm, mask, np.zeros((ntp, 3)))
+    finally:
+        S.set_pair_mode(S.PAIR_EXACT)
+    ref = O.accel_pltp(rt, r, Gm, mask, np.zeros((ntp, 3)))
+    keep = np.arange(ntp)
+    keep = keep[(keep != ntp // 2) & (keep != ntp - 1)]  # the others' factors leave the normal range
+    d = rt[keep, None, :] - r[None, :, :]
+    terms = (Gm[None, :, None] * np.abs(d) / ((d * d).sum(-1) ** 1.5)[..., None]).sum(1)
+    # each factor within 8 ulp of the exact mode's, then npl roundings of partial
+    # sums no larger than the sum of the terms' sizes, on both sides
+    assert (np.abs(fast - ref)[keep] <= 2 * (npl + 8) * 2.0**-52 * terms).all()
