@@ -31,28 +31,6 @@ static inline int cdiv(int64_t a, int b) { return (int)((a + b - 1) / b); }
 // leaf kernels (AoS in HBM, as the reference lays its (3,n) arrays out)
 // ---------------------------------------------------------------------------
 
-// int_one_pl contribution of pair (i, j) to body b's ahi (b == i) or ahj (b == j)
-__device__ inline void one_pl_half(double rji2, double xr, double yr, double zr, double Gm_other, bool b_is_i,
-                                   double &ax, double &ay, double &az, int fast)
-{
-    double fac;
-    if (fast) {
-        fac = gm_over_r3_fast(Gm_other, rji2);
-    } else {
-        double irij3 = 1.0 / (rji2 * sqrt(rji2));
-        fac = Gm_other * irij3;
-    }
-    if (b_is_i) {
-        ax = fma(fac, xr, ax);
-        ay = fma(fac, yr, ay);
-        az = fma(fac, zr, az);
-    } else {
-        ax = fma(-fac, xr, ax);
-        ay = fma(-fac, yr, ay);
-        az = fma(-fac, zr, az);
-    }
-}
-
 // swiftest_kick_getacch_int_all_tri_{rad,norad}_pl (swiftest_kick.f90:165-371):
 // the rows of B bodies per workgroup, the terms evaluated by several
 // wavefronts and folded in partner order by others (swg_rows.h).
@@ -80,41 +58,106 @@ static void launch_leaf_tri(hipStream_t st, int npl, int nplm, const double *r, 
     kern<<<cdiv(npl, B), RowsLds<B, KE>::THREADS, 0, st>>>(npl, nplm, r, Gm, R, acc);
 }
 
-// swiftest_kick_getacch_int_all_flat_{rad,norad}_pl (swiftest_kick.f90:69-162)
-// gathered per body: rows = pair ids with index1 == b, cols = index2 == b,
-// each in list order (built on the host).
-__global__ void k_leaf_flat(int npl, const int32_t *k, const double *r, const double *Gm, const double *R,
-                            const int64_t *rs, const int64_t *cs, const int64_t *rowl, const int64_t *coll,
-                            double *acc, int fast)
+// swiftest_kick_getacch_int_all_flat_{rad,norad}_pl (swiftest_kick.f90:69-162):
+// pair p adds a term to body index1's ahi and one to index2's ahj, each in list
+// order.  One thread per pair forms both terms, entry p and entry n + p, as a
+// factor and the separation (zeros where the radii leave the pair out: the sums
+// start at +0 and are never -0, so fma(0, 0, s) = s); a stable sort of the
+// entries by body and side gives each sum's terms in list order, whatever the
+// list's; 16 lanes per sum gather them and fold them in that order.  Bound: about
+// fifteen short launches and the transfer of the list.  Measured, 200003 pairs
+// among 5000 bodies: the call 780 us with the lists built by the host and one
+// thread a body, XX us now.
+constexpr int64_t FLAT_PAIRS = 1 << 20;  // pairs of one round: bounds the scratch at about 112 MB
+
+__global__ __launch_bounds__(256) void k_flat_terms(int n, const int2 *k, int npl, const double *r, const double *Gm,
+                                                    const double *R, int fast, uint32_t *key, uint32_t *val, double4 *term,
+                                                    int32_t *seg, int32_t *bad)
 {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= npl) return;
-    double hix = 0, hiy = 0, hiz = 0, hjx = 0, hjy = 0, hjz = 0;
-    for (int64_t q = rs[b]; q < rs[b + 1]; q++) {
-        int64_t p = rowl[q];
-        int i = k[2 * p] - 1, j = k[2 * p + 1] - 1;
-        double xr = r[3 * j] - r[3 * i], yr = r[3 * j + 1] - r[3 * i + 1], zr = r[3 * j + 2] - r[3 * i + 2];
-        double rji2 = dot3(xr, yr, zr, xr, yr, zr);
-        if (R) {
-            double s = R[i] + R[j];
-            if (!(rji2 > s * s)) continue;
-        }
-        one_pl_half(rji2, xr, yr, zr, Gm[j], true, hix, hiy, hiz, fast);
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t < npl) {
+        seg[t] = seg[npl + t] = 0;  // first and past-last entry of the two sums
+        seg[2 * npl + t] = seg[3 * npl + t] = 0;
     }
-    for (int64_t q = cs[b]; q < cs[b + 1]; q++) {
-        int64_t p = coll[q];
-        int i = k[2 * p] - 1, j = k[2 * p + 1] - 1;
-        double xr = r[3 * j] - r[3 * i], yr = r[3 * j + 1] - r[3 * i + 1], zr = r[3 * j + 2] - r[3 * i + 2];
-        double rji2 = dot3(xr, yr, zr, xr, yr, zr);
-        if (R) {
-            double s = R[i] + R[j];
-            if (!(rji2 > s * s)) continue;
+    if (t >= n) return;
+    int i = k[t].x - 1, j = k[t].y - 1;
+    double4 a = make_double4(0.0, 0.0, 0.0, 0.0), b = a;
+    if (i < 0 || i >= npl || j < 0 || j >= npl) {
+        *bad = 1;
+        i = j = 0;
+    } else {
+        const double xi = r[3 * (int64_t)i], yi = r[3 * (int64_t)i + 1], zi = r[3 * (int64_t)i + 2];
+        const double xr = r[3 * (int64_t)j] - xi, yr = r[3 * (int64_t)j + 1] - yi, zr = r[3 * (int64_t)j + 2] - zi;
+        const double r2 = dot3(xr, yr, zr, xr, yr, zr);
+        const double rs = R ? R[i] + R[j] : 0.0;
+        if (!R || r2 > rs * rs) {
+            double fi, fj;
+            if (fast) {
+                fi = gm_over_r3_fast(Gm[j], r2);
+                fj = gm_over_r3_fast(Gm[i], r2);
+            } else {
+                const double irij3 = 1.0 / (r2 * sqrt(r2));
+                fi = Gm[j] * irij3;
+                fj = Gm[i] * irij3;
+            }
+            a = make_double4(xr, yr, zr, fi);
+            b = make_double4(xr, yr, zr, -fj);
         }
-        one_pl_half(rji2, xr, yr, zr, Gm[i], false, hjx, hjy, hjz, fast);
     }
-    acc[3 * b] = (acc[3 * b] + hix) + hjx;
-    acc[3 * b + 1] = (acc[3 * b + 1] + hiy) + hjy;
-    acc[3 * b + 2] = (acc[3 * b + 2] + hiz) + hjz;
+    key[t] = (uint32_t)i;
+    key[n + t] = (uint32_t)npl + (uint32_t)j;
+    val[t] = (uint32_t)t;
+    val[n + t] = (uint32_t)(n + t);
+    term[t] = a;
+    term[n + t] = b;
+}
+
+// where each sum's entries begin and end among the m sorted ones
+__global__ __launch_bounds__(256) void k_flat_bounds(int m, int npl, const uint32_t *key, int32_t *seg)
+{
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= m) return;
+    const uint32_t q = key[t];
+    if (t == 0 || key[t - 1] != q) seg[q] = t;
+    if (t == m - 1 || key[t + 1] != q) seg[2 * (int64_t)npl + q] = t + 1;
+}
+
+// Sum s (body s's ahi, or body s - npl's ahj), 16 lanes: each fetches an entry's
+// term, and the first three fold the components.  sum carries on from the round
+// before unless first.
+__global__ __launch_bounds__(256) void k_flat_fold(int npl, const uint32_t *ent, const double4 *term, const int32_t *seg,
+                                                   double *sum, int first)
+{
+    // rows of the wavefront's four sums, two doubles apart in the banks
+    __shared__ __align__(16) double lt[4][4][66];
+    const int lane = threadIdx.x & 63, l = lane & 15, g = lane >> 4, comp = min(l, 2);
+    double *row = lt[threadIdx.x >> 6][g];
+    const int64_t s = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+    const bool on = s < 2 * (int64_t)npl;
+    const int e0 = on ? seg[s] : 0, e1 = on ? seg[2 * (int64_t)npl + s] : 0;
+    double h = on && !first ? sum[3 * s + comp] : 0.0;
+    // the entry numbers run a round ahead of the terms
+    uint32_t e = e0 + l < e1 ? ent[e0 + l] : 0;
+    for (int b = e0; __any(b < e1); b += 16) {
+        const double4 v = b + l < e1 ? term[e] : make_double4(0.0, 0.0, 0.0, 0.0);
+        e = b + 16 + l < e1 ? ent[b + 16 + l] : 0;
+        row[4 * l] = v.x;
+        row[4 * l + 1] = v.y;
+        row[4 * l + 2] = v.z;
+        row[4 * l + 3] = v.w;
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int q = 0; q < 16; q++) h = fma(row[4 * q + 3], row[4 * q + comp], h);
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (on && l < 3) sum[3 * s + l] = h;
+}
+
+// acc = (acc + ahi) + ahj, left as it is when an index was out of range
+__global__ __launch_bounds__(256) void k_flat_add(int npl, const double *sum, const int32_t *bad, double *acc)
+{
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, n = 3 * (int64_t)npl;
+    if (t < n && !*bad) acc[t] = (acc[t] + sum[t]) + sum[n + t];
 }
 
 // swiftest_kick_getacch_int_all_tp (swiftest_kick.f90:374-415): particle sum
@@ -1298,53 +1341,44 @@ int swg_kick_getacch_int_all_flat_pl(swg_ctx *ctx, int32_t npl, int64_t nplpl, c
     if (!ctx || npl < 0 || nplpl < 0) return fail(SWG_ERR_ARG, "bad argument");
     if (npl == 0) return 0;
     if (!r || !Gmass || !acc || (nplpl && !k_plpl)) return fail(SWG_ERR_ARG, "NULL array");
-    // per-body pair lists in list order (host counting sort)
-    std::vector<int64_t> rs(npl + 1, 0), cs(npl + 1, 0), rowl(nplpl ? nplpl : 1), coll(nplpl ? nplpl : 1);
-    for (int64_t p = 0; p < nplpl; p++) {
-        int i = k_plpl[2 * p] - 1, j = k_plpl[2 * p + 1] - 1;
-        if (i < 0 || i >= npl || j < 0 || j >= npl) return fail(SWG_ERR_ARG, "pair index out of range");
-        rs[i + 1]++;
-        cs[j + 1]++;
-    }
-    for (int b = 0; b < npl; b++) {
-        rs[b + 1] += rs[b];
-        cs[b + 1] += cs[b];
-    }
-    {
-        std::vector<int64_t> fr(rs.begin(), rs.end() - 1), fc(cs.begin(), cs.end() - 1);
-        for (int64_t p = 0; p < nplpl; p++) {
-            rowl[fr[k_plpl[2 * p] - 1]++] = p;
-            coll[fc[k_plpl[2 * p + 1] - 1]++] = p;
-        }
-    }
     int rc = 0;
     hipStream_t st = ctx->stream;
-    GETBUF(dr, double, 0, 3 * npl);
+    const int64_t m = std::min(nplpl, FLAT_PAIRS);
+    GETBUF(dr, double, 0, 3 * (int64_t)npl);
     GETBUF(dg, double, 1, npl);
-    GETBUF(da, double, 2, 3 * npl);
+    GETBUF(da, double, 2, 3 * (int64_t)npl);
     GETBUF(dk, int32_t, 4, 2 * (nplpl ? nplpl : 1));
-    GETBUF(drs, int64_t, 5, npl + 1);
-    GETBUF(dcs, int64_t, 6, npl + 1);
-    GETBUF(drl, int64_t, 7, rowl.size());
-    GETBUF(dcl, int64_t, 8, coll.size());
+    GETBUF(seg, int32_t, 5, 4 * (int64_t)npl);
+    GETBUF(sum, double, 6, 6 * (int64_t)npl);
+    GETBUF(term, double4, 7, 2 * (m ? m : 1));
+    GETBUF(keys, uint32_t, 8, 8 * (m ? m : 1));
+    GETBUF(bad, int32_t, 9, 1);
+    uint32_t *kin = keys, *vin = keys + 2 * m, *kout = keys + 4 * m, *vout = keys + 6 * m;
     double *dR = nullptr;
     if (radius) {
         GETBUF(t, double, 3, npl);
         dR = t;
-        HIPCHK(hipMemcpyAsync(dR, radius, npl * sizeof(double), hipMemcpyHostToDevice, st));
     }
-    HIPCHK(hipMemcpyAsync(dr, r, 3 * npl * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dg, Gmass, npl * sizeof(double), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(da, acc, 3 * npl * sizeof(double), hipMemcpyHostToDevice, st));
-    if (nplpl) HIPCHK(hipMemcpyAsync(dk, k_plpl, 2 * nplpl * sizeof(int32_t), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(drs, rs.data(), (npl + 1) * sizeof(int64_t), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dcs, cs.data(), (npl + 1) * sizeof(int64_t), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(drl, rowl.data(), rowl.size() * sizeof(int64_t), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(dcl, coll.data(), coll.size() * sizeof(int64_t), hipMemcpyHostToDevice, st));
-    k_leaf_flat<<<cdiv(npl, 128), 128, 0, st>>>(npl, dk, dr, dg, dR, drs, dcs, drl, dcl, da, ctx->pair_mode);
+    int32_t bad_h = 0;
+    const XferItem in[] = {xfer_i32(k_plpl, dk, 2 * nplpl),           xfer_words(r, dr, 3 * (int64_t)npl),
+                           xfer_words(Gmass, dg, npl),                xfer_words(radius, dR, radius ? npl : 0),
+                           xfer_words(acc, da, 3 * (int64_t)npl),     xfer_i32(&bad_h, bad, 1)};
+    HIPCHK(ctx->leaf->stage.in(st, in, 6));
+    int bits = 1;
+    while ((1ll << bits) < 2 * (int64_t)npl) bits++;
+    for (int64_t p = 0; p == 0 || p < nplpl; p += FLAT_PAIRS) {
+        const int n = (int)std::min(nplpl - p, FLAT_PAIRS);
+        k_flat_terms<<<cdiv(std::max(n, npl), 256), 256, 0, st>>>(n, (const int2 *)dk + p, npl, dr, dg, dR,
+                                                                  ctx->pair_mode != 0, kin, vin, term, seg, bad);
+        HIPCHK(sort_by_key(st, ctx->leaf->sort, kin, vin, kout, vout, 2 * (int64_t)n, bits));
+        if (n) k_flat_bounds<<<cdiv(2 * n, 256), 256, 0, st>>>(2 * n, npl, kout, seg);
+        k_flat_fold<<<cdiv(2 * (int64_t)npl, 16), 256, 0, st>>>(npl, vout, term, seg, sum, p == 0);
+    }
+    k_flat_add<<<cdiv(3 * (int64_t)npl, 256), 256, 0, st>>>(npl, sum, bad, da);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(acc, da, 3 * npl * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
+    const XferItem out[] = {xfer_words(acc, da, 3 * (int64_t)npl), xfer_i32(&bad_h, bad, 1)};
+    HIPCHK(ctx->leaf->stage.out(st, out, 2));
+    if (bad_h) return fail(SWG_ERR_ARG, "pair index out of range");
     return 0;
 }
 

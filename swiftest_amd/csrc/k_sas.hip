@@ -486,6 +486,12 @@ hipError_t sas_fill(hipStream_t st, SasWork &w, ListDev &pp, PlDev pl, int npl, 
     return hipGetLastError();
 }
 
+hipError_t sort_by_key(hipStream_t st, SasWork &w, const uint32_t *kin, const uint32_t *vin, uint32_t *kout,
+                       uint32_t *vout, int64_t n, int bits)
+{
+    return radix_sort<uint32_t>(st, w, kin, vin, kout, vout, n, 0, bits, nullptr, 0);
+}
+
 hipError_t sas_adjacency(hipStream_t st, SasWork &w, ListDev &pp, int npl, int64_t npp)
 {
     if (!npp) return hipSuccess;

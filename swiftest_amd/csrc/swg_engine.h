@@ -230,6 +230,7 @@ struct LeafState {
     ~LeafState();
     void *get(int slot, size_t bytes, int *rc);
     Stage stage;  // transfers of every call on the context, resident systems included
+    SasWork sort; // sort scratch of the pair-list sums
 };
 
 }  // namespace swg

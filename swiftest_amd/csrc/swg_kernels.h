@@ -175,6 +175,10 @@ hipError_t sas_fill(hipStream_t st, SasWork &w, ListDev &pp, PlDev pl, int npl, 
 // index2-side adjacency
 hipError_t sas_adjacency(hipStream_t st, SasWork &w, ListDev &pp, int npl, int64_t npp);
 
+// stable sort of n values by the low bits of their keys
+hipError_t sort_by_key(hipStream_t st, SasWork &w, const uint32_t *kin, const uint32_t *vin, uint32_t *kout,
+                       uint32_t *vout, int64_t n, int bits);
+
 // ---- SyMBA recursion, level 0 (k_enc.hip) ----
 void launch_list_check_pp(hipStream_t st, ListDev pp, PlDev pl, SysDev sy, int64_t n, int irec, double dt,
                           int32_t *any);
