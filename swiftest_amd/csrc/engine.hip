@@ -388,6 +388,7 @@ int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const in
     } else {
         launch_snapshot(st, pl, tp, sy, nsys, npl, 0);
         launch_init_tp_vb(st, tp, sy, ntp);
+        launch_reset_levels(st, pl, tp, sy, d_sub_stats, npl, ntp, nsys);
     }
     HIPCHK(hipStreamSynchronize(st));
     HIPCHK(hipGetLastError());
@@ -619,8 +620,8 @@ int Ensemble::recur0()
     // reads them while the device works
     if (int rc = build_begin(1, nullptr)) return rc;
     launch_level_kicks(st, la, nullptr, npl, ntp, 0, dth);
-    launch_drift(st, pl.rh, pl.vb, pl.status, pl.levelg, pl.sys, sy.GMcb, sy.err, sy.frozen, npl, dt, 0, 1, 0);
-    launch_drift(st, tp.rh, tp.vb, tp.status, tp.levelg, tp.sys, sy.GMcb, sy.err, sy.frozen, ntp, dt, 0, 1, 1);
+    launch_drift(st, DriftSet{pl.rh, pl.vb, pl.status, pl.levelg, pl.sys, npl},
+                 DriftSet{tp.rh, tp.vb, tp.status, tp.levelg, tp.sys, ntp}, sy, dt, 0, 1);
     int32_t lenc = 0;
     if (int rc = build_wait(lenc)) return rc;
     if (lenc) {
@@ -1024,10 +1025,13 @@ int Ensemble::step_helio_symba()
     st_.npltp_enc = 0;
     st_.max_depth = -1;
     st_.nsubsteps = 0;
-    launch_reset_levels(st, pl, tp, sy, d_sub_stats, npl, ntp, nsys);
     npp = npt = 0;
     bool any = false;
+    int max_npl = 0;
+    for (int s = 0; s < nsys; s++) max_npl = std::max(max_npl, h_pl_off[s + 1] - h_pl_off[s]);
     if (symba) {
+        // HELIO steps use none of these; they stay as the build left them
+        launch_reset_levels(st, pl, tp, sy, d_sub_stats, npl, ntp, nsys);
         if (int rc = prm.encounter_check == 1 ? detect_pp_sas(dt) : detect_pp(dt)) return rc;
         trace_mark(st, "detect pl-pl");
         if (int rc = err_code()) return rc;
@@ -1059,31 +1063,24 @@ int Ensemble::step_helio_symba()
     auto kick_tp = [&](int lbeg) -> int {
         if (ktiming && ntiles_tp)
             if (int rc = record_kernel_event(ev_tp, nev_tp)) return rc;
-        launch_kick_tp(st, tune, tp, pl, sy, pt, d_tiles_tp, ntiles_tp, dth, lbeg, npt > 0);
+        launch_kick_tp(st, tune, tp, pl, sy, pt, d_tiles_tp, ntiles_tp, dth, lbeg, npt > 0, lbeg ? TP_PRE : TP_POST);
         if (ktiming && ntiles_tp)
             if (int rc = record_kernel_event(ev_tp, nev_tp)) return rc;
         return 0;
     };
     // first half: pl then tp
     auto first_half = [&]() -> int {
-        launch_sums_begin(st, pl, sy, nsys, 0);
-        launch_pl_begin_apply(st, pl, sy, npl, dth, 0);
+        launch_sums_begin(st, pl, sy, nsys, npl, max_npl, dth, 0);
         if (int rc = kick_pl(1)) return rc;
-        launch_drift(st, pl.rh, pl.vb, pl.status, pl.levelg, pl.sys, sy.GMcb, sy.err, sy.frozen, npl, dt, -1, symba,
-                     0);
-        launch_tp_pre(st, tp, sy, ntp, dth);
-        if (int rc = kick_tp(1)) return rc;
-        launch_drift(st, tp.rh, tp.vb, tp.status, tp.levelg, tp.sys, sy.GMcb, sy.err, sy.frozen, ntp, dt, -1, symba,
-                     1);
+        if (int rc = kick_tp(1)) return rc;  // at the massive bodies' rbeg, so their drift can wait
+        launch_drift(st, DriftSet{pl.rh, pl.vb, pl.status, pl.levelg, pl.sys, npl},
+                     DriftSet{tp.rh, tp.vb, tp.status, tp.levelg, tp.sys, ntp}, sy, dt, -1, symba);
         return 0;
     };
     auto second_half = [&]() -> int {
         if (int rc = kick_pl(0)) return rc;
-        launch_sums_end(st, pl, sy, nsys);
-        launch_pl_end_apply(st, pl, sy, npl, dth);
+        launch_sums_end(st, pl, sy, nsys, npl, max_npl, dth);
         if (int rc = kick_tp(0)) return rc;
-        launch_tp_post(st, tp, sy, ntp, dth);
-        launch_lfirst_update(st, sy, nsys);
         return 0;
     };
     if (int rc = run_phase(0, first_half)) return rc;
@@ -1274,9 +1271,9 @@ int Ensemble::time_kernels(int reps, double *ms_tp, double *ms_pl)
     const int use_radius = prm.integrator == SWG_SYMBA || prm.lclose;
     float ms = 0.f;
     if (ms_tp) {
-        launch_kick_tp(st, tune, tp, pl, sy, pt, d_tiles_tp, ntiles_tp, 0.0, 1, 0);  // warm-up
+        launch_kick_tp(st, tune, tp, pl, sy, pt, d_tiles_tp, ntiles_tp, 0.0, 1, 0, TP_KICK);  // warm-up
         HIPCHK(hipEventRecord(ev0, st));
-        for (int r = 0; r < reps; r++) launch_kick_tp(st, tune, tp, pl, sy, pt, d_tiles_tp, ntiles_tp, 0.0, 1, 0);
+        for (int r = 0; r < reps; r++) launch_kick_tp(st, tune, tp, pl, sy, pt, d_tiles_tp, ntiles_tp, 0.0, 1, 0, TP_KICK);
         HIPCHK(hipEventRecord(ev1, st));
         HIPCHK(hipEventSynchronize(ev1));
         HIPCHK(hipEventElapsedTime(&ms, ev0, ev1));
@@ -1497,7 +1494,7 @@ int Ensemble::accel(double *pl_acc, double *tp_acc)
     }
     const int use_radius = prm.integrator == SWG_SYMBA || prm.lclose;
     launch_kick_pl(st, tune, pl, sy, pp, d_tiles_pl, ntiles_pl, 1.0, 1, use_radius, 0);
-    launch_kick_tp(st, tune, tp, pl, sy, pt, d_tiles_tp, ntiles_tp, 1.0, 1, 0);
+    launch_kick_tp(st, tune, tp, pl, sy, pt, d_tiles_tp, ntiles_tp, 1.0, 1, 0, TP_KICK);
     HIPCHK(hipGetLastError());
     const XferItem x[] = {xfer_vec3(pl_acc, pl.vb, pl_acc ? npl : 0), xfer_vec3(tp_acc, tp.vb, tp_acc ? ntp : 0)};
     HIPCHK(stage->out(st, x, 2));

@@ -65,6 +65,10 @@ __global__ void k_reset_levels(PlDev pl, TpDev tp, SysDev sy, int32_t *sub_stats
 // side by side) 53 -> 14.5 us, against staging and adding in turn with eight
 // terms read ahead.
 constexpr int SUM_T = 256, SUM_CH = 384;
+// largest system whose bodies the workgroup of its sums updates too: four rounds
+// of its threads take about what a launch does (2.5 us for a few bodies, 4.8 us
+// at 2000)
+constexpr int SUM_APPLY = 1024;
 
 struct SumStage {
     // the terms of up to six sums; two words more a row than the banks wrap at,
@@ -182,15 +186,32 @@ __device__ inline double sums_gm_vh(SumStage &S, const PlDev &pl, int p0, int p1
     return acc;
 }
 
+// vb = vh + cb%vb when lfirst; then the linear drift rh += pt*dt
+// (helio_drift.f90:129-163, masked)
+__device__ inline void pl_begin_one(const PlDev &pl, int i, bool first, const double *cb, const double *pt, double dth)
+{
+    if (first) {
+        pl.vb.x[i] = pl.vh.x[i] + cb[0];
+        pl.vb.y[i] = pl.vh.y[i] + cb[1];
+        pl.vb.z[i] = pl.vh.z[i] + cb[2];
+    }
+    if (pl_active(pl, i)) {
+        pl.rh.x[i] = fma(pt[0], dth, pl.rh.x[i]);
+        pl.rh.y[i] = fma(pt[1], dth, pl.rh.y[i]);
+        pl.rh.z[i] = fma(pt[2], dth, pl.rh.z[i]);
+    }
+}
+
 // Start of a step:
 //   vh->vb (swiftest_util.f90:424-459) when lfirst: cb%vb = -sum(Gm vh) / (GM_cb + sum(Gm))
 //   lindrift pt (helio_drift.f90:129-163): pt = sum_masked(Gm vb) / GM_cb
 // Lane 0 sums Gm, lanes 1-3 the components of sum(Gm vh); then lanes 0-2 the
-// components of pt.
-__global__ __launch_bounds__(SUM_T) void k_sums_begin(PlDev pl, SysDev sy, int nsys, int force)
+// components of pt.  With apply the workgroup goes on to its bodies what
+// k_pl_begin_apply does.
+__global__ __launch_bounds__(SUM_T) void k_sums_begin(PlDev pl, SysDev sy, int nsys, int force, double dth, int apply)
 {
     __shared__ SumStage S;
-    __shared__ double shr[4], scb[3];
+    __shared__ double shr[4], scb[3], spt[3];
     const int s = blockIdx.x, tid = threadIdx.x;
     const int p0 = sy.pl_off[s], p1 = sy.pl_off[s + 1];
     if (p1 == p0 || sy.frozen[s]) return;
@@ -221,26 +242,21 @@ __global__ __launch_bounds__(SUM_T) void k_sums_begin(PlDev pl, SysDev sy, int n
         [&](int b, int n) {
             if (tid < 3) pt = chain(pt, S.t[b][tid], n);
         });
-    if (tid < 3) sy.ptbeg[3 * s + tid] = pt / sy.GMcb[s];
+    if (tid < 3) spt[tid] = sy.ptbeg[3 * s + tid] = pt / sy.GMcb[s];
+    if (!apply) return;
+    __syncthreads();
+    const double cb[3] = {first ? scb[0] : 0.0, first ? scb[1] : 0.0, first ? scb[2] : 0.0};
+    const double p[3] = {spt[0], spt[1], spt[2]};
+    for (int i = p0 + tid; i < p1; i += SUM_T) pl_begin_one(pl, i, first, cb, p, dth);
 }
 
-// vb = vh + cb%vb when lfirst; then the linear drift rh += pt*dt
 __global__ void k_pl_begin_apply(PlDev pl, SysDev sy, int npl, double dth, int force)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= npl) return;
     int s = pl.sys[i];
     if (sy.frozen[s]) return;
-    if (force || sy.lfirst[s]) {
-        pl.vb.x[i] = pl.vh.x[i] + sy.cbvb[3 * s];
-        pl.vb.y[i] = pl.vh.y[i] + sy.cbvb[3 * s + 1];
-        pl.vb.z[i] = pl.vh.z[i] + sy.cbvb[3 * s + 2];
-    }
-    if (pl_active(pl, i)) {
-        pl.rh.x[i] = fma(sy.ptbeg[3 * s], dth, pl.rh.x[i]);
-        pl.rh.y[i] = fma(sy.ptbeg[3 * s + 1], dth, pl.rh.y[i]);
-        pl.rh.z[i] = fma(sy.ptbeg[3 * s + 2], dth, pl.rh.z[i]);
-    }
+    pl_begin_one(pl, i, force || sy.lfirst[s], sy.cbvb + 3 * s, sy.ptbeg + 3 * s, dth);
 }
 
 // Massive-body half kick (helio_kick_vb_pl, helio_kick.f90:91-132):
@@ -632,16 +648,49 @@ __global__ __launch_bounds__(64 * K) void k_kick_pl_fast(PlDev pl, SysDev sy, Li
     }
 }
 
+// What a step does to particle j before its first half kick (phase TP_PRE) and
+// after its second (TP_POST): part of the kicks, on the kick's lane, in place of
+// two launches that pass over the particles again (3.7 us each for 20000; with
+// the sums' updates, both drifts in one launch and no reset, a HELIO step is
+// seven launches in place of fifteen: five driver steps of a small system 904 ->
+// 786 us).
+// Before: vb = vh - ptbeg when lfirst (swiftest_util.f90:398-421), then
+// rh += ptbeg*dt (helio_drift.f90:166-200).
+__device__ inline void tp_pre(const TpDev &tp, const SysDev &sy, int s, int j, double dth)
+{
+    const double px = sy.ptbeg[3 * s], py = sy.ptbeg[3 * s + 1], pz = sy.ptbeg[3 * s + 2];
+    if (sy.lfirst[s]) {
+        tp.vb.x[j] = tp.vh.x[j] + (-px);
+        tp.vb.y[j] = tp.vh.y[j] + (-py);
+        tp.vb.z[j] = tp.vh.z[j] + (-pz);
+    }
+    tp.rh.x[j] = fma(px, dth, tp.rh.x[j]);
+    tp.rh.y[j] = fma(py, dth, tp.rh.y[j]);
+    tp.rh.z[j] = fma(pz, dth, tp.rh.z[j]);
+}
+// After: rh += ptend*dt, vh = vb + ptend (vb2vh with vbcb = -ptend)
+__device__ inline void tp_post(const TpDev &tp, const SysDev &sy, int s, int j, double dth)
+{
+    const double px = sy.ptend[3 * s], py = sy.ptend[3 * s + 1], pz = sy.ptend[3 * s + 2];
+    tp.rh.x[j] = fma(px, dth, tp.rh.x[j]);
+    tp.rh.y[j] = fma(py, dth, tp.rh.y[j]);
+    tp.rh.z[j] = fma(pz, dth, tp.rh.z[j]);
+    tp.vh.x[j] = tp.vb.x[j] - (-px);
+    tp.vh.y[j] = tp.vb.y[j] - (-py);
+    tp.vh.z[j] = tp.vb.z[j] - (-pz);
+}
+
 // Test particles: one lane per particle, the massive bodies at wave-uniform
 // indices, four per iteration.
 template <int BLK>
 __global__ __launch_bounds__(BLK) void k_kick_tp_fast(TpDev tp, PlDev pl, SysDev sy, ListDev pt, const Tile *tiles,
-                                                      double dt, int lbeg, int do_pairs)
+                                                      double dt, int lbeg, int do_pairs, int phase)
 {
     const Tile tl = tiles[blockIdx.x];
     const int p0 = sy.pl_off[tl.s], p1 = sy.pl_off[tl.s + 1];
     const int j = tl.b0 + (int)threadIdx.x;
     const bool valid = (j < tl.b1) && tp_active(tp, j);
+    if (phase == TP_PRE && valid) tp_pre(tp, sy, tl.s, j, dt);
     const Vec3p rp = lbeg ? pl.rbeg : pl.rend;
     double xt = 0.0, yt = 0.0, zt = 0.0;
     if (valid) {
@@ -715,24 +764,29 @@ __global__ __launch_bounds__(BLK) void k_kick_tp_fast(TpDev tp, PlDev pl, SysDev
     tp.vb.x[j] = fma(ax, dt, tp.vb.x[j]);
     tp.vb.y[j] = fma(ay, dt, tp.vb.y[j]);
     tp.vb.z[j] = fma(az, dt, tp.vb.z[j]);
+    if (phase == TP_POST) tp_post(tp, sy, tl.s, j, dt);
 }
 
 // Danby drift of the masked bodies (helio_drift_body, helio_drift.f90:14-54,
 // with the SyMBA level mask of symba_drift.f90:14-61): mu = GM_cb, (rh, vb).
-__global__ __launch_bounds__(256) void k_drift(Vec3p r, Vec3p v, int32_t *status, const int32_t *levelg, const int32_t *sys,
-                        const double *GMcb, int32_t *err, const int32_t *frozen, int n, double dt, int irec,
-                        int use_level, int is_tp)
+// The massive bodies take the first pl_blocks workgroups, the particles the
+// others: one launch for both.
+__global__ __launch_bounds__(256) void k_drift(DriftSet pl, DriftSet tp, int pl_blocks, SysDev sy, double dt, int irec,
+                                               int use_level)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int st = status[i];
+    const bool is_tp = (int)blockIdx.x >= pl_blocks;
+    const DriftSet &d = is_tp ? tp : pl;
+    const int i = ((int)blockIdx.x - (is_tp ? pl_blocks : 0)) * blockDim.x + threadIdx.x;
+    if (i >= d.n) return;
+    const Vec3p r = d.r, v = d.v;
+    int st = d.status[i];
     bool m = is_tp ? (st == ACTIVE) : (st != INACTIVE);
-    if (use_level) m = m && (levelg[i] == irec);
+    if (use_level) m = m && (d.levelg[i] == irec);
     if (!m) return;
-    int s = sys[i];
-    if (frozen[s]) return;
+    int s = d.sys[i];
+    if (sy.frozen[s]) return;
     double rx = r.x[i], ry = r.y[i], rz = r.z[i], vx = v.x[i], vy = v.y[i], vz = v.z[i];
-    int fl = drift_one(GMcb[s], rx, ry, rz, vx, vy, vz, dt);
+    int fl = drift_one(sy.GMcb[s], rx, ry, rz, vx, vy, vz, dt);
     r.x[i] = rx;
     r.y[i] = ry;
     r.z[i] = rz;
@@ -740,28 +794,9 @@ __global__ __launch_bounds__(256) void k_drift(Vec3p r, Vec3p v, int32_t *status
     v.y[i] = vy;
     v.z[i] = vz;
     if (fl != 0) {
-        status[i] = DISCARDED_DRIFTERR;
-        if (!is_tp) atomicOr(&err[s], 2);
+        d.status[i] = DISCARDED_DRIFTERR;
+        if (!is_tp) atomicOr(&sy.err[s], 2);
     }
-}
-
-// Test particles at the start of a step: vb = vh - ptbeg when lfirst
-// (swiftest_util.f90:398-421), then rh += ptbeg*dt (helio_drift.f90:166-200).
-__global__ void k_tp_pre(TpDev tp, SysDev sy, int ntp, double dth)
-{
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= ntp || !tp_active(tp, j)) return;
-    int s = tp.sys[j];
-    if (sy.frozen[s]) return;
-    double px = sy.ptbeg[3 * s], py = sy.ptbeg[3 * s + 1], pz = sy.ptbeg[3 * s + 2];
-    if (sy.lfirst[s]) {
-        tp.vb.x[j] = tp.vh.x[j] + (-px);
-        tp.vb.y[j] = tp.vh.y[j] + (-py);
-        tp.vb.z[j] = tp.vh.z[j] + (-pz);
-    }
-    tp.rh.x[j] = fma(px, dth, tp.rh.x[j]);
-    tp.rh.y[j] = fma(py, dth, tp.rh.y[j]);
-    tp.rh.z[j] = fma(pz, dth, tp.rh.z[j]);
 }
 
 // Test-particle half kick (helio_kick_vb_tp, helio_kick.f90:135-169):
@@ -772,13 +807,14 @@ __global__ void k_tp_pre(TpDev tp, SysDev sy, int ntp, double dth)
 //       order (symba_kick.f90:106-119);  vb += ah*dt.
 template <int BLK>
 __global__ __launch_bounds__(BLK) void k_kick_tp(TpDev tp, PlDev pl, SysDev sy, ListDev pt, const Tile *tiles,
-                                                 double dt, int lbeg, int do_pairs)
+                                                 double dt, int lbeg, int do_pairs, int phase)
 {
     __shared__ double sx[BLK], syy[BLK], sz[BLK], sgm[BLK];
     const Tile tl = tiles[blockIdx.x];
     const int p0 = sy.pl_off[tl.s], p1 = sy.pl_off[tl.s + 1];
     const int j = tl.b0 + (int)threadIdx.x;
     const bool valid = (j < tl.b1) && tp_active(tp, j);
+    if (phase == TP_PRE && valid) tp_pre(tp, sy, tl.s, j, dt);
     const Vec3p rp = lbeg ? pl.rbeg : pl.rend;
     double xt = 0.0, yt = 0.0, zt = 0.0;
     if (valid) {
@@ -859,6 +895,20 @@ __global__ __launch_bounds__(BLK) void k_kick_tp(TpDev tp, PlDev pl, SysDev sy, 
     tp.vb.x[j] = fma(ax, dt, tp.vb.x[j]);
     tp.vb.y[j] = fma(ay, dt, tp.vb.y[j]);
     tp.vb.z[j] = fma(az, dt, tp.vb.z[j]);
+    if (phase == TP_POST) tp_post(tp, sy, tl.s, j, dt);
+}
+
+// rh += ptend*dt (masked); vh = vb - cb%vb (all bodies)
+__device__ inline void pl_end_one(const PlDev &pl, int i, const double *cb, const double *pt, double dth)
+{
+    if (pl_active(pl, i)) {
+        pl.rh.x[i] = fma(pt[0], dth, pl.rh.x[i]);
+        pl.rh.y[i] = fma(pt[1], dth, pl.rh.y[i]);
+        pl.rh.z[i] = fma(pt[2], dth, pl.rh.z[i]);
+    }
+    pl.vh.x[i] = pl.vb.x[i] - cb[0];
+    pl.vh.y[i] = pl.vb.y[i] - cb[1];
+    pl.vh.z[i] = pl.vb.z[i] - cb[2];
 }
 
 // Per-system sums at the end of a step:
@@ -866,12 +916,19 @@ __global__ __launch_bounds__(BLK) void k_kick_tp(TpDev tp, PlDev pl, SysDev sy, 
 //   vb->vh (swiftest_util.f90:363-395): cb%vb -= Gm vb / GM_cb over
 //   i = npl..1, active only (backward, lanes 3-5): the two walk the bodies
 //   from both ends side by side
-__global__ __launch_bounds__(SUM_T) void k_sums_end(PlDev pl, SysDev sy, int nsys)
+// With apply the workgroup goes on to its bodies what k_pl_end_apply does.
+// lfirst: the HELIO branch clears it after its vh->vb; the encounter branch
+// keeps it (helio_step.f90:58-61 vs symba_step.f90:81, then symba_step.f90:47);
+// nothing of a step reads it after this.
+__global__ __launch_bounds__(SUM_T) void k_sums_end(PlDev pl, SysDev sy, int nsys, double dth, int apply)
 {
     __shared__ SumStage S;
+    __shared__ double sv[6];
     const int s = blockIdx.x, tid = threadIdx.x;
     const int p0 = sy.pl_off[s], p1 = sy.pl_off[s + 1];
-    if (p1 == p0 || sy.frozen[s]) return;
+    if (sy.frozen[s]) return;
+    if (tid == 0 && sy.lfirst[s] && !(sy.enc_pp[s] || sy.enc_pt[s])) sy.lfirst[s] = 0;
+    if (p1 == p0) return;
     const double gm = sy.GMcb[s];
     double acc = 0.0;
     sums_chunks<true>(
@@ -887,51 +944,21 @@ __global__ __launch_bounds__(SUM_T) void k_sums_end(PlDev pl, SysDev sy, int nsy
         [&](int b, int n) {
             if (tid < 6) acc = chain(acc, S.t[b][tid], n);
         });
-    if (tid < 3) sy.ptend[3 * s + tid] = acc / gm;
-    else if (tid < 6) sy.cbvb[3 * s + tid - 3] = acc;
+    if (tid < 3) sv[tid] = sy.ptend[3 * s + tid] = acc / gm;
+    else if (tid < 6) sv[tid] = sy.cbvb[3 * s + tid - 3] = acc;
+    if (!apply) return;
+    __syncthreads();
+    const double p[3] = {sv[0], sv[1], sv[2]}, cb[3] = {sv[3], sv[4], sv[5]};
+    for (int i = p0 + tid; i < p1; i += SUM_T) pl_end_one(pl, i, cb, p, dth);
 }
 
-// rh += ptend*dt (masked); vh = vb - cb%vb (all bodies)
 __global__ void k_pl_end_apply(PlDev pl, SysDev sy, int npl, double dth)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= npl) return;
     int s = pl.sys[i];
     if (sy.frozen[s]) return;
-    if (pl_active(pl, i)) {
-        pl.rh.x[i] = fma(sy.ptend[3 * s], dth, pl.rh.x[i]);
-        pl.rh.y[i] = fma(sy.ptend[3 * s + 1], dth, pl.rh.y[i]);
-        pl.rh.z[i] = fma(sy.ptend[3 * s + 2], dth, pl.rh.z[i]);
-    }
-    pl.vh.x[i] = pl.vb.x[i] - sy.cbvb[3 * s];
-    pl.vh.y[i] = pl.vb.y[i] - sy.cbvb[3 * s + 1];
-    pl.vh.z[i] = pl.vb.z[i] - sy.cbvb[3 * s + 2];
-}
-
-// Test particles at the end of a step: rh += ptend*dt, vh = vb + ptend
-// (vb2vh with vbcb = -ptend)
-__global__ void k_tp_post(TpDev tp, SysDev sy, int ntp, double dth)
-{
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= ntp || !tp_active(tp, j)) return;
-    int s = tp.sys[j];
-    if (sy.frozen[s]) return;
-    double px = sy.ptend[3 * s], py = sy.ptend[3 * s + 1], pz = sy.ptend[3 * s + 2];
-    tp.rh.x[j] = fma(px, dth, tp.rh.x[j]);
-    tp.rh.y[j] = fma(py, dth, tp.rh.y[j]);
-    tp.rh.z[j] = fma(pz, dth, tp.rh.z[j]);
-    tp.vh.x[j] = tp.vb.x[j] - (-px);
-    tp.vh.y[j] = tp.vb.y[j] - (-py);
-    tp.vh.z[j] = tp.vb.z[j] - (-pz);
-}
-
-// The HELIO branch clears lfirst after its vh->vb; the encounter branch keeps
-// it (helio_step.f90:58-61 vs symba_step.f90:81, then symba_step.f90:47).
-__global__ void k_lfirst_update(SysDev sy, int nsys)
-{
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsys || sy.frozen[s]) return;
-    if (sy.lfirst[s] && !(sy.enc_pp[s] || sy.enc_pt[s])) sy.lfirst[s] = 0;
+    pl_end_one(pl, i, sy.cbvb + 3 * s, sy.ptend + 3 * s, dth);
 }
 
 // Snapshot coordinate refresh (swiftest_util.f90:2663-2682): pl vh->vb, then
@@ -1025,13 +1052,13 @@ void launch_reset_levels(hipStream_t st, PlDev pl, TpDev tp, SysDev sy, int32_t 
     const int n = std::max(std::max(npl, ntp), std::max(nsys, 4));
     k_reset_levels<<<cdiv(n, 256), 256, 0, st>>>(pl, tp, sy, sub_stats, npl, ntp, nsys);
 }
-void launch_sums_begin(hipStream_t st, PlDev pl, SysDev sy, int nsys, int force)
+// max_npl: the largest system's bodies.  Up to SUM_APPLY the sums' workgroup
+// updates its bodies itself.
+void launch_sums_begin(hipStream_t st, PlDev pl, SysDev sy, int nsys, int npl, int max_npl, double dth, int force)
 {
-    k_sums_begin<<<nsys, SUM_T, 0, st>>>(pl, sy, nsys, force);
-}
-void launch_pl_begin_apply(hipStream_t st, PlDev pl, SysDev sy, int npl, double dth, int force)
-{
-    if (npl) k_pl_begin_apply<<<cdiv(npl, 256), 256, 0, st>>>(pl, sy, npl, dth, force);
+    const int apply = max_npl <= SUM_APPLY;
+    k_sums_begin<<<nsys, SUM_T, 0, st>>>(pl, sy, nsys, force, dth, apply);
+    if (npl && !apply) k_pl_begin_apply<<<cdiv(npl, 256), 256, 0, st>>>(pl, sy, npl, dth, force);
 }
 void launch_kick_pl(hipStream_t st, const Tuning &tu, PlDev pl, SysDev sy, ListDev pp, const Tile *tiles,
                     int ntiles, double dt, int lbeg, int use_radius, int do_pairs)
@@ -1070,51 +1097,34 @@ void launch_kick_pl(hipStream_t st, const Tuning &tu, PlDev pl, SysDev sy, ListD
     default: k_kick_pl<256><<<ntiles, 256, 0, st>>>(pl, sy, pp, tiles, dt, lbeg, use_radius, do_pairs); break;
     }
 }
-void launch_drift(hipStream_t st, Vec3p r, Vec3p v, int32_t *status, int32_t *levelg, const int32_t *sys,
-                  const double *GMcb, int32_t *err, const int32_t *frozen, int n, double dt, int irec, int use_level,
-                  int is_tp)
+void launch_drift(hipStream_t st, const DriftSet &pl, const DriftSet &tp, SysDev sy, double dt, int irec, int use_level)
 {
-    if (n)
-        k_drift<<<cdiv(n, 128), 128, 0, st>>>(r, v, status, levelg, sys, GMcb, err, frozen, n, dt, irec, use_level,
-                                              is_tp);
-}
-void launch_tp_pre(hipStream_t st, TpDev tp, SysDev sy, int ntp, double dth)
-{
-    if (ntp) k_tp_pre<<<cdiv(ntp, 256), 256, 0, st>>>(tp, sy, ntp, dth);
+    const int pb = cdiv(pl.n, 128), tb = cdiv(tp.n, 128);
+    if (pb + tb) k_drift<<<pb + tb, 128, 0, st>>>(pl, tp, pb, sy, dt, irec, use_level);
 }
 void launch_kick_tp(hipStream_t st, const Tuning &tu, TpDev tp, PlDev pl, SysDev sy, ListDev pt,
-                    const Tile *tiles, int ntiles, double dt, int lbeg, int do_pairs)
+                    const Tile *tiles, int ntiles, double dt, int lbeg, int do_pairs, int phase)
 {
     if (!ntiles) return;
     if (tu.pair_fast) {
         switch (tu.kick_tp_block) {
-        case 64: k_kick_tp_fast<64><<<ntiles, 64, 0, st>>>(tp, pl, sy, pt, tiles, dt, lbeg, do_pairs); break;
-        case 128: k_kick_tp_fast<128><<<ntiles, 128, 0, st>>>(tp, pl, sy, pt, tiles, dt, lbeg, do_pairs); break;
-        default: k_kick_tp_fast<256><<<ntiles, 256, 0, st>>>(tp, pl, sy, pt, tiles, dt, lbeg, do_pairs); break;
+        case 64: k_kick_tp_fast<64><<<ntiles, 64, 0, st>>>(tp, pl, sy, pt, tiles, dt, lbeg, do_pairs, phase); break;
+        case 128: k_kick_tp_fast<128><<<ntiles, 128, 0, st>>>(tp, pl, sy, pt, tiles, dt, lbeg, do_pairs, phase); break;
+        default: k_kick_tp_fast<256><<<ntiles, 256, 0, st>>>(tp, pl, sy, pt, tiles, dt, lbeg, do_pairs, phase); break;
         }
         return;
     }
     switch (tu.kick_tp_block) {
-    case 64: k_kick_tp<64><<<ntiles, 64, 0, st>>>(tp, pl, sy, pt, tiles, dt, lbeg, do_pairs); break;
-    case 128: k_kick_tp<128><<<ntiles, 128, 0, st>>>(tp, pl, sy, pt, tiles, dt, lbeg, do_pairs); break;
-    default: k_kick_tp<256><<<ntiles, 256, 0, st>>>(tp, pl, sy, pt, tiles, dt, lbeg, do_pairs); break;
+    case 64: k_kick_tp<64><<<ntiles, 64, 0, st>>>(tp, pl, sy, pt, tiles, dt, lbeg, do_pairs, phase); break;
+    case 128: k_kick_tp<128><<<ntiles, 128, 0, st>>>(tp, pl, sy, pt, tiles, dt, lbeg, do_pairs, phase); break;
+    default: k_kick_tp<256><<<ntiles, 256, 0, st>>>(tp, pl, sy, pt, tiles, dt, lbeg, do_pairs, phase); break;
     }
 }
-void launch_sums_end(hipStream_t st, PlDev pl, SysDev sy, int nsys)
+void launch_sums_end(hipStream_t st, PlDev pl, SysDev sy, int nsys, int npl, int max_npl, double dth)
 {
-    k_sums_end<<<nsys, SUM_T, 0, st>>>(pl, sy, nsys);
-}
-void launch_pl_end_apply(hipStream_t st, PlDev pl, SysDev sy, int npl, double dth)
-{
-    if (npl) k_pl_end_apply<<<cdiv(npl, 256), 256, 0, st>>>(pl, sy, npl, dth);
-}
-void launch_tp_post(hipStream_t st, TpDev tp, SysDev sy, int ntp, double dth)
-{
-    if (ntp) k_tp_post<<<cdiv(ntp, 256), 256, 0, st>>>(tp, sy, ntp, dth);
-}
-void launch_lfirst_update(hipStream_t st, SysDev sy, int nsys)
-{
-    k_lfirst_update<<<cdiv(nsys, 256), 256, 0, st>>>(sy, nsys);
+    const int apply = max_npl <= SUM_APPLY;
+    k_sums_end<<<nsys, SUM_T, 0, st>>>(pl, sy, nsys, dth, apply);
+    if (npl && !apply) k_pl_end_apply<<<cdiv(npl, 256), 256, 0, st>>>(pl, sy, npl, dth);
 }
 void launch_snapshot(hipStream_t st, PlDev pl, TpDev tp, SysDev sy, int nsys, int npl, int ntp)
 {

@@ -73,20 +73,22 @@ struct CopyList {
     int n;
 };
 void launch_copy_list(hipStream_t st, const CopyList &c);
-void launch_sums_begin(hipStream_t st, PlDev pl, SysDev sy, int nsys, int force_vh2vb);
-void launch_pl_begin_apply(hipStream_t st, PlDev pl, SysDev sy, int npl, double dth, int force_vh2vb);
+void launch_sums_begin(hipStream_t st, PlDev pl, SysDev sy, int nsys, int npl, int max_npl, double dth, int force_vh2vb);
 void launch_kick_pl(hipStream_t st, const Tuning &tu, PlDev pl, SysDev sy, ListDev pp, const Tile *tiles,
                     int ntiles, double dt, int lbeg, int use_radius, int do_pairs);
-void launch_drift(hipStream_t st, Vec3p r, Vec3p v, int32_t *status, int32_t *levelg, const int32_t *sys,
-                  const double *GMcb, int32_t *err, const int32_t *frozen, int n, double dt, int irec, int use_level,
-                  int is_tp);
-void launch_tp_pre(hipStream_t st, TpDev tp, SysDev sy, int ntp, double dth);
+// massive bodies or particles to drift (n = 0: none)
+struct DriftSet {
+    Vec3p r, v;
+    int32_t *status;
+    const int32_t *levelg, *sys;
+    int n;
+};
+void launch_drift(hipStream_t st, const DriftSet &pl, const DriftSet &tp, SysDev sy, double dt, int irec, int use_level);
+// what of a step the kick takes along (a kick by itself: TP_KICK)
+enum { TP_KICK = 0, TP_PRE = 1, TP_POST = 2 };
 void launch_kick_tp(hipStream_t st, const Tuning &tu, TpDev tp, PlDev pl, SysDev sy, ListDev pt,
-                    const Tile *tiles, int ntiles, double dt, int lbeg, int do_pairs);
-void launch_sums_end(hipStream_t st, PlDev pl, SysDev sy, int nsys);
-void launch_pl_end_apply(hipStream_t st, PlDev pl, SysDev sy, int npl, double dth);
-void launch_tp_post(hipStream_t st, TpDev tp, SysDev sy, int ntp, double dth);
-void launch_lfirst_update(hipStream_t st, SysDev sy, int nsys);
+                    const Tile *tiles, int ntiles, double dt, int lbeg, int do_pairs, int phase);
+void launch_sums_end(hipStream_t st, PlDev pl, SysDev sy, int nsys, int npl, int max_npl, double dth);
 void launch_snapshot(hipStream_t st, PlDev pl, TpDev tp, SysDev sy, int nsys, int npl, int ntp);
 void launch_init_tp_vb(hipStream_t st, TpDev tp, SysDev sy, int ntp);
 void launch_init_one(hipStream_t st, PlDev pl, TpDev tp, SysDev sy, int s);
