@@ -622,6 +622,10 @@ __global__ void k_whm_h2j_all(WhmArgs a, int nsys)
 // prefixes, ah0, ah2) is formed by each lane from the terms the bodies' lanes
 // put in LDS, added in the order of whm_coord.f90 / whm_kick.f90, so every
 // value equals the one the per-step kernels above (and the oracle) produce.
+// Bound: the latency of one step's chain on the bodies' wavefront (maps, drift,
+// accelerations).  Pairs are taken four at a time, their factors side by side,
+// the sums' terms are read ahead, and what holds for the whole run is formed
+// once: 8 bodies and 1000 particles 9.5 -> 7.3 us a step.
 // ---------------------------------------------------------------------------
 constexpr int WR_N = 64;
 
@@ -631,6 +635,20 @@ __device__ inline void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// gm_over_r3 of four pairs, side by side; use: the pair's factor is needed
+__device__ inline void whm_factors(const double (&g)[4], const double (&r2)[4], const bool (&use)[4], bool gok,
+                                   double (&f)[4])
+{
+    uint32_t far = 0;
+#pragma unroll
+    for (int u = 0; u < 4; u++) far = max(far, use[u] ? (uint32_t)(__double2hiint(r2[u]) - PAIR_R2_LO_HI) : 0u);
+    pair_factors<4>(g, r2, f);
+    if (!gok || __any(far > PAIR_R2_HI_HI - PAIR_R2_LO_HI)) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) f[u] = g[u] / (r2[u] * sqrt(r2[u]));
+    }
 }
 
 __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4 *tiles, double dt, int nsteps)
@@ -677,14 +695,40 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
         sr[lane] = pl.R[i];
         sact[lane] = st != INACTIVE;
     }
+    // what holds for the whole run: the exact cores' range of the masses, and
+    // the denominators of ah2 (running sums over the active bodies 1..lane)
+    const bool gok = !plw || __all(pair_g_ok_int(gm));
+    double etaj = GMcb;
+    if (plw) {
+        wave_sync();
+        if (isb)
+            for (int k = 1; k <= lane; k++)
+                if (sact[k]) etaj = etaj + sg[k - 1];
+    }
+    double hf = 0.0;  // this lane's body's ah0 factor at rh
+    auto ah0_factor = [&](double r2) __attribute__((always_inline)) { hf = gm * (1.0 / (r2 * sqrt(r2))); };
     // positions and ah0 factor of this lane's body into slot q
     auto publish = [&](int q) __attribute__((always_inline)) {
         if (!isb) return;
-        double r2 = dot3(rh[0], rh[1], rh[2], rh[0], rh[1], rh[2]);
         bx[q][lane] = rh[0];
         by[q][lane] = rh[1];
         bz[q][lane] = rh[2];
-        bf[q][lane] = gm * (1.0 / (r2 * sqrt(r2)));
+        bf[q][lane] = hf;
+    };
+    // the sum, from zero and in order, of the terms lo <= k < end (end per
+    // lane) of three LDS arrays.  Every lane passes over all of them, the reads
+    // ahead of the adds: a term past its end counts as +0.0, which changes no
+    // sum that starts at +0
+    auto sum_to = [&](const double *A, const double *B, const double *C, int lo, int end, double (&o)[3])
+                      __attribute__((always_inline)) {
+#pragma unroll 8
+        for (int k = lo; k < n; k++) {
+            const bool in = k < end;
+            const double ta = A[k], tb = B[k], tc = C[k];
+            o[0] = o[0] + (in ? ta : 0.0);
+            o[1] = o[1] + (in ? tb : 0.0);
+            o[2] = o[2] + (in ? tc : 0.0);
+        }
     };
     // ah of the massive bodies at rh / xj, added to ah (whm_kick_getacch_pl,
     // as whm_getacch_pl above)
@@ -697,7 +741,8 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
         ir3j = ir / r2j;
         wave_sync();
         if (isb) {
-            sf[lane] = gm * (1.0 / (r2 * sqrt(r2)));
+            ah0_factor(r2);
+            sf[lane] = hf;
             sx[lane] = rh[0];
             sy[lane] = rh[1];
             sz[lane] = rh[2];
@@ -720,40 +765,39 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
                     ah[d] = ah[d] + GMcb * (a1j - a1h);
                 }
             // ah2: the running sums over the active bodies 1..lane
-            double etaj = GMcb;
-            for (int k = 1; k <= lane; k++)
-                if (sact[k]) etaj = etaj + sg[k - 1];
             fac = ((gm * GMcb) * ir3j) / etaj;
-            su[lane] = fac * xj[0];
-            sv[lane] = fac * xj[1];
-            sw[lane] = fac * xj[2];
+            const bool act = st != INACTIVE;
+            su[lane] = act ? fac * xj[0] : 0.0;
+            sv[lane] = act ? fac * xj[1] : 0.0;
+            sw[lane] = act ? fac * xj[2] : 0.0;
         }
         wave_sync();
         if (!isb) return;
         if (lane >= 1 && st != INACTIVE) {
             double ah2o[3] = {0, 0, 0};
-            for (int k = 1; k <= lane; k++) {
-                if (!sact[k]) continue;
-                ah2o[0] = ah2o[0] + su[k];
-                ah2o[1] = ah2o[1] + sv[k];
-                ah2o[2] = ah2o[2] + sw[k];
-            }
+            sum_to(su, sv, sw, 1, lane + 1, ah2o);
             for (int d = 0; d < 3; d++) ah[d] = ah[d] + ah2o[d];
         }
         double ax = ah[0], ay = ah[1], az = ah[2];
-#pragma unroll 8
-        for (int u = 0; u < n; u++) {
-            if (u == lane) continue;
-            double rx = sx[u] - rh[0], ry = sy[u] - rh[1], rz = sz[u] - rh[2];
-            double rji2 = dot3(rx, ry, rz, rx, ry, rz);
-            if (a.lclose) {
-                double rs = sr[lane] + sr[u];
-                if (!(rji2 > rs * rs)) continue;
+        for (int u0 = 0; u0 < n; u0 += 4) {
+            double rx[4], ry[4], rz[4], r2[4], g[4], f[4];
+            bool use[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int q = min(u0 + u, n - 1);
+                rx[u] = sx[q] - rh[0], ry[u] = sy[q] - rh[1], rz[u] = sz[q] - rh[2];
+                r2[u] = dot3(rx[u], ry[u], rz[u], rx[u], ry[u], rz[u]);
+                g[u] = sg[q];
+                const double rs = sr[lane] + sr[q];
+                use[u] = u0 + u < n && q != lane && (!a.lclose || r2[u] > rs * rs);
             }
-            double f = gm_over_r3(sg[u], rji2, pair_g_ok(sg[u]));
-            ax = fma(f, rx, ax);
-            ay = fma(f, ry, ay);
-            az = fma(f, rz, az);
+            whm_factors(g, r2, use, gok, f);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                ax = use[u] ? fma(f[u], rx[u], ax) : ax;
+                ay = use[u] ? fma(f[u], ry[u], ay) : ay;
+                az = use[u] ? fma(f[u], rz[u], az) : az;
+            }
         }
         ah[0] = ax;
         ah[1] = ay;
@@ -775,10 +819,8 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
                 for (int d = 0; d < 3; d++) xj[d] = rh[d], vj[d] = vh[d];
                 if (lane > 0) {
                     double cx[3] = {0, 0, 0}, cv[3] = {0, 0, 0};
-                    for (int k = 0; k < lane; k++) {
-                        cx[0] = cx[0] + sx[k], cx[1] = cx[1] + sy[k], cx[2] = cx[2] + sz[k];
-                        cv[0] = cv[0] + su[k], cv[1] = cv[1] + sv[k], cv[2] = cv[2] + sw[k];
-                    }
+                    sum_to(sx, sy, sz, 0, lane, cx);
+                    sum_to(su, sv, sw, 0, lane, cv);
                     for (int d = 0; d < 3; d++) {
                         double cap = cx[d] / seta[lane - 1], capv = cv[d] / seta[lane - 1];
                         xj[d] = rh[d] - cap;
@@ -805,7 +847,7 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
                 for (int d = 0; d < 3; d++) vj[d] = vh[d];
             } else {
                 double cv[3] = {0, 0, 0};
-                for (int k = 0; k < lane; k++) cv[0] = cv[0] + su[k], cv[1] = cv[1] + sv[k], cv[2] = cv[2] + sw[k];
+                sum_to(su, sv, sw, 0, lane, cv);
                 for (int d = 0; d < 3; d++) vj[d] = vh[d] - cv[d] / seta[lane - 1];
             }
             if (st != INACTIVE) fl = drift_one(muj, xj[0], xj[1], xj[2], vj[0], vj[1], vj[2], dt);
@@ -821,28 +863,20 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
             su[lane] = (gm * xj[0]) / seta[lane];
             sv[lane] = (gm * xj[1]) / seta[lane];
             sw[lane] = (gm * xj[2]) / seta[lane];
+            sx[lane] = (gm * vj[0]) / seta[lane];
+            sy[lane] = (gm * vj[1]) / seta[lane];
+            sz[lane] = (gm * vj[2]) / seta[lane];
         }
         wave_sync();
         if (isb) {
-            double cx[3] = {0, 0, 0};
-            for (int k = 0; k < lane; k++) cx[0] = cx[0] + su[k], cx[1] = cx[1] + sv[k], cx[2] = cx[2] + sw[k];
+            double cx[3] = {0, 0, 0}, cv[3] = {0, 0, 0};
+            sum_to(su, sv, sw, 0, lane, cx);
+            sum_to(sx, sy, sz, 0, lane, cv);
             if (lane == 0) {
                 for (int d = 0; d < 3; d++) rh[d] = xj[d], vh[d] = vj[d];
             } else {
-                for (int d = 0; d < 3; d++) rh[d] = xj[d] + cx[d];
+                for (int d = 0; d < 3; d++) rh[d] = xj[d] + cx[d], vh[d] = vj[d] + cv[d];
             }
-        }
-        wave_sync();
-        if (isb) {
-            su[lane] = (gm * vj[0]) / seta[lane];
-            sv[lane] = (gm * vj[1]) / seta[lane];
-            sw[lane] = (gm * vj[2]) / seta[lane];
-        }
-        wave_sync();
-        if (isb && lane > 0) {
-            double cv[3] = {0, 0, 0};
-            for (int k = 0; k < lane; k++) cv[0] = cv[0] + su[k], cv[1] = cv[1] + sv[k], cv[2] = cv[2] + sw[k];
-            for (int d = 0; d < 3; d++) vh[d] = vj[d] + cv[d];
         }
         if (isb) ah[0] = ah[1] = ah[2] = 0.0;
         getacch();
@@ -868,6 +902,7 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
     }
     // kick with ah0 and the direct sum at the positions in slot q (as
     // k_whm_tp_ah0 / k_whm_tp_kick)
+    bool tgok = true;  // set below, once the bodies' masses are in LDS
     auto tp_kick = [&](int q, bool recompute) __attribute__((always_inline)) {
         if (!ist || tst != ACTIVE) return;
         if (recompute) {
@@ -879,14 +914,25 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
                 h0[2] = fma(-bf[q][u], bz[q][u], h0[2]);
             }
             double px = 0.0, py = 0.0, pz = 0.0;
-#pragma unroll 8
-            for (int u = 0; u < n; u++) {
-                double rx = trh[0] - bx[q][u], ry = trh[1] - by[q][u], rz = trh[2] - bz[q][u];
-                double rji2 = dot3(rx, ry, rz, rx, ry, rz);
-                double f = a.fast ? gm_over_r3_fast(sg[u], rji2) : gm_over_r3(sg[u], rji2, pair_g_ok(sg[u]));
-                px = fma(-f, rx, px);
-                py = fma(-f, ry, py);
-                pz = fma(-f, rz, pz);
+            for (int u0 = 0; u0 < n; u0 += 4) {
+                double rx[4], ry[4], rz[4], r2[4], g[4], f[4];
+                bool use[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int b = min(u0 + u, n - 1);
+                    rx[u] = trh[0] - bx[q][b], ry[u] = trh[1] - by[q][b], rz[u] = trh[2] - bz[q][b];
+                    r2[u] = dot3(rx[u], ry[u], rz[u], rx[u], ry[u], rz[u]);
+                    g[u] = sg[b];
+                    use[u] = u0 + u < n;
+                    if (a.fast) f[u] = gm_over_r3_fast(g[u], r2[u]);
+                }
+                if (!a.fast) whm_factors(g, r2, use, tgok, f);
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    px = use[u] ? fma(-f[u], rx[u], px) : px;
+                    py = use[u] ? fma(-f[u], ry[u], py) : py;
+                    pz = use[u] ? fma(-f[u], rz[u], pz) : pz;
+                }
             }
             tah[0] = (0.0 + h0[0]) + px;
             tah[1] = (0.0 + h0[1]) + py;
@@ -902,6 +948,7 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
         // prologue: the bodies' positions before step 0 (slot 0) and after
         // it (slot 1)
         if (n && nsteps > 0) {
+            ah0_factor(dot3(rh[0], rh[1], rh[2], rh[0], rh[1], rh[2]));
             publish(0);
             if (!pl_step(1) && lane == 0) sfail = 1;
         }
@@ -937,6 +984,7 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
         }
     } else {
         __syncthreads();
+        tgok = __all(lane >= n || pair_g_ok_int(sg[lane]));
         for (int k = 0; k < nsteps && !sfail; k++) {
             // the particles' step k: kick at the start positions (reusing the
             // last step's accelerations unless this is the first kick),
