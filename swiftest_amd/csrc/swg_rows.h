@@ -18,8 +18,8 @@
 // before, one lane per component of a body.  B = 16 (one fold wavefront, its
 // lanes holding x, y and z of the 16 bodies) gives four times the workgroups
 // of B = 64 (a fold wavefront per component, every lane of it in use): the
-// first is bound by the fold's chain of about 10 cycles a term, the second,
-// for systems that fill the chip either way, by FP64 issue.
+// first is bound by the fold, about 1 us a chunk of its chain and LDS reads, the
+// second, for systems that fill the chip either way, by FP64 issue.
 // Measured: 2000 bodies 32.6 us (64-body tiles with the partners staged in LDS
 // and read there for every term: 69), 10000 bodies 267 us (338), 32000 bodies
 // 2.0 ms (2.0); the leaf rows of 10007 bodies 267 us (one lane a body: 4466);

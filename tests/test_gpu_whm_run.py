@@ -74,22 +74,3 @@ def test_whole_step_launches_fast_pair_mode(monkeypatch):
     fused.run(300)
     stepwise.run(300)
     _equal(fused.state(), stepwise.state(), "fast")
-
-
-@pytest.mark.parametrize("lclose", [False, True])
-@pytest.mark.parametrize("npl", [2, 3, 4, 5, 7, 9, 63])
-def test_groups_of_four_bodies(npl, lclose):
-    """The pair groups' remainders, with a mass outside the exact cores' range
-    and, with radii, two bodies that overlap."""
-    d = ics.whm_solar(seed=90 + npl, npl=npl, ntp=5)
-    if lclose:
-        d.Gmass[-1] = 1e-180
-        if npl > 3:
-            d.pl_rh[2] = d.pl_rh[1] * (1.0 + 1e-6)
-            d.pl_vh[2] = d.pl_vh[1]
-            d.radius[1] = d.radius[2] = 1e-4
-    o = O.OracleSystem(O.WHM, d, 0.01, lclose=lclose)
-    g = S.GpuSystem(S.WHM, d, 0.01, lclose=lclose)
-    assert o.run(7) == 0
-    g.run(7)
-    _equal(o.state(), g.state(), (npl, lclose))
