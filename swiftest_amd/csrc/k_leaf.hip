@@ -612,16 +612,19 @@ __global__ void k_whm_h2j_all(WhmArgs a, int nsys)
 // Whole WHM steps in one launch (systems of at most WR_N massive bodies).
 // One workgroup of two wavefronts per tile: a system and up to 64 of its
 // test particles.  The first wavefront integrates the system's massive
-// bodies, one lane per body (every tile of a system computes the same values
-// from the same inputs; its first tile writes them back); the second
-// integrates the tile's particles, one lane each.  They run one step apart:
-// while the particles take step k, which needs the bodies' positions at the
-// start and at the end of step k, the bodies already take step k+1.  The
-// positions after each step pass through three LDS buffers; one workgroup
-// barrier per step.  Each sum over the bodies in order (the Jacobi maps'
-// prefixes, ah0, ah2) is formed by each lane from the terms the bodies' lanes
-// put in LDS, added in the order of whm_coord.f90 / whm_kick.f90, so every
-// value equals the one the per-step kernels above (and the oracle) produce.
+// bodies, one lane per body: every tile of a system computes the same values
+// from the same inputs, and the last of them to finish writes them back
+// (WhmDev::finished counts them).  A tile may start after another has ended,
+// when there are more tiles than the chip holds at once, and still has to load
+// the state the run begins with.  The second wavefront integrates the tile's
+// particles, one lane each.  They run one step apart: while the particles take
+// step k, which needs the bodies' positions at the start and at the end of
+// step k, the bodies already take step k+1.  The positions after each step pass
+// through three LDS buffers; one workgroup barrier per step.  Each sum over the
+// bodies in order (the Jacobi maps' prefixes, ah0, ah2) is formed by each lane
+// from the terms the bodies' lanes put in LDS, added in the order of
+// whm_coord.f90 / whm_kick.f90, so every value equals the one the per-step
+// kernels above (and the oracle) produce.
 // Bound: the latency of one step's chain on the bodies' wavefront (maps, drift,
 // accelerations).  Pairs are taken four at a time, their factors side by side,
 // the sums' terms are read ahead, and what holds for the whole run is formed
@@ -662,7 +665,6 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
     const int4 tl = tiles[blockIdx.x];
     const int s = tl.x, lane = threadIdx.x & 63;
     const bool plw = threadIdx.x < 64;  // the bodies' wavefront
-    const bool writer = tl.w != 0;
     const PlDev &pl = a.pl;
     const WhmDev &w = a.w;
     const int p0 = a.sy.pl_off[s], n = a.sy.pl_off[s + 1] - p0;
@@ -960,6 +962,14 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
             __syncthreads();
         }
         const int fail = sfail;
+        // the fence: this tile's loads come before its count
+        bool writer = true;
+        if (tl.w > 1) {
+            unsigned k = 0;
+            __threadfence();
+            if (lane == 0) k = atomicInc((unsigned *)&w.finished[s], (unsigned)tl.w - 1u);  // back to 0 after the last
+            writer = __builtin_amdgcn_readfirstlane(k) == (unsigned)tl.w - 1u;
+        }
         if (writer) {
             if (isb) {
                 pl.rh.x[i] = rh[0], pl.rh.y[i] = rh[1], pl.rh.z[i] = rh[2];
@@ -1026,7 +1036,8 @@ static WhmArgs whm_args(Ensemble &e)
 int Ensemble::whm_setup()
 {
     if (alloc_vec(whm.xj, npl) || alloc_vec(whm.vj, npl) || alloc_vec(whm.ah, npl) || alloc_vec(whm.tah, ntp) ||
-        own(&whm.eta, npl) || own(&whm.muj, npl) || own(&whm.ir3h, npl) || own(&whm.ir3j, npl))
+        own(&whm.eta, npl) || own(&whm.muj, npl) || own(&whm.ir3h, npl) || own(&whm.ir3j, npl) ||
+        own(&whm.finished, nsys))
         return SWG_ERR_HIP;
     // whm_util_set_mu_eta_pl (whm_util.f90:175-198), per system
     std::vector<double> eta(npl), muj(npl);
@@ -1048,9 +1059,9 @@ int Ensemble::whm_setup()
     for (double *p : {whm.tah.x, whm.tah.y, whm.tah.z})
         HIPCHK(copy_wait(stream, p, z.data(), ntp * sizeof(double), hipMemcpyHostToDevice));
     // tiles of the whole-step kernel: every system with at most WR_N massive
-    // bodies qualifies; each gets ceil(ntp/64) tiles (one if it has none),
-    // the first of which writes the massive bodies back.  SWG_WHM_STEPWISE=1
-    // keeps the per-step kernels.
+    // bodies qualifies; each gets ceil(ntp/64) tiles (one if it has none), and
+    // each tile knows how many they are.  SWG_WHM_STEPWISE=1 keeps the per-step
+    // kernels.
     whm_fused = true;
     for (int s = 0; s < nsys; s++) whm_fused = whm_fused && (h_pl_off[s + 1] - h_pl_off[s]) <= WR_N;
     const char *sw = getenv("SWG_WHM_STEPWISE");
@@ -1058,13 +1069,11 @@ int Ensemble::whm_setup()
     if (whm_fused) {
         std::vector<int4> t;
         for (int s = 0; s < nsys; s++) {
-            const int b = h_tp_off[s], e = h_tp_off[s + 1];
-            int k = 0;
-            do {
-                t.push_back(make_int4(s, b + 64 * k, std::min(b + 64 * (k + 1), e), k == 0));
-                k++;
-            } while (b + 64 * k < e);
+            const int b = h_tp_off[s], e = h_tp_off[s + 1], n = std::max(1, (e - b + 63) / 64);
+            for (int k = 0; k < n; k++) t.push_back(make_int4(s, b + 64 * k, std::min(b + 64 * (k + 1), e), n));
         }
+        const std::vector<int32_t> none(nsys, 0);
+        HIPCHK(copy_wait(stream, whm.finished, none.data(), nsys * sizeof(int32_t), hipMemcpyHostToDevice));
         HIPCHK(hipMalloc((void **)&d_tiles_whm, t.size() * sizeof(int4)));
         owned.push_back((void *)d_tiles_whm);
         HIPCHK(copy_wait(stream, d_tiles_whm, t.data(), t.size() * sizeof(int4), hipMemcpyHostToDevice));

@@ -20,6 +20,7 @@ struct WhmDev {
     Vec3p xj, vj, ah, tah;
     double *eta, *muj, *ir3h, *ir3j;
     int32_t *iflag;
+    int32_t *finished;  // tiles of each system that have ended the current launch (k_whm_run)
 };
 
 // Padding of a slot beyond the system it holds: inactive massive bodies
