@@ -661,7 +661,11 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
     __shared__ int sact[WR_N];
     // positions (and ah0 factors) of the bodies after j steps, in slot j % 3
     __shared__ double bx[3][WR_N], by[3][WR_N], bz[3][WR_N], bf[3][WR_N];
-    __shared__ int sfail;
+    // the step the run stops before: nsteps, or the step of a failed drift of
+    // the bodies.  The bodies' wavefront sets it while the particles still take
+    // the step before that one, so it says where to stop and not to stop now:
+    // both wavefronts leave the loop at the same step whenever they read it.
+    __shared__ int sstop;
     const int4 tl = tiles[blockIdx.x];
     const int s = tl.x, lane = threadIdx.x & 63;
     const bool plw = threadIdx.x < 64;  // the bodies' wavefront
@@ -670,7 +674,7 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
     const int p0 = a.sy.pl_off[s], n = a.sy.pl_off[s + 1] - p0;
     const double GMcb = a.sy.GMcb[s], dth = 0.5 * dt;
     const int lfirst0 = a.sy.lfirst[s];
-    if (threadIdx.x == 0) sfail = 0;
+    if (threadIdx.x == 0) sstop = nsteps;
 
     // ---- the bodies' wavefront: state in registers, one lane per body ----
     const bool isb = plw && lane < n;
@@ -952,16 +956,14 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
         if (n && nsteps > 0) {
             ah0_factor(dot3(rh[0], rh[1], rh[2], rh[0], rh[1], rh[2]));
             publish(0);
-            if (!pl_step(1) && lane == 0) sfail = 1;
+            if (!pl_step(1) && lane == 0) sstop = 0;
         }
         __syncthreads();
-        int done = 0;  // particle steps taken
-        for (int k = 0; k < nsteps && !sfail; k++) {
-            if (n && k + 1 < nsteps && !pl_step((k + 2) % 3) && lane == 0) sfail = 2;
-            done = k + 1;
+        for (int k = 0; k < sstop; k++) {
+            if (n && k + 1 < nsteps && !pl_step((k + 2) % 3) && lane == 0) sstop = k + 1;
             __syncthreads();
         }
-        const int fail = sfail;
+        const int stop = sstop;
         // the fence: this tile's loads come before its count
         bool writer = true;
         if (tl.w > 1) {
@@ -987,15 +989,15 @@ __global__ __launch_bounds__(128) void k_whm_run(WhmArgs a, TpDev tp, const int4
                 a.sy.lfirst[s] = lfirst;
                 // the first-kick flag of the last step begun: lfirst0 for
                 // step 0 (and for every step when no body clears lfirst)
-                const int last = fail == 1 ? 0 : (fail == 2 ? done : done - 1);
+                const int last = min(stop, nsteps - 1);
                 a.tlfirst[s] = (n == 0 || last == 0) ? lfirst0 : 0;
-                if (fail) a.sy.err[s] |= 2;
+                if (stop < nsteps) a.sy.err[s] |= 2;
             }
         }
     } else {
         __syncthreads();
         tgok = __all(lane >= n || pair_g_ok_int(sg[lane]));
-        for (int k = 0; k < nsteps && !sfail; k++) {
+        for (int k = 0; k < sstop; k++) {
             // the particles' step k: kick at the start positions (reusing the
             // last step's accelerations unless this is the first kick),
             // drift, kick at the end positions
