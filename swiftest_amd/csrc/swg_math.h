@@ -236,10 +236,15 @@ __host__ __device__ inline double cdiv(double x, double c, double r)
 // quotients use cdiv: each one feeds 1 - q, and a quotient too small to be
 // normal (|x| < 2^-1014) leaves 1 - q = 1 whichever way it rounds, so
 // c0..c3 equal the IEEE evaluation for every finite x.
+// An infinite argument (a velocity whose square overflows) stays infinite under
+// the quartering; the bound, above the 514 quarterings of the largest finite
+// double, ends its loop, and the drift fails on the results, which are not
+// finite.
+constexpr int STUMPFF_QUARTERS = 520;
 __host__ __device__ inline void stumpff(double x, double &c0, double &c1, double &c2, double &c3)
 {
     int n = 0;
-    while (fabs(x) >= 0.1) {
+    while (fabs(x) >= 0.1 && n < STUMPFF_QUARTERS) {
         n += 1;
         x = x / 4.0;
     }

@@ -7,7 +7,9 @@
 //    x**THIRD in 80-bit long double: the double nearest to powl's value,
 //    wherever powl's value is not within 2^-8 ulp of a rounding midpoint
 //    (there an 80-bit evaluation cannot decide the rounding); outside
-//    [2^-1000, 2^1000] it must equal pow(x, THIRD).
+//    [2^-1000, 2^1000] it must equal pow(x, THIRD);
+//  - swg::stumpff ends for every argument, the infinite ones included, whose
+//    results are not finite.
 // Prints "ok <count>" or the first mismatches.
 #include <cmath>
 #include <cstdint>
@@ -93,6 +95,12 @@ int main(int argc, char **argv)
         std::memcpy(&b, &g, 8);
         tot++;
         if (a != b && bad++ < 5) std::printf("mismatch pow_third(%a) = %a, pow %a\n", x, y, g);
+    }
+    for (double x : {1e300, -1e300, 1.7976931348623157e308, (double)INFINITY, -(double)INFINITY, (double)NAN}) {
+        double c0, c1, c2, c3;
+        swg::stumpff(x, c0, c1, c2, c3);
+        tot++;
+        if (!(std::fabs(x) < INFINITY) && std::isfinite(c2) && bad++ < 5) std::printf("stumpff(%a): finite c2 %a\n", x, c2);
     }
     if (skipped > n / 64) {
         std::printf("too many near-midpoint cases skipped: %ld\n", skipped);

@@ -61,3 +61,18 @@ def test_ensemble_of_degenerate_systems_equals_the_oracle(integ):
                 assert np.array_equal(so[key], sg[key][off_pl[k]:off_pl[k + 1]]), (blk, k, key)
             for key in ("tp_rh", "tp_vh", "tp_vb"):
                 assert np.array_equal(so[key], sg[key][off_tp[k]:off_tp[k + 1]]), (blk, k, key)
+
+
+@pytest.mark.parametrize("speed", [np.inf, -np.inf, 1e200, np.nan])
+def test_drift_fails_for_speeds_whose_square_overflows(speed):
+    """The body is flagged and stays where it is; its neighbours drift as alone."""
+    d = ics.whm_solar(seed=3, npl=1, ntp=70)
+    x, v = d.tp_rh.copy(), d.tp_vh.copy()
+    mask = np.ones(70, np.int32)
+    ax, av, af = S.swiftest_drift_all(d.GMcb, x, v, 70, 0.01, mask)
+    v[33] = (0.0, speed, 0.0)
+    bx, bv, bf = S.swiftest_drift_all(d.GMcb, x, v, 70, 0.01, mask)
+    rest = np.arange(70) != 33
+    assert np.array_equal(ax[rest], bx[rest]) and np.array_equal(av[rest], bv[rest])
+    assert not bf[rest].any() and bf[33] != 0
+    assert np.array_equal(bx[33], x[33]) and np.array_equal(bv[33], v[33], equal_nan=True)

@@ -10,7 +10,8 @@ shell factors of symba_kick.f90:150-200 and the encounter radii of
 symba_util.f90:245-267) with the powers evaluated at run time, and checks
 pow_third, the correctly rounded x**THIRD of the cubic first guess
 (swiftest_drift.f90:486-533), against 80-bit powl and on its exact cubes and
-out-of-range fallbacks.
+out-of-range fallbacks.  The Stumpff series' argument reduction ends for an
+infinite argument too.
 """
 import os
 import shutil
