@@ -27,6 +27,14 @@ static inline int cdiv(int64_t a, int b) { return (int)((a + b - 1) / b); }
         if (e_ != hipSuccess) return hipfail(e_, #x); \
     } while (0)
 
+// ordering of LDS accesses between the lanes of one wavefront
+__device__ inline void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------------------
 // leaf kernels (AoS in HBM, as the reference lays its (3,n) arrays out)
 // ---------------------------------------------------------------------------
@@ -145,10 +153,10 @@ __global__ __launch_bounds__(256) void k_flat_fold(int npl, const uint32_t *ent,
         row[4 * l + 1] = v.y;
         row[4 * l + 2] = v.z;
         row[4 * l + 3] = v.w;
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
 #pragma unroll
         for (int q = 0; q < 16; q++) h = fma(row[4 * q + 3], row[4 * q + comp], h);
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
     }
     if (on && l < 3) sum[3 * s + l] = h;
 }
@@ -631,14 +639,6 @@ __global__ void k_whm_h2j_all(WhmArgs a, int nsys)
 // once: 8 bodies and 1000 particles 9.5 -> 7.3 us a step.
 // ---------------------------------------------------------------------------
 constexpr int WR_N = 64;
-
-// ordering of LDS accesses between the lanes of one wavefront
-__device__ inline void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // gm_over_r3 of four pairs, side by side; use: the pair's factor is needed
 __device__ inline void whm_factors(const double (&g)[4], const double (&r2)[4], const bool (&use)[4], bool gok,
