@@ -455,7 +455,7 @@ struct LdsSet {
     union {
         KTerm kt[L_KC];
         struct {
-            KTerm kt_wave[64];            // wave mode's terms (kt[0, 64))
+            KTerm kt_wave[65];            // wave mode's terms (kt[0, 64)), and one that adds nothing
             double shr[MAXLEV + 1][64];  // and its entries' shell radii, by level from the one it started at
         };
         int16_t posu[L_NE + L_NET];  // while the list is built
@@ -1112,7 +1112,10 @@ __device__ inline void wave_store(LdsSet &S, int k, const WaveLane &W)
 }
 
 // The sums of the terms [u, hi), in order (fold_terms for few terms per body):
-// four are read at once, the ones past the end as zeros.
+// four are read at once, and in place of the ones past the end, which are
+// another body's, the term that adds nothing (its product is -0, and s + (-0) = s
+// for every s).
+constexpr int WAVE_NO_TERM = 64;
 __device__ inline void wave_fold(const KTerm *kt, int u, int hi, KCache &c)
 {
     c.p = c.m = make_double3(0.0, 0.0, 0.0);
@@ -1120,18 +1123,16 @@ __device__ inline void wave_fold(const KTerm *kt, int u, int hi, KCache &c)
     do {
         KTerm a[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) a[q] = kt[min(u + q, 63)];
+        for (int q = 0; q < 4; q++) a[q] = kt[u + q < hi ? u + q : WAVE_NO_TERM];
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const bool on = u + q < hi;
-            const double fp = on ? a[q].fp : 0.0, fm = on ? a[q].fm : 0.0;
-            c.p.x = fma(fp, a[q].dx, c.p.x);
-            c.p.y = fma(fp, a[q].dy, c.p.y);
-            c.p.z = fma(fp, a[q].dz, c.p.z);
-            c.m.x = fma(fm, a[q].dx, c.m.x);
-            c.m.y = fma(fm, a[q].dy, c.m.y);
-            c.m.z = fma(fm, a[q].dz, c.m.z);
-            c.fl |= on ? a[q].fl : 0;
+            c.p.x = fma(a[q].fp, a[q].dx, c.p.x);
+            c.p.y = fma(a[q].fp, a[q].dy, c.p.y);
+            c.p.z = fma(a[q].fp, a[q].dz, c.p.z);
+            c.m.x = fma(a[q].fm, a[q].dx, c.m.x);
+            c.m.y = fma(a[q].fm, a[q].dy, c.m.y);
+            c.m.z = fma(a[q].fm, a[q].dz, c.m.z);
+            c.fl |= a[q].fl;
         }
         u += 4;
     } while (u < hi);
@@ -1203,6 +1204,12 @@ __device__ __attribute__((noinline)) int2 wave_recursion(int nE, int dw, double 
     const bool tps = S.wnT > 0;
     const int dmax = min(S.dmax, MAXLEV);
     if (w0) wave_load(S, nE, lane, W);
+    if (threadIdx.x == 0) {
+        KTerm &z = S.kt[WAVE_NO_TERM];
+        z.dx = z.dy = z.dz = -0.0;
+        z.fp = z.fm = 0.0;
+        z.fl = 0;
+    }
     int dl = -1;  // the level the next five belong to
     double dtl = 0.0, dth = 0.0, rsh = 0.0, sqp = 0.0, sqm = 0.0;
     // shell-kick sums of level d for the body of this lane, into c
