@@ -1237,10 +1237,11 @@ __device__ __attribute__((noinline)) int2 wave_recursion(int nE, int dw, double 
     for (;;) {
         if (dl != d) {
             dl = d;
-            dtl = S.dtl[d];
-            rsh = S.rsh[d + 1];
-            sqp = S.ssq[d + 1];
-            sqm = S.ssq[d];
+            const int e = min(d, MAXLEV);  // one past the level stack stops below
+            dtl = S.dtl[e];
+            rsh = S.rsh[e + 1];
+            sqp = S.ssq[e + 1];
+            sqm = S.ssq[e];
             dth = 0.5 * dtl;
         }
         if (!resume) {
