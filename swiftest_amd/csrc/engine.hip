@@ -948,7 +948,8 @@ uint64_t Ensemble::graph_key() const
                           pt.colstart, pt.status, d_arena,   (const void *)(intptr_t)ntiles_pl,
                           (const void *)(intptr_t)ntiles_tp, (const void *)(intptr_t)tune.kick_pl_block,
                           (const void *)(intptr_t)tune.kick_tp_block, (const void *)(intptr_t)tune.pair_fast,
-                          (const void *)(intptr_t)tune.kick_pl_split, (const void *)(intptr_t)tune.kick_pl_eval};
+                          (const void *)(intptr_t)tune.kick_pl_split, (const void *)(intptr_t)tune.kick_pl_eval,
+                          (const void *)(intptr_t)tune.any_tiny};
     uint64_t h = 1469598103934665603ull;
     for (const void *p : ptrs) {
         h ^= (uint64_t)(uintptr_t)p;
