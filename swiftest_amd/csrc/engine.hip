@@ -252,7 +252,7 @@ int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const in
         own(&sy.ptbeg, 3 * nsys) || own(&sy.ptend, 3 * nsys) || own(&sy.lfirst, nsys) || own(&sy.enc_pp, nsys) ||
         own(&sy.enc_pt, nsys) || own(&sy.flag_pp, nsys) || own(&sy.flag_pt, nsys) || own(&sy.err, nsys) ||
         own(&sy.frozen, nsys) || own(&d_active, nsys) || own(&d_any, 4) || own(&d_total, 4) || own(&d_pt_run, nsys) ||
-        own(&sy.nplm, nsys) || own(&d_cb_pl, nsys + 1) || own(&d_cb_tp, nsys + 1))
+        own(&sy.nplm, nsys) || own(&sy.nreal, nsys) || own(&d_cb_pl, nsys + 1) || own(&d_cb_tp, nsys + 1))
         return SWG_ERR_HIP;
     hipStream_t st = stream;
     {
@@ -315,6 +315,7 @@ int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const in
         }
         HIPCHK(put(pl.tiny, tiny.data(), npl * sizeof(int32_t)));
         HIPCHK(put(sy.nplm, nplm.data(), nsys * sizeof(int32_t)));
+        HIPCHK(put(sy.nreal, h_nreal_pl.data(), nsys * sizeof(int32_t)));
         tune.any_tiny = any_tiny;
     }
 
@@ -1426,9 +1427,9 @@ int Ensemble::load(int s, int npl_new, int ntp_new, double GMcb_new, const doubl
             }
         }
         if (cap_pl) HIPCHK(put(pl.tiny + p0, tiny.data(), cap_pl * sizeof(int32_t)));
-        // the padding sits after the system's own bodies: as partners of
-        // the fully interacting rows they add exact zeros
+        const int32_t n = npl_new;
         HIPCHK(put(sy.nplm + s, &m, sizeof m));
+        HIPCHK(put(sy.nreal + s, &n, sizeof n));
         if (m < npl_new) {
             any_tiny = true;
             tune.any_tiny = 1;

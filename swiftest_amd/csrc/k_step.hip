@@ -434,7 +434,10 @@ __global__ __launch_bounds__((RowsLds<B, KE, A>::THREADS), (RowsLds<B, KE, A>::W
     __shared__ RowsLds<B, KE, A> S;
     __shared__ double hpart[2][3][B];
     const Tile tl = tiles[blockIdx.x];
-    const int p0 = sy.pl_off[tl.s], n = sy.pl_off[tl.s + 1] - p0;
+    const int p0 = sy.pl_off[tl.s];
+    // a slot's padding adds exact zeros to rows, but is not among the bodies
+    // whose number chooses the branch
+    const int n = TINY ? sy.nreal[tl.s] : sy.pl_off[tl.s + 1] - p0;
     const int nm = TINY ? sy.nplm[tl.s] : n;
     const bool tri = TINY && n - nm > nm;
     const int lane = (int)(threadIdx.x & 63u), w = (int)(threadIdx.x >> 6);

@@ -834,6 +834,7 @@ int Ensemble::upload_merged(const void *hs, const std::vector<char> &hit, const 
     MCHK(hipMemcpyAsync(sy.cbvb, cbvb, 3 * nsys * sizeof(double), hipMemcpyHostToDevice, st));
     MCHK(hipMemcpyAsync(sy.pl_off, h_pl_off.data(), (nsys + 1) * sizeof(int32_t), hipMemcpyHostToDevice, st));
     MCHK(hipMemcpyAsync(sy.nplm, h_nplm.data(), nsys * sizeof(int32_t), hipMemcpyHostToDevice, st));
+    MCHK(hipMemcpyAsync(sy.nreal, h_nreal_pl.data(), nsys * sizeof(int32_t), hipMemcpyHostToDevice, st));
     // bit-matrix layout of the next step's detection and its column blocks
     std::vector<int64_t> woff(nsys);
     std::vector<int32_t> nb(nsys), cb(nsys + 1, 0);

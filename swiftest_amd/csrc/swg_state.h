@@ -47,6 +47,7 @@ struct SysDev {
     int32_t *err;                 // error bits: 1 collision, 2 pl drift failure
     int32_t *frozen;              // 1 = system left out of the steps (its state is kept as is)
     int32_t *nplm;                // fully interacting massive bodies (the first nplm of the system); may be NULL
+    int32_t *nreal;               // massive bodies without a slot's padding, which follows them
 };
 
 // A (pl, pl) or (pl, tp) encounter list with its bit matrix and adjacency.

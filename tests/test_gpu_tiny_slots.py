@@ -1,6 +1,7 @@
 """Semi-interacting bodies (GMTINY) in systems that are loaded anew, against the
 oracle's run of each alone, bit for bit: the first such bodies of an ensemble,
-after steps that were captured without any."""
+after steps that were captured without any, and slots with room to spare, whose
+padding must not count among them."""
 import numpy as np
 import pytest
 
@@ -39,3 +40,21 @@ def test_first_semi_interacting_bodies_after_captured_steps():
     g.use_graphs(True)
     _run_slot(g, heavy, "heavy")
     _run_slot(g, mixed, "mixed")
+
+
+@pytest.mark.parametrize("cap,n,mlo", [(96, 60, 3e-4), (300, 33, 6e-4), (200, 90, 1e-5)])
+@pytest.mark.parametrize("mode", [S.PAIR_EXACT, S.PAIR_FAST])
+def test_padding_does_not_count_as_semi_interacting(cap, n, mlo, mode):
+    """The accelerations themselves: a velocity hides the order of a sum."""
+    print(f"gmtiny slot of {cap} with {n}, mode {mode}", flush=True)
+    g = S.GpuSystem.slots(S.SYMBA, [cap], [10], 0.005, lclose=False, gmtiny=GT, pair_mode=mode)
+    d = _disk(62 + n, n, mlo)
+    tight = S.GpuSystem(S.SYMBA, d, 0.005, lclose=False, gmtiny=GT, pair_mode=mode)
+    g.load(0, d)
+    a, b = g.accel()[0][:n], tight.accel()[0]
+    assert np.array_equal(a, b)
+    if mode == S.PAIR_EXACT:
+        k = np.argsort(-d.Gmass, kind="stable")
+        nplm = int((d.Gmass >= GT).sum())
+        assert 0 < nplm < n
+        assert np.array_equal(a, O.accel_plpl(d.pl_rh[k], d.Gmass[k], d.radius[k], np.zeros((n, 3)), nplm=nplm))
