@@ -389,8 +389,8 @@ int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const in
     } else {
         launch_snapshot(st, pl, tp, sy, nsys, npl, 0);
         launch_init_tp_vb(st, tp, sy, ntp);
-        launch_reset_levels(st, pl, tp, sy, d_sub_stats, npl, ntp, nsys);
     }
+    launch_reset_levels(st, pl, tp, sy, d_sub_stats, npl, ntp, nsys);  // WHM steps use none of these but the counters
     HIPCHK(hipStreamSynchronize(st));
     HIPCHK(hipGetLastError());
     st_.max_depth = -1;

@@ -43,7 +43,7 @@ __global__ void k_reset_levels(PlDev pl, TpDev tp, SysDev sy, int32_t *sub_stats
         sy.enc_pp[i] = 0;
         sy.enc_pt[i] = 0;
     }
-    if (sub_stats && i < 4) sub_stats[i] = 0;
+    if (sub_stats && i < 4) sub_stats[i] = i == 1 ? -1 : 0;  // [1]: the deepest level, -1 = none
     if (i < npl) {
         pl.levelg[i] = -1;
         pl.levelm[i] = -1;

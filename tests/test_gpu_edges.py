@@ -76,3 +76,21 @@ def test_drift_fails_for_speeds_whose_square_overflows(speed):
     assert np.array_equal(ax[rest], bx[rest]) and np.array_equal(av[rest], bv[rest])
     assert not bf[rest].any() and bf[33] != 0
     assert np.array_equal(bx[33], x[33]) and np.array_equal(bv[33], v[33], equal_nan=True)
+
+
+def test_counters_without_recursion():
+    """No substeps and depth -1 in WHM, HELIO and a SyMBA step without
+    encounters, whatever the memory held before: systems that recursed give
+    theirs back first."""
+    d = compact_disk(seed=5, npl=60, ntp=20)
+    for _ in range(4):
+        g = S.GpuSystem(S.SYMBA, d, 0.005, lclose=False)
+        g.run(2)
+        assert g.stats()["nsubsteps"] > 0
+        del g
+        for integ, n, m in ((S.WHM, 8, 20), (S.HELIO, 8, 20), (S.SYMBA, 1, 0)):
+            w = S.GpuSystem(integ, ics.whm_solar(seed=6, npl=n, ntp=m), 0.005)
+            w.run(2)
+            s = w.stats()
+            assert (s["nsubsteps"], s["max_depth"], s["nplpl_enc"], s["npltp_enc"]) == (0, -1, 0, 0)
+            del w
