@@ -160,19 +160,23 @@ int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const in
     tune.pair_fast = p.pair_mode == SWG_PAIR_FAST;
     nsys = ns;
     if (const char *e = getenv("SWG_KICK_PL_EVAL")) {
-        // exact-mode massive-body kernel before any autotuning: 0 one lane
-        // per body, 4 / 8 evaluating wavefronts per 16- / 64-body tile (2: as 4)
+        // exact-mode massive-body kernel before any autotuning
         const int k = atoi(e);
-        if (k == 0 || k == 2 || k == 4 || k == 8) tune.kick_pl_eval = k;
+        if (k == KPL_LANES || k == KPL_BODIES || k == KPL_ROWS_SMALL || k == KPL_ROWS_LARGE) tune.kick_pl_eval = k;
     } else {
         // with fewer than two wavefronts per SIMD in the one-lane-per-body
         // kernel, the terms go to several wavefronts per tile instead
-        int64_t npl_all = 0, large = 0;
+        int64_t npl_all = 0, large = 0, tiles = 0;
         for (int s = 0; s < ns; s++) {
-            npl_all += npl_s[s] > 0 ? npl_s[s] : 0;
-            large += npl_s[s] > 0 ? npl_s[s] / RW_LARGE : 0;
+            const int n = std::max(npl_s[s], 0);
+            npl_all += n;
+            large += n / RW_LARGE;
+            tiles += (n + 63) / 64;
         }
-        if ((npl_all + 63) / 64 < 2048) tune.kick_pl_eval = large < RW_LARGE_TILES ? 4 : 8;
+        if ((npl_all + 63) / 64 < 2048) {
+            const bool shorts = npl_all > (int64_t)KPLB_NPL_MIN * ns && npl_all <= (int64_t)KPLB_NPL * ns;
+            tune.kick_pl_eval = shorts && tiles >= KPLB_TILES ? KPL_BODIES : large < RW_LARGE_TILES ? KPL_ROWS_SMALL : KPL_ROWS_LARGE;
+        }
     }
     h_pl_off.assign(nsys + 1, 0);
     h_tp_off.assign(nsys + 1, 0);
@@ -1590,16 +1594,16 @@ int Ensemble::autotune(int reps, int32_t *pl_block, int32_t *tp_block)
         return 0;
     }
     // exact mode: the pl-tp tile size, and for the massive bodies one lane
-    // per body with 64, 128 or 256-body tiles, or 16- or 64-body tiles
-    // shared by 4 or 8 evaluating wavefronts (reported as -4, -8)
-    const int evals[2] = {4, 8};
+    // per body with 64, 128 or 256-body tiles, or tiles shared by several
+    // wavefronts (reported as -2, -4, -8: KickPl)
+    const int evals[3] = {KPL_BODIES, KPL_ROWS_SMALL, KPL_ROWS_LARGE};
     double best_tp = 1e300, best_pl = 1e300;
     int btp = tune.kick_tp_block, bpl = tune.kick_pl_block, bev = tune.kick_pl_eval;
-    for (int k = 0; k < 5; k++) {
+    for (int k = 0; k < 6; k++) {
         if (k < 3) {
             tune.kick_tp_block = cand[k];
             tune.kick_pl_block = cand[k];
-            tune.kick_pl_eval = 0;
+            tune.kick_pl_eval = KPL_LANES;
         } else {
             tune.kick_pl_eval = evals[k - 3];
         }

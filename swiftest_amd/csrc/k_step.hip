@@ -513,6 +513,178 @@ __global__ __launch_bounds__((RowsLds<B, KE, A>::THREADS), (RowsLds<B, KE, A>::W
 }
 
 // ---------------------------------------------------------------------------
+// The same with one body per lane, for ensembles of many short systems: a tile
+// of 64 bodies, eight evaluating wavefronts that each form the factors of their
+// eight partners of a 64-partner chunk for all 64 bodies (the exact cores,
+// grouped and branch-free as in k_kick_pl) into LDS, a zero where a term is not
+// taken, and three that fold the chunk before in j order, one component each.
+// The partners are staged in LDS a chunk ahead.  A short system's workgroup
+// spends most of its time on starting up and on the chunk that holds the tile
+// itself, where a body's zero separation from itself sends whole groups of terms
+// through the IEEE operations in k_kick_pl_rows and none here.
+// Measured, this kernel / k_kick_pl_rows with 64 and with 16 bodies a tile, us:
+// 512 systems of 128 bodies 22 / 32 / 43, 1024 of 4 to 512 89 / 102 / 116, 128
+// of 512 67 / 70 / 98, 64 of 1024 128 / 123 / 171, one of 2000 67 / - / 30.
+// ---------------------------------------------------------------------------
+constexpr int KPLS_C = 64;  // partners per chunk
+constexpr int KPLS_KE = 8;  // evaluating wavefronts
+
+__global__ __launch_bounds__(64 * (KPLS_KE + 3)) void k_kick_pl_split(PlDev pl, SysDev sy, ListDev pp, const Tile *tiles,
+                                                                     double dt, int lbeg, int use_radius, int do_pairs)
+{
+    constexpr int KE = KPLS_KE;
+    static_assert(KPLS_C % (4 * KE) == 0, "each evaluation wavefront takes whole groups of four partners");
+    static_assert(KPLS_C == 64, "one partner per lane when a chunk is staged");
+    __shared__ double facb[2][KPLS_C][64];
+    __shared__ double hpart[2][3][64];
+    __shared__ double fsum[3][64];  // each component's fold
+    // the partners of chunk c (x, y, z, Gm, R) in slot c % 3: the chunk being
+    // folded, the one being evaluated and the next one
+    __shared__ double pj[3][5][KPLS_C];
+    const Tile tl = tiles[blockIdx.x];
+    const int p0 = sy.pl_off[tl.s], p1 = sy.pl_off[tl.s + 1];
+    const int lane = (int)(threadIdx.x & 63u);
+    // wavefronts 0..KE-1 evaluate; KE, KE+1, KE+2 fold the x, y, z sums
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int i = tl.b0 + lane;
+    const bool valid = i < tl.b1;
+    double xi = 0.0, yi = 0.0, zi = 0.0, Ri = 0.0;
+    if (valid) {
+        xi = pl.rh.x[i];
+        yi = pl.rh.y[i];
+        zi = pl.rh.z[i];
+        Ri = pl.R[i];
+    }
+    const int n = p1 - p0, nch = (n + KPLS_C - 1) / KPLS_C;
+    constexpr int PER = KPLS_C / KE;
+    // staging of chunk c by the first wavefront, one partner per lane
+    auto stage = [&](int c) {
+        const int jt = p0 + c * KPLS_C, jn = min(KPLS_C, p1 - jt);
+        if (lane < jn) {
+            const int j = jt + lane;
+            double(*d)[KPLS_C] = pj[c % 3];
+            d[0][lane] = pl.rh.x[j];
+            d[1][lane] = pl.rh.y[j];
+            d[2][lane] = pl.rh.z[j];
+            d[3][lane] = pl.Gm[j];
+            d[4][lane] = pl.R[j];
+        }
+    };
+    // evaluation of chunk c into buffer c & 1 (wavefronts 0 .. KE-1)
+    auto evaluate = [&](int c) {
+        const int jt = p0 + c * KPLS_C, jn = min(KPLS_C, p1 - jt);
+        const double(*d)[KPLS_C] = pj[c % 3];
+        // every mass of the chunk inside the exact cores' range: one column per lane
+        const bool gok_lane = lane >= jn || pair_g_ok(d[3][lane]);
+        const bool tile_gok = __all(gok_lane);
+        double(*fb)[64] = facb[c & 1];
+        for (int q0 = w * PER; q0 < (w + 1) * PER; q0 += 4) {
+            double r2[4], fac[4], rx[4], ry[4], rz[4];
+            bool take[4], need[4];
+            bool any_need = false;
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int q = q0 + u;
+                const int qq = min(q, jn - 1);  // in range; a column past the end is not taken
+                rx[u] = d[0][qq] - xi;
+                ry[u] = d[1][qq] - yi;
+                rz[u] = d[2][qq] - zi;
+                r2[u] = dot3(rx[u], ry[u], rz[u], rx[u], ry[u], rz[u]);
+                const double rs = Ri + d[4][qq];
+                take[u] = (q < jn) & (jt + q != i) & (!use_radius | (r2[u] > rs * rs));
+                fac[u] = div_core(d[3][qq], r2[u] * sqrt_core(r2[u]));
+                need[u] = take[u] & !(tile_gok & (r2[u] >= PAIR_R2_LO) & (r2[u] <= PAIR_R2_HI));
+                any_need = any_need | need[u];
+            }
+            if (__ballot(any_need)) {
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    if (need[u]) fac[u] = d[3][min(q0 + u, jn - 1)] / (r2[u] * sqrt(r2[u]));
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) fb[q0 + u][lane] = take[u] ? fac[u] : 0.0;
+        }
+    };
+    double acc = 0.0;  // a fold wavefront's component sum
+    const int comp = w - KE;
+    const double ci = comp == 0 ? xi : (comp == 1 ? yi : zi);
+    if (w == 0) {
+        if (nch > 0) stage(0);
+        if (nch > 1) stage(1);
+    }
+    __syncthreads();
+    if (w < KE && nch > 0) evaluate(0);
+    __syncthreads();
+    for (int c = 0; c < nch; c++) {
+        if (w < KE) {
+            if (c + 1 < nch) evaluate(c + 1);
+            if (w == 0 && c + 2 < nch) stage(c + 2);
+        } else {
+            // fold chunk c in j order, one component per wavefront
+            const int jt = p0 + c * KPLS_C, jn = min(KPLS_C, p1 - jt);
+            const double(*fb)[64] = facb[c & 1];
+            const double *dc = pj[c % 3][comp];
+            for (int q = 0; q < jn; q++) acc = fma(fb[q][lane], dc[q] - ci, acc);
+        }
+        __syncthreads();
+    }
+    if (w >= KE) fsum[comp][lane] = acc;
+    if (do_pairs && w < 2 && valid) {
+        // w = 0: ahj over pairs (p, i), p < i; w = 1: ahi over pairs (i, j)
+        double hx = 0.0, hy = 0.0, hz = 0.0;
+        if (w == 0) {
+            const int64_t c0 = pp.colstart[i], c1 = c0 + pp.colcnt[i];
+            for (int64_t c = c0; c < c1; c++) {
+                const int p = pp.i1[pp.col[c]];
+                const double rx = xi - pl.rh.x[p], ry = yi - pl.rh.y[p], rz = zi - pl.rh.z[p];
+                const double rji2 = dot3(rx, ry, rz, rx, ry, rz);
+                const double rs = pl.R[p] + Ri;
+                if (rji2 > rs * rs) {
+                    const double fac = pl.Gm[p] * (1.0 / (rji2 * sqrt(rji2)));
+                    hx = fma(-fac, rx, hx);
+                    hy = fma(-fac, ry, hy);
+                    hz = fma(-fac, rz, hz);
+                }
+            }
+        } else {
+            const int64_t r0 = pp.rowstart[i], r1 = r0 + pp.rowcnt[i];
+            for (int64_t k = r0; k < r1; k++) {
+                const int q = pp.i2[k];
+                const double rx = pl.rh.x[q] - xi, ry = pl.rh.y[q] - yi, rz = pl.rh.z[q] - zi;
+                const double rji2 = dot3(rx, ry, rz, rx, ry, rz);
+                const double rs = Ri + pl.R[q];
+                if (rji2 > rs * rs) {
+                    const double fac = pl.Gm[q] * (1.0 / (rji2 * sqrt(rji2)));
+                    hx = fma(fac, rx, hx);
+                    hy = fma(fac, ry, hy);
+                    hz = fma(fac, rz, hz);
+                }
+            }
+        }
+        hpart[w][0][lane] = hx;
+        hpart[w][1][lane] = hy;
+        hpart[w][2][lane] = hz;
+    }
+    __syncthreads();
+    if (w != KE || !valid) return;
+    double ax = fsum[0][lane], ay = fsum[1][lane], az = fsum[2][lane];
+    if (do_pairs) {
+        ax = ax - ((0.0 + hpart[1][0][lane]) + hpart[0][0][lane]);
+        ay = ay - ((0.0 + hpart[1][1][lane]) + hpart[0][1][lane]);
+        az = az - ((0.0 + hpart[1][2][lane]) + hpart[0][2][lane]);
+    }
+    Vec3p rb = lbeg ? pl.rbeg : pl.rend;
+    rb.x[i] = xi;
+    rb.y[i] = yi;
+    rb.z[i] = zi;
+    if (pl_active(pl, i)) {
+        pl.vb.x[i] = fma(ax, dt, pl.vb.x[i]);
+        pl.vb.y[i] = fma(ay, dt, pl.vb.y[i]);
+        pl.vb.z[i] = fma(az, dt, pl.vb.z[i]);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Fast pair mode (SWG_PAIR_FAST): the same sums in the same j order, with the
 // pair factor from the hardware reciprocal square root (gm_over_r3_fast,
 // within a few ulp of the IEEE factor).  The partners' positions, masses and
@@ -1083,7 +1255,9 @@ void launch_kick_pl(hipStream_t st, const Tuning &tu, PlDev pl, SysDev sy, ListD
         return;
     }
     if (tu.kick_pl_eval) {
-        if (tu.kick_pl_eval == 8)
+        if (tu.kick_pl_eval == KPL_BODIES)
+            k_kick_pl_split<<<ntiles, 64 * (KPLS_KE + 3), 0, st>>>(pl, sy, pp, tiles, dt, lbeg, use_radius, do_pairs);
+        else if (tu.kick_pl_eval == KPL_ROWS_LARGE)
             k_kick_pl_rows<RW_LARGE, 8, 1, false, false><<<ntiles, RowsLds<RW_LARGE, 8>::THREADS, 0, st>>>(
                 pl, sy, pp, tiles, dt, lbeg, use_radius, do_pairs);
         else if (ntiles <= RW_FEW)

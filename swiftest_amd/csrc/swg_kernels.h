@@ -32,13 +32,20 @@ struct Tuning {
     int kick_tp_block = 256;
     int pair_fast = 0;         // 1: pair factors from the reciprocal square root (SWG_PAIR_FAST)
     int kick_pl_split = 8;     // fast mode: wavefronts sharing one 64-body tile's rows (1, 2, 4, 8, 16)
-    int kick_pl_eval = 0;      // exact mode: 0 one lane per body (k_kick_pl), else k_kick_pl_rows with that
-                               // many evaluating wavefronts: 4 for 16-body tiles, 8 for 64-body tiles
+    int kick_pl_eval = 0;      // exact mode: the massive-body kernel, one of KickPl
     int any_tiny = 0;          // some system has semi-interacting bodies: k_kick_pl_rows, 16-body tiles
     // bodies per massive-body tile of the kernel launch_kick_pl takes
     int pl_tile() const;
 };
-// bodies per massive-body tile of the fast pair kernel
+// the exact massive-body kernels (SWG_KICK_PL_EVAL, and negated as the
+// autotuner reports them)
+enum KickPl {
+    KPL_LANES = 0,       // k_kick_pl, one lane per body, kick_pl_block bodies a tile
+    KPL_BODIES = 2,      // k_kick_pl_split, 64-body tiles, eight evaluating wavefronts with one body per lane
+    KPL_ROWS_SMALL = 4,  // k_kick_pl_rows, 16-body tiles, four evaluating wavefronts with one partner per lane
+    KPL_ROWS_LARGE = 8,  // k_kick_pl_rows, 64-body tiles, eight such wavefronts
+};
+// bodies per massive-body tile of the fast pair kernel and of k_kick_pl_split
 constexpr int KPL_FAST_TILE = 64;
 
 // the two tile sizes of k_kick_pl_rows and of the leaf rows
@@ -47,6 +54,13 @@ constexpr int RW_SMALL = 16, RW_LARGE = 64;
 // 16 / 64 bodies a tile: 10000 bodies 267 / 320 us, 13000 bodies 450 / 405 us,
 // 32000 bodies 2.7 / 2.0 ms).
 constexpr int RW_LARGE_TILES = 192;
+// One body per lane (KPL_BODIES) for systems of up to 512 bodies on average
+// with at least one 64-body tile per compute unit, and more than 16 bodies
+// (measured, KPL_BODIES / the better of the rows, us: 256 systems of 64 bodies
+// 6.3 / 8.6, 128 of 64 6.1 / 6.6, 64 of 64 6.1 / 4.7; 512 of 32 7.8 / 9.9, 1024
+// of 16 12.1 / 9.6; 64 of 256 13.1 / 14.4, 16 of 256 12.2 / 7.3; 64 of 512 36.6
+// / 40.1, 64 of 768 75.6 / 76.3, 64 of 1024 127.5 / 122.9).
+constexpr int KPLB_TILES = 256, KPLB_NPL = 512, KPLB_NPL_MIN = 16;
 // Up to one 16-body tile per compute unit the fold takes the registers to read
 // two sets of terms ahead (2000 bodies 32.6 us, 36.2 one set ahead); from two
 // tiles on the other wavefronts fill the waits, and the registers cost the third
@@ -57,7 +71,7 @@ inline int Tuning::pl_tile() const
 {
     if (any_tiny) return RW_SMALL;
     if (pair_fast) return KPL_FAST_TILE;
-    return kick_pl_eval == 0 ? kick_pl_block : kick_pl_eval == 8 ? RW_LARGE : RW_SMALL;
+    return kick_pl_eval == KPL_LANES ? kick_pl_block : kick_pl_eval == KPL_ROWS_SMALL ? RW_SMALL : 64;
 }
 
 // ---- step kernels (k_step.hip) ----

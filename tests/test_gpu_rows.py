@@ -116,3 +116,25 @@ def test_particles_at_tile_edges(npl, ntp):
     # each factor within 8 ulp of the exact mode's, then npl roundings of partial
     # sums no larger than the sum of the terms' sizes, on both sides
     assert (np.abs(fast - ref)[keep] <= 2 * (npl + 8) * 2.0**-52 * terms).all()
+
+
+def test_ensemble_of_short_systems():
+    """An ensemble large enough for the kernel with one body per lane, its
+    systems at the edges of the 64-body tiles and 64-partner chunks, one of
+    them with overlapping bodies and masses outside the exact cores' range."""
+    sizes = [17, 63, 64, 65, 100, 127, 128, 129, 1] * 36
+    systems = [compact_disk(seed=200 + k % 18, npl=n, mlo=1e-8, mhi=1e-3) for k, n in enumerate(sizes)]
+    d = systems[7]
+    d.pl_rh[40] = d.pl_rh[90] + 1e-7
+    d.radius[40] = d.radius[90] = 1e-5
+    d.Gmass[3], d.Gmass[100] = 1e-180, 0.0
+    g = S.GpuSystem(S.SYMBA, systems, 0.005, lclose=False)
+    st, (a, _) = g.state(), g.accel()
+    off = np.cumsum([0] + sizes)
+    for k in range(18):
+        s, ids = slice(off[k], off[k + 1]), st["pl_id"][off[k]:off[k + 1]] - 1
+        ref = O.accel_plpl(st["pl_rh"][s], systems[k].Gmass[ids], systems[k].radius[ids])
+        assert np.array_equal(ref, a[s]), k
+    for k in range(18, len(sizes)):
+        if k % 18 != 7:
+            assert np.array_equal(a[off[k]:off[k + 1]], a[off[k % 18]:off[k % 18 + 1]]), k
