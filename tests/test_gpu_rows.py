@@ -1,6 +1,6 @@
-"""GPU parity of the row kernel (terms evaluated by several wavefronts, folded
-in partner order) at the edges of its 16-body tiles and 64-partner chunks,
-against the oracle bit for bit."""
+"""GPU parity of the row kernels (terms evaluated by several wavefronts, folded
+in partner order) at the edges of their 16- and 64-body tiles and 64-partner
+chunks, against the oracle bit for bit."""
 import numpy as np
 import pytest
 
@@ -35,6 +35,36 @@ def test_rows_at_tile_edges(n, nplm, with_radius):
     ref = O.accel_plpl(r, Gm, rad, acc, nplm=nplm)
     got = S.swiftest_kick_getacch_int_all_tri(n, nplm, r, Gm, rad, acc)
     assert np.array_equal(ref.view(np.int64), got.view(np.int64))
+
+
+@pytest.mark.parametrize("n,nplm", [(4096, 4096), (4097, 2100), (10007, 10007), (12287, 6200), (12288, 12288), (12351, 6200),
+                                    (6001, 2000)])
+@pytest.mark.parametrize("with_radius", [True, False])
+def test_large_systems_at_tile_edges(n, nplm, with_radius):
+    """Either side of the limits between the row kernels (4096 bodies, 192
+    tiles of 64), partial last tiles and a first semi-interacting body inside a
+    tile; overlapping bodies, two at one place, a body at NaN (left out with
+    radii) and masses outside the exact cores' range in some chunks."""
+    print(f"large rows n={n} nplm={nplm} radius={with_radius}", flush=True)
+    rng, r, Gm, R = _bodies(n, n + nplm)
+    r[n // 2] = r[n // 2 + 1] + 1e-3
+    R[n // 2] = R[n // 2 + 1] = 1e-2
+    r[700] = r[900]
+    Gm[1500], Gm[n - 1], Gm[64] = 1e-200, 1e-170, 0.0
+    acc = rng.normal(0, 1e-3, (n, 3))
+    acc[0] = acc[n - 1] = -0.0
+    rad = R if with_radius else None
+    ref = O.accel_plpl(r, Gm, rad, acc, nplm=nplm)
+    got = S.swiftest_kick_getacch_int_all_tri(n, nplm, r, Gm, rad, acc)
+    assert np.array_equal(ref, got, equal_nan=True)
+    if with_radius:
+        assert np.isfinite(ref).all()
+        assert np.array_equal(ref.view(np.int64), got.view(np.int64))
+        r[2100, 1] = np.nan
+        ref = O.accel_plpl(r, Gm, rad, acc, nplm=nplm)
+        got = S.swiftest_kick_getacch_int_all_tri(n, nplm, r, Gm, rad, acc)
+        assert np.isfinite(ref).all()
+        assert np.array_equal(ref.view(np.int64), got.view(np.int64))
 
 
 @pytest.mark.parametrize("n,nplm", [(70, 70), (70, 20)])

@@ -100,10 +100,11 @@ def test_plpl_tiles(n):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("integ", ["HELIO", "SYMBA"])
-@pytest.mark.parametrize("n", [1, 15, 16, 31, 383, 384, 385, 400, 800])
+@pytest.mark.parametrize("n", [1, 15, 16, 31, 383, 384, 385, 400, 800, 1024, 1025])
 def test_sums_at_chunk_edges(integ, n):
     """Two steps (the second without vh -> vb) at the edges of the sums'
-    chunks and register sets, bit for bit."""
+    chunks and register sets, and either side of the size up to which their
+    workgroup updates the bodies, bit for bit."""
     print(f"sums {integ} {n}", flush=True)
     d = compact_disk(seed=n, npl=n, ntp=5, mlo=1e-10, mhi=1e-8)
     kind_o, kind_g = (O.HELIO, S.HELIO) if integ == "HELIO" else (O.SYMBA, S.SYMBA)
