@@ -217,7 +217,7 @@ __global__ __launch_bounds__(64) void k_leaf_tp(int ntp, int npl, const double *
                 else far = max(far, (uint32_t)(__double2hiint(r2[u]) - PAIR_R2_LO_HI));
             }
             if (!FAST) {
-                pair_factors<G>(m, r2, f);
+                pair_factors(m, r2, f);
                 if (!gok || __any(far > PAIR_R2_HI_HI - PAIR_R2_LO_HI)) {
 #pragma unroll
                     for (int u = 0; u < G; u++) f[u] = m[u] / (r2[u] * sqrt(r2[u]));
@@ -283,15 +283,6 @@ __global__ __launch_bounds__(256) void k_leaf_drift(const double *mu, double *x,
     v[3 * i] = vx;
     v[3 * i + 1] = vy;
     v[3 * i + 2] = vz;
-}
-
-__global__ void k_aos_to_soa(const double *a, Vec3p s, int n)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    s.x[i] = a[3 * i];
-    s.y[i] = a[3 * i + 1];
-    s.z[i] = a[3 * i + 2];
 }
 
 __global__ void k_fill_i32(int32_t *p, int n, int32_t v)
@@ -647,7 +638,7 @@ __device__ inline void whm_factors(const double (&g)[4], const double (&r2)[4], 
     uint32_t far = 0;
 #pragma unroll
     for (int u = 0; u < 4; u++) far = max(far, use[u] ? (uint32_t)(__double2hiint(r2[u]) - PAIR_R2_LO_HI) : 0u);
-    pair_factors<4>(g, r2, f);
+    pair_factors(g, r2, f);
     if (!gok || __any(far > PAIR_R2_HI_HI - PAIR_R2_LO_HI)) {
 #pragma unroll
         for (int u = 0; u < 4; u++) f[u] = g[u] / (r2[u] * sqrt(r2[u]));
@@ -1380,9 +1371,12 @@ int swg_kick_getacch_int_all_tri_pl(swg_ctx *ctx, int32_t npl, int32_t nplm, con
     const XferItem in[] = {xfer_words(r, dr, 3 * (int64_t)npl), xfer_words(Gmass, dg, npl),
                            xfer_words(acc, da, 3 * (int64_t)npl), xfer_words(radius, dR, radius ? npl : 0)};
     HIPCHK(ctx->leaf->stage.in(st, in, 4));
-    // the triangular sums take 16-body tiles at any size: two copies of the fold
-    // leave 64-body ones no registers (13000 bodies, 5000 of them fully
-    // interacting: 0.63 ms, 3.6 ms with 64)
+    // the triangular sums take 16-body tiles and the registers of two sets of
+    // terms ahead at any size: two copies of the fold leave 64-body tiles none
+    // (13000 bodies, 5000 of them fully interacting: 0.63 ms, 3.6 ms with 64),
+    // and those of one set ahead spill (the call, 10 % of the bodies fully
+    // interacting, one set / two: 200 bodies 53 / 39 us, 2000 296 / 121 us,
+    // 8000 1185 / 170 us, 32768 6959 / 1532 us)
     const bool fast = ctx->pair_mode != 0;
     if (npl - nplm > nplm) launch_leaf_tri<RW_SMALL, 4, 2, true>(st, npl, nplm, dr, dg, dR, da, fast);
     else if (cdiv(npl, RW_SMALL) <= RW_FEW) launch_leaf_tri<RW_SMALL, 4, 2, false>(st, npl, nplm, dr, dg, dR, da, fast);

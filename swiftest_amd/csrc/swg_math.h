@@ -105,24 +105,21 @@ __device__ inline double gm_over_r3(double g, double r2, bool gok)
     return g / (r2 * sqrt(r2));
 }
 
-// Holds two or four values in registers at this point of the program: the
-// empty asm statement (no instruction) keeps the compiler from moving their
-// computation past it, so that their chains advance side by side.
-template <int G>
-__device__ inline void side_by_side(double (&a)[G])
+// Holds four values in registers at this point of the program: the empty asm
+// statement (no instruction) keeps the compiler from moving their computation
+// past it, so that their chains advance side by side.
+__device__ inline void side_by_side(double (&a)[4])
 {
-    static_assert(G == 2 || G == 4, "two or four");
-    if constexpr (G == 2) asm volatile("" : "+v"(a[0]), "+v"(a[1]));
-    else asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
+    asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
 }
 
-// f = div_core(g, r2 * sqrt_core(r2)) of G pairs, step by step.  Each chain is
+// f = div_core(g, r2 * sqrt_core(r2)) of four pairs, step by step.  Each chain is
 // 20 operations deep and the compiler, left to itself, takes one after another,
 // which a wavefront alone on its SIMD spends waiting (64 particles' 500 terms
 // 66 -> 50 us; the rows of 10007 bodies, several wavefronts to a SIMD, 315 -> 298).
-template <int G>
-__device__ inline void pair_factors(const double (&gm)[G], const double (&r2)[G], double (&f)[G])
+__device__ inline void pair_factors(const double (&gm)[4], const double (&r2)[4], double (&f)[4])
 {
+    constexpr int G = 4;
     double y[G], g[G], h[G], d[G], b[G];
 #define EACH(stmt)                        \
     _Pragma("unroll") for (int u = 0; u < G; u++) stmt;

@@ -23,7 +23,8 @@
 // Measured: 2000 bodies 32.6 us (64-body tiles with the partners staged in LDS
 // and read there for every term: 69), 10000 bodies 267 us (338), 32000 bodies
 // 2.0 ms (2.0); the leaf rows of 10007 bodies 267 us (one lane a body: 4466);
-// half of 2000 bodies semi-interacting 60 us (one lane a body: 930).
+// half of 2000 bodies semi-interacting 60 us (one lane a body: 930).  Many
+// short systems keep one body per lane (k_kick_pl_split, which says why).
 #pragma once
 #include "swg_math.h"
 
@@ -78,9 +79,12 @@ __device__ inline double rows_uniform(double v)
 // bodies 35 us, 45 us without); not where two copies of the function stand in
 // one kernel, which have no registers for it.
 // ZERO (rows whose sums start at +0): a term not taken is folded as a zero
-// factor, fma(0, d, s) = s bit for bit (d finite; a sum that starts at +0 is
-// never -0); otherwise the sum is kept by selection, also for a first value
-// of -0 and for partners at infinity.
+// factor, fma(0, d, s) = s bit for bit (a sum that starts at +0 is never -0)
+// for finite d: a body at NaN, which a radius test leaves out of every sum,
+// makes them NaN here.  In a step its own failed drift ends the run.  (Selection
+// in the chunks with such a separation costs 3 % at every size.)  Otherwise the
+// sum is kept by selection, also for a first value of -0 and for partners at
+// infinity.
 // SELF: the bodies are the partners themselves and leave themselves out;
 // otherwise tgt holds others (test particles; nplm = npl, rows).
 template <bool FULL, bool ZERO, bool SELF, int B, int KE, int A, class Init>
@@ -88,7 +92,7 @@ __device__ __attribute__((always_inline)) inline void rows_sums(RowsLds<B, KE, A
                                                                 Init init, int b0, int b1, int nplm, int npl, bool tri,
                                                                 int fast, bool use_radius)
 {
-    constexpr int NB = B / KE, G = NB < 4 ? NB : 4;
+    constexpr int NB = B / KE, G = 4;
     static_assert(NB * KE == B && NB % G == 0, "whole groups of bodies per wavefront");
     static_assert(B == 16 || B == 64, "a chunk holds all of a tile's bodies or none");
     const int lane = (int)(threadIdx.x & 63u), w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -176,7 +180,7 @@ __device__ __attribute__((always_inline)) inline void rows_sums(RowsLds<B, KE, A
                             // by the high word: the exponent alone decides
                             far = max(far, (uint32_t)(__double2hiint(r2[u]) - PAIR_R2_LO_HI));
                         }
-                        pair_factors<G>(gm, r2, fc);
+                        pair_factors(gm, r2, fc);
                         if (tri) {
 #pragma unroll
                             for (int u = 0; u < G; u++) fc[u] = p[3] * fc[u];

@@ -4,9 +4,9 @@
 // and moves 18-38 GB/s; a kernel that reads or writes pinned host memory
 // moves about 50 GB/s and takes many arrays in one launch.  A transfer here
 // is a list of arrays laid end to end (an "image" of 8-byte words).  It goes
-// through the ring chunk by chunk: host memcpy on one side, k_stage_in /
-// k_stage_out on the other, which also turn the callers' (3,n) arrays into
-// the device's component arrays and back.
+// through the ring chunk by chunk: host memcpy on one side, k_stage (either
+// way) on the other, which also turns the callers' (3,n) arrays into the
+// device's component arrays and back.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>

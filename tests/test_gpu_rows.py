@@ -69,8 +69,9 @@ def test_large_systems_at_tile_edges(n, nplm, with_radius):
 
 @pytest.mark.parametrize("n,nplm", [(70, 70), (70, 20)])
 def test_rows_outside_the_fast_range(n, nplm):
-    """Separations and masses outside the exact cores' range, overlapping
-    bodies at infinity or NaN (left out with radii), bit for bit."""
+    """Separations and masses outside the exact cores' range, then a body at
+    NaN, which radii leave out of every other's sum, and one at infinity, which
+    they do not, bit for bit."""
     rng, r, Gm, R = _bodies(n, 5)
     r[:10] *= 1e-130
     r[10:20] *= 1e130
@@ -80,6 +81,10 @@ def test_rows_outside_the_fast_range(n, nplm):
     got = S.swiftest_kick_getacch_int_all_tri(n, nplm, r, Gm, None, acc)
     assert np.array_equal(ref, got, equal_nan=True)
     r[40] = np.nan
+    ref = O.accel_plpl(r, Gm, R, acc, nplm=nplm)
+    got = S.swiftest_kick_getacch_int_all_tri(n, nplm, r, Gm, R, acc)
+    assert np.isfinite(np.delete(ref, slice(0, 20), 0)).all()
+    assert np.array_equal(ref, got, equal_nan=True)
     r[50] = np.inf
     ref = O.accel_plpl(r, Gm, R, acc, nplm=nplm)
     got = S.swiftest_kick_getacch_int_all_tri(n, nplm, r, Gm, R, acc)
