@@ -349,6 +349,9 @@ int swg_system_get_bodies(swg_system *sys, int32_t *id, double *mass, double *Gm
  * change) and keep the fastest for the following steps.  Reports the choice.
  * With SWG_PAIR_FAST the massive-body tiles are 64 bodies and *pl_block
  * reports the number of wavefronts sharing each tile's rows (2 ... 16).
+ * With SWG_PAIR_EXACT a negative *pl_block names a kernel that shares a tile
+ * among several wavefronts: -2 one body per lane, 64 bodies a tile; -4 and -8
+ * one partner per lane, 16 and 64 bodies a tile.
  * No counterpart in the reference (its loops are OpenMP-scheduled). */
 int swg_system_autotune(swg_system *sys, int32_t reps, int32_t *pl_block, int32_t *tp_block);
 /* Live timing: while enabled, every launch of the pl-tp and pl-pl

@@ -1181,13 +1181,15 @@ __device__ inline bool wave_encounter(const LdsSet &S, int i, int j, double renc
 //
 // One wavefront's serial chain is all there is to run here, so its
 // instructions and LDS round trips are the time: a substep of about ten
-// bodies takes 3.7 us (check 0.4, opening kicks 0.35, drift 1.6-2.9, closing
-// kicks 0.8), against 6.9 us with the indices walked through LDS in every
-// phase, branches around each role and both cube roots of an unbound drift on
-// one lane; four steps of a 1024-body system among four, 117 ms instead of
-// 182.  The function is kept out of the kernel's body: inlined there, the
-// kernel's many pointers spill its scalars and addresses (154 ms).  Returns the substeps taken and the deepest level;
-// sets S.wstop when the recursion must stop (error flagged).
+// bodies takes 3.2 to 4.6 us (check 0.4, opening kicks 0.35, drift 1.6-2.9,
+// closing kicks 0.8), 4.5 to 4.8 us in a 32768-body system's deeper sets,
+// against 6.9 us with the indices walked through LDS in every phase, branches
+// around each role and both cube roots of an unbound drift on one lane.  Four
+// steps of a slot pool of four systems, the largest of 1024 bodies: 117 ms,
+// 182 ms before.  The function is kept out of the kernel's body: inlined
+// there, the kernel's many pointers spill its scalars and addresses (154 ms).
+// Returns the substeps taken and the deepest level; sets S.wstop when the
+// recursion must stop (error flagged).
 __device__ __attribute__((noinline)) int2 wave_recursion(int nE, int dw, double mu, int short_circuit, int32_t *err,
                                                          int prof_on)
 {
