@@ -389,6 +389,10 @@ int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const in
 
     // ---- device part of the initialize sequence: vh->vb, tp vb = vh + cb%vb ----
     if (prm.integrator == SWG_WHM) {
+        // WHM steps hold vh alone; vb, which the state returns too, is zero
+        const std::vector<double> z(3 * (size_t)std::max(npl, ntp), 0.0);
+        const XferItem x[] = {xfer_vec3(z.data(), pl.vb, npl), xfer_vec3(z.data(), tp.vb, ntp)};
+        HIPCHK(stage->in(st, x, 2));
         if (int rc = whm_setup()) return rc;
     } else {
         launch_snapshot(st, pl, tp, sy, nsys, npl, 0);

@@ -93,4 +93,6 @@ def test_counters_without_recursion():
             w.run(2)
             s = w.stats()
             assert (s["nsubsteps"], s["max_depth"], s["nplpl_enc"], s["npltp_enc"]) == (0, -1, 0, 0)
+            if integ == S.WHM:  # which has no use for vb
+                assert not w.state()["pl_vb"].any() and not w.state()["tp_vb"].any()
             del w
