@@ -175,7 +175,9 @@ int Ensemble::create(const swg_params &p, int ns, const int32_t *npl_s, const in
         }
         if ((npl_all + 63) / 64 < 2048) {
             const bool shorts = npl_all > (int64_t)KPLB_NPL_MIN * ns && npl_all <= (int64_t)KPLB_NPL * ns;
-            tune.kick_pl_eval = shorts && tiles >= KPLB_TILES ? KPL_BODIES : large < RW_LARGE_TILES ? KPL_ROWS_SMALL : KPL_ROWS_LARGE;
+            tune.kick_pl_eval = shorts && tiles >= KPLB_TILES ? KPL_BODIES
+                                : large < RW_LARGE_TILES      ? KPL_ROWS_SMALL
+                                                              : KPL_ROWS_LARGE;
         }
     }
     h_pl_off.assign(nsys + 1, 0);

@@ -77,11 +77,12 @@ struct SumStage {
 };
 
 // The serial chain over a staged chunk: acc + t[0] + ... + t[n-1] in order.
-// The reads of the next 32 terms are issued before the adds of the current 32, in two sets of registers that change places.  A sum that subtracts
-// stages its terms negated (s - x = s + (-x) bit for bit), and a body a masked
-// sum skips stages +0.0 instead: the chains start at +0.0, a sum that starts at
-// +0 is never -0 (x + (-x) = +0 in round-to-nearest), and s + (+0) = s bit for
-// bit for every other s, so the sums are the masked ones exactly.
+// The reads of the next 32 terms are issued before the adds of the current 32,
+// in two sets of registers that change places.  A sum that subtracts stages its
+// terms negated (s - x = s + (-x) bit for bit), and a body a masked sum skips
+// stages +0.0 instead: the chains start at +0.0, a sum that starts at +0 is
+// never -0 (x + (-x) = +0 in round-to-nearest), and s + (+0) = s bit for bit
+// for every other s, so the sums are the masked ones exactly.
 __device__ inline double chain(double acc, const double *t, int n)
 {
     constexpr int G = 16;  // pairs of terms per set
